@@ -274,7 +274,7 @@ struct SpmvLayout {
     // slots (8 bytes of x), so the counts, starts and slots above are in
     // padded units; P = StageSlotCap bounds their total.
     //   st_head / st_tail float[T]  partial sums of the rows crossing tile ends
-    //   st_metric uint64            distinct x lines per tile, summed
+    //   st_metric uint32[T]         distinct x lines of each tile
     // The header's staged_flag says which path Preprocess chose.
     bool staged = false;
     int64_t st_tiles = 0, st_parts = 0, st_part_size = 0, st_tile_items = 0;
@@ -572,7 +572,7 @@ inline SpmvLayout ComputeLayout(uint64_t rows, uint64_t cols, uint64_t nnz, acls
         l.st_perm_offset = AlignUp(l.st_scan_offset + l.st_scan_bytes + 256);  // re-aligned to 256 at use
         l.st_cl_offset = AlignUp(l.st_perm_offset + n8 * sizeof(uint16_t));
         l.st_metric_offset = AlignUp(l.st_cl_offset + n8 * sizeof(uint16_t));
-        l.total = AlignUp(l.st_metric_offset + sizeof(uint64_t));
+        l.total = AlignUp(l.st_metric_offset + static_cast<size_t>(t) * sizeof(uint32_t));
     }
     if (!transpose && StageEligible(rows, cols, nnz, stageValueBytes)) {
         l.staged = true;
@@ -612,7 +612,7 @@ inline SpmvLayout ComputeLayout(uint64_t rows, uint64_t cols, uint64_t nnz, acls
         l.st_head_offset = AlignUp(l.st_xg_offset + s8 * stageValueBytes);
         l.st_tail_offset = AlignUp(l.st_head_offset + static_cast<size_t>(t) * sizeof(float));
         l.st_metric_offset = AlignUp(l.st_tail_offset + static_cast<size_t>(t) * sizeof(float));
-        l.total = AlignUp(l.st_metric_offset + sizeof(uint64_t));
+        l.total = AlignUp(l.st_metric_offset + static_cast<size_t>(t) * sizeof(uint32_t));
     }
     if (!transpose && narrowTypes && rows > 0 && nnz >= static_cast<uint64_t>(kNarrowMinNnz)) {
         l.narrow = true;

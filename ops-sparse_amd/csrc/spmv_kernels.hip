@@ -3112,9 +3112,50 @@ int BuildTasks(const SpmvLaunch& l, hipStream_t s)
     return 0;
 }
 
+// Checks whose outcome is one bit for the whole matrix: atomics on one address
+// take about 12 ns each, one after the other (agent-scope loads of it no
+// less), so one per wave cost a random matrix of 22.6 M entries 544 µs for its
+// 45 600 row blocks.  A check therefore runs on at most kCheckWgs workgroups
+// of kCheckThreads (eight waves per SIMD over the chip), whose waves loop over
+// the row blocks and stop as soon as one of their workgroup has found an
+// entry that does not fit, and a workgroup raises the flag once.
+constexpr int kCheckThreads = 1024;
+constexpr int64_t kCheckWgs = 512;
+
+unsigned CheckGrid(int64_t waves)
+{
+    const int64_t wgs = (waves + kCheckThreads / kWave - 1) / (kCheckThreads / kWave);
+    return static_cast<unsigned>(wgs < 1 ? 1 : wgs < kCheckWgs ? wgs : kCheckWgs);
+}
+
+// fn(b, lane) for the blocks b of this wave until it returns true for some
+// lane of the workgroup; then *flag = 1.
+template <typename F>
+__device__ __forceinline__ void CheckBlocks(int64_t n, uint32_t* flag, F fn)
+{
+    __shared__ int found;
+    if (threadIdx.x == 0) found = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1);
+    constexpr int kW = kCheckThreads / kWave;
+    for (int64_t b = static_cast<int64_t>(blockIdx.x) * kW + threadIdx.x / kWave; b < n;
+         b += static_cast<int64_t>(gridDim.x) * kW) {
+        const bool out = fn(b, lane);
+        if (__ballot(out) != 0) {
+            if (lane == 0) __hip_atomic_store(&found, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            break;
+        }
+        if (__hip_atomic_load(&found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0) break;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && found != 0) __hip_atomic_fetch_or(flag, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Narrow columns: one wave per row block writes each entry's column as a
 // signed 16-bit offset from the block's first row (nc[k] = col[k] - base -
-// r0); a wave that finds an entry out of that range sets narrow_bad.  Entries
+// r0); an entry out of that range raises narrow_bad (CheckBlocks: the copy is
+// then not used, and a matrix of scattered columns leaves after about one
+// block per wave: 7.2 M random entries 175 -> 12 µs, 22.6 M 544 -> 15).  Entries
 // outside every block (before the first row's offset or after the last) are
 // never summed and are not written.  Nothing is written when the staged
 // gather was chosen: its tables share the storage.
@@ -3161,38 +3202,34 @@ __global__ __launch_bounds__(kThreads) void EntryBlocksKernel(const RowT* norm, 
 // Every entry-aligned block must have at most kWaveRows rows and end within
 // kWaveChunk entries of its window's start; otherwise entry_bad is set.
 template <typename RowT>
-__global__ __launch_bounds__(kThreads) void EntryCheckKernel(const int32_t* eb, const RowT* en, int64_t numE,
-                                                            uint32_t* bad)
+__global__ __launch_bounds__(kCheckThreads) void EntryCheckKernel(const int32_t* eb, const RowT* en, int64_t numE,
+                                                                  uint32_t* bad)
 {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    bool out = false;
-    if (t < numE) {
-        out = eb[t + 1] - eb[t] > kWaveRows ||
-              static_cast<int64_t>(en[t + 1]) > t * kEntryChunk + kWaveChunk;
-    }
-    if (__ballot(out) != 0 && (threadIdx.x & (kWave - 1)) == 0) {
-        __hip_atomic_fetch_or(bad, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    CheckBlocks((numE + kWave - 1) / kWave, bad, [&](int64_t b, int lane) {  // one entry-aligned block per lane
+        const int64_t t = b * kWave + lane;
+        return t < numE && (eb[t + 1] - eb[t] > kWaveRows ||
+                            static_cast<int64_t>(en[t + 1]) > t * kEntryChunk + kWaveChunk);
+    });
 }
 
 template <typename RowT>
-__global__ __launch_bounds__(kThreads) void NarrowColKernel(NarrowParams q)
+__global__ __launch_bounds__(kCheckThreads) void NarrowColKernel(NarrowParams q)
 {
-    const int64_t b = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
     if (*q.flag == 1U) return;
     const bool entry = q.eblocks != nullptr && *q.entry_bad == 0U;  // the partition the kernel will use
-    if (b >= (entry ? q.num_eblocks : q.num_blocks)) return;
-    const int64_t rb = static_cast<int64_t>(entry ? q.eblocks[b] : q.blocks[b]) + q.base;
+    const int32_t* blocks = entry ? q.eblocks : q.blocks;
     const RowT* bn = static_cast<const RowT*>(entry ? q.eblock_nnz : q.block_nnz);
-    const int64_t k1 = static_cast<int64_t>(bn[b + 1]);
-    bool bad = false;
-    for (int64_t k = static_cast<int64_t>(bn[b]) + lane; k < k1; k += kWave) {
-        const int64_t d = static_cast<int64_t>(q.col[k]) - rb;
-        bad |= d < -32768 || d > 32767;
-        q.nc[k] = static_cast<int16_t>(d);
-    }
-    if (__ballot(bad) != 0 && lane == 0) __hip_atomic_fetch_or(q.bad, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    CheckBlocks(entry ? q.num_eblocks : q.num_blocks, q.bad, [&](int64_t b, int lane) {
+        const int64_t rb = static_cast<int64_t>(blocks[b]) + q.base;
+        const int64_t k1 = static_cast<int64_t>(bn[b + 1]);
+        bool bad = false;
+        for (int64_t k = static_cast<int64_t>(bn[b]) + lane; k < k1; k += kWave) {
+            const int64_t d = static_cast<int64_t>(q.col[k]) - rb;
+            bad |= d < -32768 || d > 32767;
+            q.nc[k] = static_cast<int16_t>(d);
+        }
+        return bad;
+    });
 }
 
 // Low 16 bits of the normalised row offsets (the pad entry reads 0).
@@ -3245,14 +3282,14 @@ void BuildNarrow(const SpmvLaunch& l, hipStream_t s)
         hipLaunchKernelGGL((EntryBlocksKernel<RowT>), dim3(eg), dim3(kThreads), 0, s,
                            At<const RowT>(l.ws, l.layout.rowptr_offset), l.rows, ne,
                            At<int32_t>(l.ws, l.layout.eb_offset), At<RowT>(l.ws, l.layout.en_offset));
-        hipLaunchKernelGGL((EntryCheckKernel<RowT>), dim3(eg), dim3(kThreads), 0, s, q.eblocks,
+        hipLaunchKernelGGL((EntryCheckKernel<RowT>), dim3(CheckGrid((ne + kWave - 1) / kWave)), dim3(kCheckThreads), 0,
+                           s, q.eblocks,
                            static_cast<const RowT*>(q.eblock_nnz), ne, &h->entry_bad);
     } else {
         hipLaunchKernelGGL(SetFlagKernel, dim3(1), dim3(1), 0, s, &h->entry_bad, 1U);
     }
     const int64_t waves = q.num_blocks > ne ? q.num_blocks : ne;
-    const unsigned grid = static_cast<unsigned>((waves + kWaves - 1) / kWaves);
-    hipLaunchKernelGGL((NarrowColKernel<RowT>), dim3(grid), dim3(kThreads), 0, s, q);
+    hipLaunchKernelGGL((NarrowColKernel<RowT>), dim3(CheckGrid(waves)), dim3(kCheckThreads), 0, s, q);
     hipLaunchKernelGGL((NarrowRowsKernel<RowT>), dim3(static_cast<unsigned>((l.rows + 2 + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, s, At<const RowT>(l.ws, l.layout.rowptr_offset), l.rows,
                        At<uint16_t>(l.ws, l.layout.nr_offset));
@@ -3266,25 +3303,25 @@ void BuildNarrow(const SpmvLaunch& l, hipStream_t s)
 // val_b); any entry out of range sets narrow_bad.  Runs only when the
 // bucketed Preprocess chose the banded kernel (flag 2), whose copies these
 // are; both regions are sort storage that only the CSC build uses.
-__global__ __launch_bounds__(kThreads) void BandedNarrowKernel(const int32_t* cblocks, const int32_t* cblockNnz,
-                                                               const int32_t* cscRow, const int32_t* cscPos,
-                                                               int64_t numBlocks, int16_t* nrow, int16_t* npos,
-                                                               const uint32_t* flag, uint32_t* bad)
+__global__ __launch_bounds__(kCheckThreads) void BandedNarrowKernel(const int32_t* cblocks, const int32_t* cblockNnz,
+                                                                    const int32_t* cscRow, const int32_t* cscPos,
+                                                                    int64_t numBlocks, int16_t* nrow, int16_t* npos,
+                                                                    const uint32_t* flag, uint32_t* bad)
 {
-    const int64_t b = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    if (b >= numBlocks || *flag != 2U) return;
-    const int64_t c0 = cblocks[b];
-    const int64_t k1 = cblockNnz[b + 1];
-    bool out = false;
-    for (int64_t k = static_cast<int64_t>(cblockNnz[b]) + lane; k < k1; k += kWave) {
-        const int64_t d1 = static_cast<int64_t>(cscRow[k]) - c0;
-        const int64_t d2 = static_cast<int64_t>(cscPos[k]) - k;
-        out |= d1 < -32768 || d1 > 32767 || d2 < -32768 || d2 > 32767;
-        nrow[k] = static_cast<int16_t>(d1);
-        npos[k] = static_cast<int16_t>(d2);
-    }
-    if (__ballot(out) != 0 && lane == 0) __hip_atomic_fetch_or(bad, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (*flag != 2U) return;
+    CheckBlocks(numBlocks, bad, [&](int64_t b, int lane) {
+        const int64_t c0 = cblocks[b];
+        const int64_t k1 = cblockNnz[b + 1];
+        bool out = false;
+        for (int64_t k = static_cast<int64_t>(cblockNnz[b]) + lane; k < k1; k += kWave) {
+            const int64_t d1 = static_cast<int64_t>(cscRow[k]) - c0;
+            const int64_t d2 = static_cast<int64_t>(cscPos[k]) - k;
+            out |= d1 < -32768 || d1 > 32767 || d2 < -32768 || d2 > 32767;
+            nrow[k] = static_cast<int16_t>(d1);
+            npos[k] = static_cast<int16_t>(d2);
+        }
+        return out;
+    });
 }
 
 // The low 16 bits of the column offsets, for the banded kernel's short blocks
@@ -3316,8 +3353,8 @@ void BuildBandedNarrow(const SpmvLaunch& l, hipStream_t s)
 {
     SpmvWsHeader* h = At<SpmvWsHeader>(l.ws, 0);
     const int64_t nb = l.layout.csc_num_blocks;
-    hipLaunchKernelGGL(BandedNarrowKernel, dim3(static_cast<unsigned>((nb + kWaves - 1) / kWaves)), dim3(kThreads), 0,
-                       s, At<const int32_t>(l.ws, l.layout.csc_blocks_offset),
+    hipLaunchKernelGGL(BandedNarrowKernel, dim3(CheckGrid(nb)), dim3(kCheckThreads), 0, s,
+                       At<const int32_t>(l.ws, l.layout.csc_blocks_offset),
                        At<const int32_t>(l.ws, l.layout.csc_block_nnz_offset),
                        At<const int32_t>(l.ws, l.layout.key_b_offset), At<const int32_t>(l.ws, l.layout.csc_pos_offset),
                        nb, At<int16_t>(l.ws, l.layout.key_a_offset), At<int16_t>(l.ws, l.layout.val_b_offset),
@@ -3336,51 +3373,46 @@ void BuildBandedNarrow(const SpmvLaunch& l, hipStream_t s)
 // band: a CSC entry more than 2^16 positions from its CSR position (its
 // value gather), or a CSR entry whose row is more than 2^16 from its column
 // (its x gather).
-__global__ __launch_bounds__(kThreads) void CbandRowKernel(const int32_t* pos, const int32_t* entryRow,
+constexpr int kCbandWgs = 2048;
+
+__global__ __launch_bounds__(kCheckThreads) void CbandRowKernel(const int32_t* pos, const int32_t* entryRow,
                                                           const int32_t* col, int32_t base, int32_t* cscRow,
                                                           int64_t nnz, uint32_t* far)
 {
-    // grid-stride: the grid is capped (GridFor)
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-    const int64_t first = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    for (int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads; i0 < nnz; i0 += stride) {  // wave-uniform
-        const int64_t i = i0 + (first - static_cast<int64_t>(blockIdx.x) * kThreads);
-        uint32_t n = 0;
-        if (i < nnz) {
-            const int32_t q = pos[i];
-            cscRow[i] = entryRow[q];
-            const int64_t dv = static_cast<int64_t>(q) - i;
-            const int64_t dx = static_cast<int64_t>(entryRow[i]) - (static_cast<int64_t>(col[i]) - base);
-            n = (dv >= 65536 || dv <= -65536 ? 1U : 0U) + (dx >= 65536 || dx <= -65536 ? 1U : 0U);
-        }
-        const uint64_t b = __ballot(n != 0U);
-        if (b != 0U) {
-            // the wave's count, by its lanes' counts of 0..2
-            const uint32_t c =
-                static_cast<uint32_t>(__popcll(b)) + static_cast<uint32_t>(__popcll(__ballot(n == 2U)));
-            if ((threadIdx.x & (kWave - 1)) == 0) {
-                __hip_atomic_fetch_add(far, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kCheckThreads;
+    uint32_t n = 0;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kCheckThreads + threadIdx.x; i < nnz; i += stride) {
+        const int32_t q = pos[i];
+        cscRow[i] = entryRow[q];
+        const int64_t dv = static_cast<int64_t>(q) - i;
+        const int64_t dx = static_cast<int64_t>(entryRow[i]) - (static_cast<int64_t>(col[i]) - base);
+        n += (dv >= 65536 || dv <= -65536 ? 1U : 0U) + (dx >= 65536 || dx <= -65536 ? 1U : 0U);
     }
+    // one atomic per workgroup: same-address atomics run one after the other
+    __shared__ uint32_t total;
+    if (threadIdx.x == 0) total = 0U;
+    __syncthreads();
+    for (int m = kWave / 2; m >= 1; m >>= 1) n += static_cast<uint32_t>(__shfl_xor(static_cast<int>(n), m, kWave));
+    if (n != 0U && (threadIdx.x & (kWave - 1)) == 0) atomicAdd(&total, n);
+    __syncthreads();
+    if (threadIdx.x == 0 && total != 0U) __hip_atomic_fetch_add(far, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // One wave per CSC block (first column cb, entries [k0, k1)): every entry's
 // row minus cb and CSR position minus its CSC index within int16, else bad.
-__global__ __launch_bounds__(kThreads) void CbandNarrowCheckKernel(const int32_t* cscRow, const int32_t* pos,
-                                                                  const int32_t* blocks, const int32_t* blockNnz,
-                                                                  int64_t numBlocks, uint32_t* bad)
+__global__ __launch_bounds__(kCheckThreads) void CbandNarrowCheckKernel(const int32_t* cscRow, const int32_t* pos,
+                                                                       const int32_t* blocks, const int32_t* blockNnz,
+                                                                       int64_t numBlocks, uint32_t* bad)
 {
-    const int64_t b = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    if (b >= numBlocks) return;
-    const int64_t cb = blocks[b], k0 = blockNnz[b], k1 = blockNnz[b + 1];
-    bool out = false;
-    for (int64_t j = k0 + lane; j < k1; j += kWave) {
-        const int64_t dr = static_cast<int64_t>(cscRow[j]) - cb, dp = static_cast<int64_t>(pos[j]) - j;
-        out = out || dr < -32768 || dr > 32767 || dp < -32768 || dp > 32767;
-    }
-    if (__ballot(out) != 0 && lane == 0) __hip_atomic_fetch_or(bad, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    CheckBlocks(numBlocks, bad, [&](int64_t b, int lane) {
+        const int64_t cb = blocks[b], k0 = blockNnz[b], k1 = blockNnz[b + 1];
+        bool out = false;
+        for (int64_t j = k0 + lane; j < k1; j += kWave) {
+            const int64_t dr = static_cast<int64_t>(cscRow[j]) - cb, dp = static_cast<int64_t>(pos[j]) - j;
+            out = out || dr < -32768 || dr > 32767 || dp < -32768 || dp > 32767;
+        }
+        return out;
+    });
 }
 
 // With flag kCbandNarrowFlag: the rows and positions packed in place of the
@@ -3662,14 +3694,14 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
             if (BuildCsc<int32_t>(l, s) != 0) return 1;
             if (l.cband && l.layout.cband) {
                 SpmvWsHeader* h = At<SpmvWsHeader>(l.ws, 0);
-                hipLaunchKernelGGL(CbandRowKernel, dim3(GridFor(l.nnz)), dim3(kThreads), 0, s,
+                hipLaunchKernelGGL(CbandRowKernel, dim3(GridFor(l.nnz) < kCbandWgs ? GridFor(l.nnz) : kCbandWgs), dim3(kCheckThreads), 0, s,
                                    At<const int32_t>(l.ws, l.layout.csc_pos_offset),
                                    At<const int32_t>(l.ws, l.layout.entry_row_offset), l.col,
                                    static_cast<int32_t>(l.base), At<int32_t>(l.ws, l.layout.val_b_offset), l.nnz,
                                    &h->narrow_bad);
                 const int64_t nb = l.layout.csc_num_blocks;
                 const unsigned bg = static_cast<unsigned>((nb + kWaves - 1) / kWaves);
-                hipLaunchKernelGGL(CbandNarrowCheckKernel, dim3(bg), dim3(kThreads), 0, s,
+                hipLaunchKernelGGL(CbandNarrowCheckKernel, dim3(CheckGrid(nb)), dim3(kCheckThreads), 0, s,
                                    At<const int32_t>(l.ws, l.layout.val_b_offset),
                                    At<const int32_t>(l.ws, l.layout.csc_pos_offset),
                                    At<const int32_t>(l.ws, l.layout.csc_blocks_offset),

@@ -96,7 +96,7 @@ struct StageParams {
     void* xg;
     float* head;
     float* tail;
-    unsigned long long* metric;
+    uint32_t* metric;  // per tile: distinct x lines (staged gather) or non-empty runs (bucketed transpose)
     uint32_t* flag;
     const uint16_t* rp16;  // low 16 bits of the normalised row offsets (the narrow copy's), or null
     int64_t part;  // pass A: bucket-ordered slots per workgroup
@@ -160,7 +160,6 @@ template <typename RowT>
 __global__ __launch_bounds__(256) void StageTileSplitKernel(StageParams q)
 {
     const int64_t t = blockIdx.x * int64_t{256} + threadIdx.x;
-    if (t == 0) *q.metric = 0ULL;
     if (t > q.tiles) return;
     const int64_t total = q.rows + q.nnz;
     const int64_t d = t * q.tile_items < total ? t * q.tile_items : total;
@@ -204,7 +203,9 @@ __device__ __forceinline__ void LoadTileCols(const StageParams& q, int64_t e0, i
 // padded to a multiple of q.chunk (column T is zero).  Also the path
 // decision's metric: the tile's distinct x lines, estimated by linear
 // counting over a 2^15-bit LDS bitmap of hashed lines (order-independent,
-// hence the same on every run), added to q.metric.  The decision follows
+// hence the same on every run), written to q.metric[t] (a sum by one atomic
+// per tile ran at the rate of same-address atomics, 12 ns each: 209 of the
+// kernel's 267 µs on the 134 M-entry Zipf matrix).  The decision follows
 // this kernel, so a matrix that keeps the row kernels skips the rest.
 constexpr int kMapBits = 1 << 15;
 constexpr int kMapWords = kMapBits / 32;
@@ -277,8 +278,7 @@ __global__ __launch_bounds__(kSortThreads) void StageCountKernel(StageParams q)
         const double mb = static_cast<double>(kMapBits);
         const double est = z >= static_cast<uint32_t>(kMapBits) ? static_cast<double>(n)
                                                                   : -mb * log1p(-static_cast<double>(z) / mb);
-        const unsigned long long lines = static_cast<unsigned long long>(est + 0.5);
-        if (lines != 0ULL) atomicAdd(q.metric, lines);
+        q.metric[t] = static_cast<uint32_t>(est + 0.5);
     }
 }
 
@@ -395,11 +395,27 @@ __global__ __launch_bounds__(kThr) void StageRankKernel(StageParams q)
     }
 }
 
+// Sum of the tiles' metrics, by a workgroup of kDecideThreads.
+constexpr int kDecideThreads = 1024;
+__device__ __forceinline__ unsigned long long SumMetric(const StageParams& q)
+{
+    using Reduce = hipcub::BlockReduce<unsigned long long, kDecideThreads>;
+    __shared__ typename Reduce::TempStorage storage;
+    __shared__ unsigned long long total;
+    unsigned long long sum = 0ULL;
+    for (int64_t t = threadIdx.x; t < q.tiles; t += kDecideThreads) sum += q.metric[t];
+    sum = Reduce(storage).Sum(sum);
+    if (threadIdx.x == 0) total = sum;
+    __syncthreads();
+    return total;
+}
+
 // The path decision: staged when the tiles' distinct x lines exceed
 // nnz / kStageLinesPerEntryDen.
-__global__ void StageDecideKernel(StageParams q)
+__global__ __launch_bounds__(kDecideThreads) void StageDecideKernel(StageParams q)
 {
-    const unsigned long long lines = *q.metric;
+    const unsigned long long lines = SumMetric(q);
+    if (threadIdx.x != 0) return;
     *q.flag = lines * static_cast<unsigned long long>(kStageLinesPerEntryDen) >
                       static_cast<unsigned long long>(q.nnz)
                   ? 1U
@@ -1182,7 +1198,7 @@ __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
 // run with an LDS atomic: the order inside a run is free, because pass 1 puts
 // every product at its own slot and pass 2 moves it to its own column-order
 // place before the columns are summed in row order, so results do not depend
-// on it.  Adds the tile's count of non-empty runs (the path metric).
+// on it.  Writes the tile's count of non-empty runs (the path metric).
 template <int kItems, typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtRankKernel(StageParams q)
 {
@@ -1259,7 +1275,7 @@ __global__ __launch_bounds__(kSortThreads) void BtRankKernel(StageParams q)
         }
     }
     __syncthreads();
-    if (tid == 0 && runCount != 0U) atomicAdd(q.metric, static_cast<unsigned long long>(runCount));
+    if (tid == 0) q.metric[t] = runCount;
 }
 
 // csc_row[j] = entry_row[csc_pos[j]] (into the inv array, no longer
@@ -1287,10 +1303,10 @@ __global__ __launch_bounds__(256) void BtCscRowKernel(StageParams q)
 // 2 M 40 -> 27-30, 4 M 78 (CSC kernels) -> 38.
 constexpr int64_t kBtWideNnz = int64_t{1} << 21;
 template <typename RowT>
-__global__ __launch_bounds__(256) void BtDecideKernel(StageParams q)
+__global__ __launch_bounds__(kDecideThreads) void BtDecideKernel(StageParams q)
 {
     __shared__ int ok;
-    const unsigned long long runs = *q.metric;
+    const unsigned long long runs = SumMetric(q);
     const bool scattered =
         runs * static_cast<unsigned long long>(kBtRunEntries) > static_cast<unsigned long long>(q.nnz) ||
         (q.nnz >= kBtWideNnz && 2ULL * runs >= static_cast<unsigned long long>(q.tiles) *
@@ -1299,7 +1315,7 @@ __global__ __launch_bounds__(256) void BtDecideKernel(StageParams q)
     __syncthreads();
     const RowT* colptr = static_cast<const RowT*>(q.colptr);
     const int64_t w = int64_t{1} << q.wshift;
-    for (int64_t b = threadIdx.x; b < q.buckets; b += 256) {
+    for (int64_t b = threadIdx.x; b < q.buckets; b += kDecideThreads) {
         const int64_t c0 = b * w;
         const int64_t c1 = c0 + w < q.cols ? c0 + w : q.cols;
         if (static_cast<int64_t>(colptr[c1]) - static_cast<int64_t>(colptr[c0]) > kBtRegionCap) ok = 0;
@@ -1747,7 +1763,7 @@ StageParams MakeStageParams(const SpmvLaunch& l)
     q.xg = At<void>(l.ws, L.st_xg_offset);
     q.head = At<float>(l.ws, L.st_head_offset);
     q.tail = At<float>(l.ws, L.st_tail_offset);
-    q.metric = At<unsigned long long>(l.ws, L.st_metric_offset);
+    q.metric = At<uint32_t>(l.ws, L.st_metric_offset);
     q.flag = &At<SpmvWsHeader>(l.ws, 0)->staged_flag;
     q.part = L.st_part_size;
     q.rp16 = l.narrow && L.narrow ? At<uint16_t>(l.ws, L.nr_offset) : nullptr;
@@ -1780,7 +1796,7 @@ int StagedPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
     hipLaunchKernelGGL((StageTileSplitKernel<RowT>), dim3(static_cast<unsigned>((T + 1 + 255) / 256)), dim3(256), 0,
                        s, q);
     hipLaunchKernelGGL(StageCountKernel, dim3(static_cast<unsigned>(T + 1)), dim3(kSortThreads), 0, s, q);
-    hipLaunchKernelGGL(StageDecideKernel, dim3(1), dim3(1), 0, s, q);  // the rank kernel runs only when staged
+    hipLaunchKernelGGL(StageDecideKernel, dim3(1), dim3(kDecideThreads), 0, s, q);  // the rank kernel runs only when staged
     const int64_t cells = static_cast<int64_t>(L.st_buckets + 1) * (T + 1);
     void* temp = reinterpret_cast<void*>(
         (reinterpret_cast<uintptr_t>(At<uint8_t>(l.ws, L.st_scan_offset)) + 255) & ~uintptr_t{255});
@@ -1824,7 +1840,7 @@ int BtPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
                        dim3(static_cast<unsigned>((T + 1 + 31) / 32), static_cast<unsigned>((L.st_buckets + 1 + 31) / 32)),
                        dim3(32, 8), 0, s, q);
     hipLaunchKernelGGL((BtRankKernel<kWide, RowT>), dim3(static_cast<unsigned>(T)), dim3(kSortThreads), 0, s, q);
-    hipLaunchKernelGGL((BtDecideKernel<RowT>), dim3(1), dim3(256), 0, s, q);
+    hipLaunchKernelGGL((BtDecideKernel<RowT>), dim3(1), dim3(kDecideThreads), 0, s, q);
     hipLaunchKernelGGL((BtCscRowKernel<RowT>), dim3(static_cast<unsigned>((l.nnz + 255) / 256)), dim3(256), 0, s, q);
     return 0;
 }
