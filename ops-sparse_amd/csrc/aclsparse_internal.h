@@ -468,8 +468,30 @@ inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valu
     return (cols + w - 1) / w <= static_cast<uint64_t>(kBtMaxBuckets);
 }
 
-// Radix-sort temporary storage for the CSC build (implemented in spmv_kernels.hip).
-size_t CscSortTempBytes(int64_t nnz, uint32_t posBytes);
+// Sort of the entries by column for the CSC build (spmv_csc_sort.hip): a
+// stable radix sort in digits of at most kSortDigitBits bits over tiles of
+// kSortTile entries; its temporary storage holds a count per digit and tile
+// and a total per digit.
+constexpr int64_t kSortTile = 16384;
+constexpr int kSortDigitBits = 8;
+inline size_t CscSortTempBytes(int64_t nnz)
+{
+    const size_t tiles = static_cast<size_t>((nnz + kSortTile - 1) / kSortTile);
+    return (tiles + 1) * (size_t{1} << kSortDigitBits) * sizeof(uint32_t);
+}
+struct CscSort {
+    const int32_t* col;
+    int64_t col_stride;
+    int32_t base;
+    int64_t rows, cols, nnz;
+    const void* norm;     // normalised row offsets, int32 or int64 (rowptr64)
+    bool rowptr64;
+    int32_t *key, *val;   // results: the columns (cols for entries outside the matrix) in order, their CSR positions
+    int32_t *key_tmp, *val_tmp;
+    void* temp;           // CscSortTempBytes
+    const uint32_t* gate; // non-null: a device word; nothing is written when it reads 1
+};
+void LaunchCscSort(const CscSort& c, void* stream);
 
 // Entries per group of the transpose's compact row table (one wave of 4 entries per lane).
 constexpr int64_t kRowGroup = 256;
@@ -536,7 +558,7 @@ inline SpmvLayout ComputeLayout(uint64_t rows, uint64_t cols, uint64_t nnz, acls
             l.val_b_offset = AlignUp(l.key_b_offset + n * sizeof(int32_t));
             l.prod_offset = l.key_a_offset;  // prod[nnz] of <= 8 bytes ends before val_b
             l.sort_offset = AlignUp(l.val_b_offset + n * rb);
-            l.sort_bytes = CscSortTempBytes(static_cast<int64_t>(nnz), l.rowptr_bytes);
+            l.sort_bytes = CscSortTempBytes(static_cast<int64_t>(nnz));
             l.csc_items_per_block = ItemsPerBlock(cols, nnz);
             l.csc_num_blocks = NumBlocks(cols, nnz);
             l.csc_blocks_offset = AlignUp(l.sort_offset + l.sort_bytes + 256);  // sort temp re-aligned to 256 at use

@@ -432,8 +432,9 @@ aclsparseStatus_t aclsparseSpMV(aclsparseHandle_t handle, aclsparseOperation_t o
     const bool planned = m->rows == 0U ||
                          PlanMatches(m->plan, MakePlan(m, vecX, vecY, opA, computeType, alg, externalBuffer, handle));
     if (!planned && aclsp::LaunchSpmvPreprocess(l, stream) != 0) return ACL_SPARSE_STATUS_EXECUTION_FAILED;
-    // pass A reads x as 16-byte vectors
-    l.staged = planned && m->rows > 0U && m->plan.staged && Aligned16(vecX->values) ? 1 : 0;
+    // pass A reads x as 16-byte vectors; the bucketed transpose, whose
+    // Preprocess leaves no CSC pattern to fall back to, element by element
+    l.staged = planned && m->rows > 0U && m->plan.staged && (IsTranspose(opA) || Aligned16(vecX->values)) ? 1 : 0;
     l.narrow = planned && m->rows > 0U && m->plan.narrow ? 1 : 0;
     l.cband = planned && m->rows > 0U && m->plan.cband ? 1 : 0;
     l.staged_choice = l.staged || l.narrow || l.cband ? StagedChoice(m, stream) : -1;

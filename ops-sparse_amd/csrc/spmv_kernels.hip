@@ -1999,55 +1999,26 @@ __device__ __forceinline__ typename AccOf<A>::T MaybeConj(typename AccOf<A>::T v
 // ------------------------- transpose by columns ------------------------------
 //
 // Preprocess sorts the entries by column (stable radix sort of (column,
-// position) pairs), so y_j = alpha * sum_{i} conj?(a_ij) * x_i + beta * y_j is
+// position) pairs, spmv_csc_sort.hip), so y_j = alpha * sum_{i} conj?(a_ij) * x_i + beta * y_j is
 // a gather over column j's entries: no atomics, a fixed summation order
 // (deterministic results, the reference's CSR_ALG2 transpose semantics,
 // sparse/spmv/arch35/spmv_kernel.cpp:861-879), and the values are read from
 // the caller's array at execution time.
 
-struct CscBuildParams {
-    const int32_t* col;
-    int64_t col_stride;
-    int32_t base;
-    int64_t rows, cols, nnz;
-    const void* norm;  // normalised row offsets (RowT)
-    int32_t* key;      // sort keys: column, or cols for entries outside the matrix
-    void* pos;         // sort values: position in the CSR arrays
-};
-
-template <typename RowT>
-__global__ __launch_bounds__(kThreads) void CscInitKernel(CscBuildParams q)
-{
-    const RowT* norm = static_cast<const RowT*>(q.norm);
-    const int64_t first = static_cast<int64_t>(norm[0]);
-    const int64_t last = static_cast<int64_t>(norm[q.rows]);
-    RowT* pos = static_cast<RowT*>(q.pos);
-    for (int64_t k = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; k < q.nnz;
-         k += static_cast<int64_t>(gridDim.x) * kThreads) {
-        const int64_t c = static_cast<int64_t>(q.col[k * q.col_stride]) - q.base;
-        const bool ok = k >= first && k < last && c >= 0 && c < q.cols;
-        q.key[k] = static_cast<int32_t>(ok ? c : q.cols);
-        pos[k] = static_cast<RowT>(k);
-    }
-}
-
-// colptr[c] = first sorted entry with column >= c, for c in [0, cols].
-template <typename RowT>
-__global__ __launch_bounds__(kThreads) void CscColPtrKernel(const int32_t* keys, int64_t nnz, int64_t cols,
-                                                            RowT* colptr)
-{
-    for (int64_t k = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; k <= nnz;
-         k += static_cast<int64_t>(gridDim.x) * kThreads) {
-        const int64_t prev = k == 0 ? -1 : static_cast<int64_t>(keys[k - 1]);
-        const int64_t cur = k == nnz ? cols : static_cast<int64_t>(keys[k]);
-        for (int64_t c = prev + 1; c <= cur; ++c) colptr[c] = static_cast<RowT>(k);
-    }
-}
+// The kernels of the CSC build do nothing when gate is non-null and reads 1:
+// the path decision was then the column-bucketed kernels, which do not need
+// the CSC pattern.
+__device__ __forceinline__ bool CscGated(const uint32_t* gate) { return gate != nullptr && *gate == 1U; }
 
 // Row of every entry in CSR order (the last row whose normalised offset is
-// <= k; entries outside [norm[0], norm[rows]) get row 0 and are never used);
-// the sorted positions move to their final array if the sort left them in
-// the other buffer.  One wave per workgroup; a wave takes kFinishSpan
+// <= k; entries outside [norm[0], norm[rows]) get row 0 and are never used),
+// and the compact row table of the product pass: per group of kRowGroup
+// entries the row of its first entry inside the matrix (-1 when the group has
+// none or spans more than 255 rows) and each entry's row minus it; the sorted
+// positions move to their final array if the sort left them in another
+// buffer, and the sorted columns give the column offsets (colptr[c] = first
+// sorted entry with column >= c, for c in [0, cols]).  One wave per
+// workgroup; a wave takes kFinishSpan
 // consecutive entries: it finds the rows ra and rb of its first and last
 // in-range entry (wave-uniform searches), marks in LDS the first entry of
 // every row after ra that starts in its span (the largest row where several
@@ -2057,6 +2028,7 @@ __global__ __launch_bounds__(kThreads) void CscColPtrKernel(const int32_t* keys,
 // coalesced.
 constexpr int kFinishPer = 16;
 constexpr int kFinishSpan = kFinishPer * kWave;
+constexpr int64_t kFinishWgs = 8192;  // one wave each, every wave slot of the chip
 template <typename RowT>
 __device__ __forceinline__ int64_t LastRowAtOrBefore(const RowT* norm, int64_t lo, int64_t hi, int64_t k)
 {
@@ -2069,23 +2041,36 @@ __device__ __forceinline__ int64_t LastRowAtOrBefore(const RowT* norm, int64_t l
 }
 
 template <typename RowT>
-__global__ __launch_bounds__(kWave) void CscFinishKernel(const RowT* sortedPos, RowT* pos, int32_t* entryRow,
-                                                         const RowT* norm, int64_t rows, int64_t n)
+__global__ __launch_bounds__(kWave) void CscFinishKernel(const int32_t* keys, RowT* colptr, int64_t cols,
+                                                         const int32_t* sortedPos, RowT* pos, int32_t* entryRow,
+                                                         int32_t* groupRow, uint32_t* delta, const RowT* norm,
+                                                         int64_t rows, int64_t n, const uint32_t* gate)
 {
+    static_assert(kFinishSpan % kRowGroup == 0 && kRowGroup == 4 * kWave, "whole groups, four entries per lane");
     __shared__ int32_t mark[kFinishSpan];
+    if (CscGated(gate)) return;
     const int64_t first = static_cast<int64_t>(norm[0]);
     const int64_t last = static_cast<int64_t>(norm[rows]);
     const int lane = threadIdx.x;
     for (int64_t w = blockIdx.x; w * kFinishSpan < n; w += gridDim.x) {
         const int64_t base = w * kFinishSpan;
         const int64_t end = base + kFinishSpan < n ? base + kFinishSpan : n;
-        if (sortedPos != pos) {
+        if constexpr (sizeof(RowT) == 8) {
             for (int64_t k = base + lane; k < end; k += kWave) pos[k] = sortedPos[k];
+        }
+        for (int64_t k = base + lane; k < (end == n ? n + 1 : end); k += kWave) {
+            const int64_t prev = k == 0 ? -1 : static_cast<int64_t>(keys[k - 1]);
+            const int64_t cur = k == n ? cols : static_cast<int64_t>(keys[k]);
+            for (int64_t c = prev + 1; c <= cur; ++c) colptr[c] = static_cast<RowT>(k);
         }
         const int64_t a = base > first ? base : first;
         const int64_t b = (end < last ? end : last) - 1;
         if (a > b) {  // no entry of the span lies in a row (uniform)
             for (int64_t k = base + lane; k < end; k += kWave) entryRow[k] = 0;
+            for (int64_t g = base / kRowGroup; g * kRowGroup < end; ++g) {
+                delta[g * kWave + lane] = 0U;
+                if (lane == 0) groupRow[g] = -1;
+            }
             continue;
         }
         const int64_t ra = LastRowAtOrBefore(norm, 0, rows - 1, a);
@@ -2124,35 +2109,26 @@ __global__ __launch_bounds__(kWave) void CscFinishKernel(const RowT* sortedPos, 
         }
         __syncthreads();
         for (int64_t k = base + lane; k < end; k += kWave) entryRow[k] = mark[k - base];
+        // the span's groups: rows are non-decreasing over [a, b]
+        for (int64_t g = base / kRowGroup; g * kRowGroup < end; ++g) {
+            const int64_t g0 = g * kRowGroup, g1 = g0 + kRowGroup - 1;
+            const int64_t kf = g0 > a ? g0 : a, kl = g1 < b ? g1 : b;
+            const bool any = kf <= kl;
+            const int32_t r0 = any ? mark[kf - base] : 0;
+            const bool narrow = any && mark[kl - base] - r0 <= 255;
+            uint32_t word = 0U;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t k = g0 + lane * 4 + j;
+                const uint32_t d = narrow && k >= kf && k <= kl ? static_cast<uint32_t>(mark[k - base] - r0) : 0U;
+                word |= d << (8 * j);
+            }
+            delta[g * kWave + lane] = word;
+            // a group with no entry inside the matrix takes the per-entry path (it reads nothing)
+            if (lane == 0) groupRow[g] = narrow ? r0 : -1;
+        }
         __syncthreads();
     }
-}
-
-// Compact row table: one workgroup per group of kRowGroup entries.  Rows are
-// non-decreasing over [norm[0], norm[rows]), so the span of a group is its
-// last in-range row minus its first; entries outside that range get delta 0.
-template <typename RowT>
-__global__ __launch_bounds__(kThreads) void CscRowDeltaKernel(const int32_t* entryRow, const RowT* norm, int64_t rows,
-                                                              int32_t* groupRow, uint8_t* delta)
-{
-    static_assert(kRowGroup == kThreads, "one thread per entry of a group");
-    const int64_t g = blockIdx.x;
-    const int64_t first = static_cast<int64_t>(norm[0]);
-    const int64_t last = static_cast<int64_t>(norm[rows]);
-    int64_t kf = g * kRowGroup, kl = kf + kRowGroup - 1;
-    kf = kf > first ? kf : first;
-    kl = kl < last - 1 ? kl : last - 1;
-    int32_t base = 0;
-    bool narrow = true;
-    if (kf <= kl) {
-        base = entryRow[kf];
-        narrow = entryRow[kl] - base <= 255;
-    }
-    const int64_t k = g * kRowGroup + threadIdx.x;
-    const int32_t r = k >= kf && k <= kl ? entryRow[k] : base;
-    delta[k] = narrow ? static_cast<uint8_t>(r - base) : uint8_t{0};
-    // a group with no entry inside the matrix takes the per-entry path (it reads nothing)
-    if (threadIdx.x == 0) groupRow[g] = narrow && kf <= kl ? base : -1;
 }
 
 struct CscParams {
@@ -2351,6 +2327,7 @@ struct PrepParams {
     int64_t items;         // T
     SpmvWsHeader* header;
     SpmvWsHeader header_value;
+    const uint32_t* gate;  // the columns' partition: part of the CSC build (CscGated)
 };
 
 template <typename SrcT>
@@ -2363,6 +2340,7 @@ __device__ __forceinline__ int64_t NormRow(const PrepParams& p, int64_t i)
 template <typename SrcT>
 __global__ __launch_bounds__(kThreads) void SpmvPreprocessKernel(PrepParams p)
 {
+    if (CscGated(p.gate)) return;
     const int64_t i = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
     if (i <= p.rows) {
         const SrcT v = static_cast<SrcT>(NormRow<SrcT>(p, i));
@@ -2605,6 +2583,20 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
     return 0;
 }
 
+// Grid of a stream kernel without task waves: one wave per row block, or,
+// when the launch may exit on the path flag, at most kStagedFallbackWgs
+// workgroups whose waves loop over the blocks (22 000 workgroups that only
+// read the flag took 5.7 µs a launch).
+unsigned FlatGrid(RowBlockParams& c)
+{
+    int64_t wgs = ((c.num_blocks + kFlatWaves - 1) / kFlatWaves + kXcds - 1) / kXcds * kXcds;
+    if (c.skip_flag != nullptr && wgs > kStagedFallbackWgs) {
+        wgs = kStagedFallbackWgs;
+        c.block_stride = wgs * kFlatWaves;
+    }
+    return static_cast<unsigned>(wgs);
+}
+
 // One-pass column kernel of banded fp32 transposes: the stream kernel on the
 // CSC pattern with each entry's row as its "column" (x gathered by row) and
 // its CSR position as its value (the value gathered by position).
@@ -2636,8 +2628,7 @@ void LaunchBandedTranspose(const SpmvLaunch& l, const RowBlockParams& p, hipStre
     c.gval_n = l.nnz;
     c.skip_flag = kGated ? &At<SpmvWsHeader>(l.ws, 0)->staged_flag : nullptr;
     c.run_mask = 1U << (kNarrowB ? kBandedNarrowFlag : 2);
-    const int64_t wgs = (c.num_blocks + kFlatWaves - 1) / kFlatWaves;
-    const unsigned g = static_cast<unsigned>((wgs + kXcds - 1) / kXcds * kXcds);
+    const unsigned g = FlatGrid(c);
     const dim3 wg(kWave * kFlatWaves);
     const bool betaNz = l.device_scalars || l.beta_re != 0.0f;
     if (betaNz) {
@@ -2908,8 +2899,7 @@ int LaunchTranspose(const SpmvLaunch& l, hipStream_t stream)
                 c.task_wgs = 0;
                 c.task_waves = 0;
                 c.skip_flag = q.skip_flag;
-                const int64_t wgs = (c.num_blocks + kFlatWaves - 1) / kFlatWaves;
-                const unsigned g = static_cast<unsigned>((wgs + kXcds - 1) / kXcds * kXcds);
+                const unsigned g = FlatGrid(c);
                 const bool betaNz = l.device_scalars || l.beta_re != 0.0f;
                 const dim3 wg(kWave * kFlatWaves);
                 if (c.skip_flag != nullptr) {
@@ -3297,41 +3287,64 @@ void BuildNarrow(const SpmvLaunch& l, hipStream_t s)
                        static_cast<const uint32_t*>(&h->narrow_bad), static_cast<const uint32_t*>(&h->entry_bad));
 }
 
-// Banded transpose on 16-bit copies: one wave per CSC row block (columns as
-// rows) writes each entry's row as an offset from the block's first column
-// (into key_a) and its CSR position as an offset from its own CSC index (into
-// val_b); any entry out of range sets narrow_bad.  Runs only when the
-// bucketed Preprocess chose the banded kernel (flag 2), whose copies these
-// are; both regions are sort storage that only the CSC build uses.
-__global__ __launch_bounds__(kCheckThreads) void BandedNarrowKernel(const int32_t* cblocks, const int32_t* cblockNnz,
-                                                                    const int32_t* cscRow, const int32_t* cscPos,
-                                                                    int64_t numBlocks, int16_t* nrow, int16_t* npos,
-                                                                    const uint32_t* flag, uint32_t* bad)
-{
-    if (*flag != 2U) return;
-    CheckBlocks(numBlocks, bad, [&](int64_t b, int lane) {
-        const int64_t c0 = cblocks[b];
-        const int64_t k1 = cblockNnz[b + 1];
-        bool out = false;
-        for (int64_t k = static_cast<int64_t>(cblockNnz[b]) + lane; k < k1; k += kWave) {
-            const int64_t d1 = static_cast<int64_t>(cscRow[k]) - c0;
-            const int64_t d2 = static_cast<int64_t>(cscPos[k]) - k;
-            out |= d1 < -32768 || d1 > 32767 || d2 < -32768 || d2 > 32767;
-            nrow[k] = static_cast<int16_t>(d1);
-            npos[k] = static_cast<int16_t>(d2);
-        }
-        return out;
-    });
-}
+// Banded transpose (flag 2): one wave per CSC row block (columns as rows)
+// writes each entry's row (csc_row, key_b) and, for the 16-bit copies, that
+// row as an offset from the block's first column (key_a) and its CSR position
+// as an offset from its own CSC index (val_b), with the low 16 bits of the
+// block's column offsets (key_a's second half) when cp16 is not null; an
+// entry out of range raises narrow_bad.  All regions are sort storage that only the CSC build uses.
+struct BandedParams {
+    const int32_t* blocks;  // the CSC pattern's row blocks
+    const int32_t* block_nnz;
+    int64_t num_blocks;
+    const int32_t* colptr;
+    int64_t cols;
+    const int32_t* pos;        // CSC: CSR position of each entry
+    const int32_t* entry_row;  // CSR: row of each entry
+    int32_t* csc_row;
+    int16_t* nrow;
+    int16_t* npos;
+    uint16_t* cp16;
+    const uint32_t* flag;
+    uint32_t* bad;
+};
 
-// The low 16 bits of the column offsets, for the banded kernel's short blocks
-// (only when the banded kernel was chosen: the region is key_a's second half).
-__global__ __launch_bounds__(kThreads) void BandedNarrowColsKernel(const int32_t* colptr, int64_t cols, uint16_t* cp16,
-                                                                   const uint32_t* flag)
+__global__ __launch_bounds__(kCheckThreads) void BandedRowsKernel(BandedParams q)
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i > cols + 1 || *flag != 2U) return;
-    cp16[i] = i <= cols ? static_cast<uint16_t>(static_cast<uint32_t>(colptr[i]) & 0xFFFFU) : uint16_t{0};
+    __shared__ int found;
+    if (*q.flag != 2U) return;
+    if (threadIdx.x == 0) found = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1);
+    constexpr int kW = kCheckThreads / kWave;
+    bool out = false;
+    for (int64_t b = static_cast<int64_t>(blockIdx.x) * kW + threadIdx.x / kWave; b < q.num_blocks;
+         b += static_cast<int64_t>(gridDim.x) * kW) {
+        const int64_t c0 = q.blocks[b], c1 = q.blocks[b + 1];
+        const int64_t k1 = q.block_nnz[b + 1];
+        for (int64_t k = static_cast<int64_t>(q.block_nnz[b]) + lane; k < k1; k += kWave) {
+            const int32_t p = q.pos[k];
+            const int32_t r = q.entry_row[p];
+            const int64_t d1 = static_cast<int64_t>(r) - c0;
+            const int64_t d2 = static_cast<int64_t>(p) - k;
+            out |= d1 < -32768 || d1 > 32767 || d2 < -32768 || d2 > 32767;
+            q.csc_row[k] = r;
+            q.nrow[k] = static_cast<int16_t>(d1);
+            q.npos[k] = static_cast<int16_t>(d2);
+        }
+        if (q.cp16 != nullptr) {
+            const int64_t end = b + 1 == q.num_blocks ? q.cols + 2 : c1;  // the last block: the end and a pad entry
+            for (int64_t c = c0 + lane; c < end; c += kWave) {
+                q.cp16[c] = c <= q.cols ? static_cast<uint16_t>(static_cast<uint32_t>(q.colptr[c]) & 0xFFFFU)
+                                        : uint16_t{0};
+            }
+        }
+    }
+    if (__ballot(out) != 0 && lane == 0) {
+        __hip_atomic_store(&found, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && found != 0) __hip_atomic_fetch_or(q.bad, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Where the banded kernel's 16-bit column offsets go: after the row offsets
@@ -3349,21 +3362,24 @@ __global__ void BandedNarrowDecideKernel(uint32_t* flag, const uint32_t* bad)
     if (*flag == 2U && *bad == 0U) *flag = static_cast<uint32_t>(kBandedNarrowFlag);
 }
 
-void BuildBandedNarrow(const SpmvLaunch& l, hipStream_t s)
+void BuildBanded(const SpmvLaunch& l, hipStream_t s)
 {
     SpmvWsHeader* h = At<SpmvWsHeader>(l.ws, 0);
-    const int64_t nb = l.layout.csc_num_blocks;
-    hipLaunchKernelGGL(BandedNarrowKernel, dim3(CheckGrid(nb)), dim3(kCheckThreads), 0, s,
-                       At<const int32_t>(l.ws, l.layout.csc_blocks_offset),
-                       At<const int32_t>(l.ws, l.layout.csc_block_nnz_offset),
-                       At<const int32_t>(l.ws, l.layout.key_b_offset), At<const int32_t>(l.ws, l.layout.csc_pos_offset),
-                       nb, At<int16_t>(l.ws, l.layout.key_a_offset), At<int16_t>(l.ws, l.layout.val_b_offset),
-                       static_cast<const uint32_t*>(&h->staged_flag), &h->narrow_bad);
-    if (uint16_t* cp16 = BandedCols16(l)) {
-        hipLaunchKernelGGL(BandedNarrowColsKernel, dim3(static_cast<unsigned>((l.cols + 2 + kThreads - 1) / kThreads)),
-                           dim3(kThreads), 0, s, At<const int32_t>(l.ws, l.layout.colptr_offset), l.cols, cp16,
-                           static_cast<const uint32_t*>(&h->staged_flag));
-    }
+    BandedParams q{};
+    q.blocks = At<const int32_t>(l.ws, l.layout.csc_blocks_offset);
+    q.block_nnz = At<const int32_t>(l.ws, l.layout.csc_block_nnz_offset);
+    q.num_blocks = l.layout.csc_num_blocks;
+    q.colptr = At<const int32_t>(l.ws, l.layout.colptr_offset);
+    q.cols = l.cols;
+    q.pos = At<const int32_t>(l.ws, l.layout.csc_pos_offset);
+    q.entry_row = At<const int32_t>(l.ws, l.layout.entry_row_offset);
+    q.csc_row = At<int32_t>(l.ws, l.layout.key_b_offset);
+    q.nrow = At<int16_t>(l.ws, l.layout.key_a_offset);
+    q.npos = At<int16_t>(l.ws, l.layout.val_b_offset);
+    q.cp16 = BandedCols16(l);
+    q.flag = &h->staged_flag;
+    q.bad = &h->narrow_bad;
+    hipLaunchKernelGGL(BandedRowsKernel, dim3(CheckGrid(q.num_blocks)), dim3(kCheckThreads), 0, s, q);
     hipLaunchKernelGGL(BandedNarrowDecideKernel, dim3(1), dim3(1), 0, s, &h->staged_flag,
                        static_cast<const uint32_t*>(&h->narrow_bad));
 }
@@ -3445,45 +3461,38 @@ __global__ void CbandDecideKernel(const uint32_t* far, const uint32_t* narrowBad
     }
 }
 
+// The CSC pattern and its row-block partition; with gate, unless *gate reads
+// 1 when they run.
 template <typename RowT>
-int BuildCsc(const SpmvLaunch& l, hipStream_t s)
+void BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
 {
     const int64_t nnz = l.nnz;
-    CscBuildParams q{};
-    q.col = l.col;
-    q.col_stride = l.col_stride;
-    q.base = l.base;
-    q.rows = l.rows;
-    q.cols = l.cols;
-    q.nnz = nnz;
-    q.norm = At<void>(l.ws, l.layout.rowptr_offset);
-    q.key = At<int32_t>(l.ws, l.layout.key_a_offset);
-    q.pos = At<void>(l.ws, l.layout.csc_pos_offset);
-    hipLaunchKernelGGL((CscInitKernel<RowT>), dim3(GridFor(nnz)), dim3(kThreads), 0, s, q);
-    hipcub::DoubleBuffer<int32_t> keys(At<int32_t>(l.ws, l.layout.key_a_offset),
-                                       At<int32_t>(l.ws, l.layout.key_b_offset));
-    hipcub::DoubleBuffer<RowT> vals(At<RowT>(l.ws, l.layout.csc_pos_offset), At<RowT>(l.ws, l.layout.val_b_offset));
-    int endBit = 1;
-    while (endBit < 31 && (int64_t{1} << endBit) <= l.cols) ++endBit;
-    void* temp = reinterpret_cast<void*>(
-        (reinterpret_cast<uintptr_t>(At<uint8_t>(l.ws, l.layout.sort_offset)) + 255) & ~uintptr_t{255});
-    size_t tempBytes = l.layout.sort_bytes;
-    if (hipcub::DeviceRadixSort::SortPairs(temp, tempBytes, keys, vals, static_cast<int>(nnz), 0, endBit, s) !=
-        hipSuccess) {
-        return 1;
-    }
-    hipLaunchKernelGGL((CscColPtrKernel<RowT>), dim3(GridFor(nnz + 1)), dim3(kThreads), 0, s, keys.Current(), nnz,
-                       l.cols, At<RowT>(l.ws, l.layout.colptr_offset));
+    CscSort c{};
+    c.col = l.col;
+    c.col_stride = l.col_stride;
+    c.base = static_cast<int32_t>(l.base);
+    c.rows = l.rows;
+    c.cols = l.cols;
+    c.nnz = nnz;
+    c.norm = At<void>(l.ws, l.layout.rowptr_offset);
+    c.rowptr64 = sizeof(RowT) == 8;
+    // 32-bit positions; CscFinishKernel widens them into csc_pos for int64 offsets
+    int32_t* a = At<int32_t>(l.ws, l.layout.csc_pos_offset);
+    int32_t* b = At<int32_t>(l.ws, l.layout.val_b_offset);
+    c.key = At<int32_t>(l.ws, l.layout.key_a_offset);
+    c.key_tmp = At<int32_t>(l.ws, l.layout.key_b_offset);
+    c.val = c.rowptr64 ? b : a;
+    c.val_tmp = c.rowptr64 ? a : b;
+    c.temp = At<void>(l.ws, l.layout.sort_offset);
+    c.gate = gate;
+    LaunchCscSort(c, s);
     const int64_t finishWaves = (nnz + kFinishSpan - 1) / kFinishSpan;
     hipLaunchKernelGGL((CscFinishKernel<RowT>),
-                       dim3(static_cast<unsigned>(finishWaves < 65536 ? (finishWaves > 0 ? finishWaves : 1) : 65536)),
-                       dim3(kWave), 0, s, vals.Current(),
-                       At<RowT>(l.ws, l.layout.csc_pos_offset), At<int32_t>(l.ws, l.layout.entry_row_offset),
-                       At<const RowT>(l.ws, l.layout.rowptr_offset), l.rows, nnz);
-    hipLaunchKernelGGL((CscRowDeltaKernel<RowT>), dim3(static_cast<unsigned>(l.layout.row_groups)), dim3(kThreads),
-                       0, s, At<const int32_t>(l.ws, l.layout.entry_row_offset),
-                       At<const RowT>(l.ws, l.layout.rowptr_offset), l.rows,
-                       At<int32_t>(l.ws, l.layout.group_row_offset), At<uint8_t>(l.ws, l.layout.row_delta_offset));
+                       dim3(static_cast<unsigned>(finishWaves < kFinishWgs ? finishWaves : kFinishWgs)),
+                       dim3(kWave), 0, s, c.key, At<RowT>(l.ws, l.layout.colptr_offset), l.cols, c.val, At<RowT>(l.ws, l.layout.csc_pos_offset),
+                       At<int32_t>(l.ws, l.layout.entry_row_offset), At<int32_t>(l.ws, l.layout.group_row_offset),
+                       At<uint32_t>(l.ws, l.layout.row_delta_offset), At<const RowT>(l.ws, l.layout.rowptr_offset),
+                       l.rows, nnz, gate);
     // Row-block partition of the columns (the column pass runs the stream
     // kernel on the CSC pattern); colptr is already normalised, so the
     // partition kernel rewrites it in place with the same values.
@@ -3500,10 +3509,10 @@ int BuildCsc(const SpmvLaunch& l, hipStream_t s)
     pp.num_blocks = l.layout.csc_num_blocks;
     pp.items = l.layout.csc_items_per_block;
     pp.header = nullptr;
+    pp.gate = gate;
     const int64_t n = (l.cols > pp.num_blocks ? l.cols : pp.num_blocks) + 1;
     hipLaunchKernelGGL((SpmvPreprocessKernel<RowT>), dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, s, pp);
-    return 0;
 }
 
 }  // namespace
@@ -3515,22 +3524,6 @@ size_t TaskScanTempBytes(int64_t n)
                                          static_cast<int32_t*>(nullptr), static_cast<int>(n)) != hipSuccess) {
         bytes = static_cast<size_t>(n) * 16 + (64 << 10);  // no device to ask: a generous bound
     }
-    return bytes;
-}
-
-size_t CscSortTempBytes(int64_t nnz, uint32_t posBytes)
-{
-    size_t bytes = 0;
-    hipcub::DoubleBuffer<int32_t> k(nullptr, nullptr);
-    hipError_t e;
-    if (posBytes == 8) {
-        hipcub::DoubleBuffer<int64_t> v(nullptr, nullptr);
-        e = hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, k, v, static_cast<int>(nnz), 0, 31);
-    } else {
-        hipcub::DoubleBuffer<int32_t> v(nullptr, nullptr);
-        e = hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, k, v, static_cast<int>(nnz), 0, 31);
-    }
-    if (e != hipSuccess) bytes = static_cast<size_t>(nnz) * 16 + (1 << 20);
     return bytes;
 }
 
@@ -3678,11 +3671,14 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
     const int64_t n = (l.rows > p.num_blocks ? l.rows : p.num_blocks) + 1;
     const unsigned grid = static_cast<unsigned>((n + kThreads - 1) / kThreads);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // a transpose that decides on the column-bucketed kernels (flag 1) needs no CSC pattern
+    const uint32_t* cscGate = l.staged ? &p.header->staged_flag : nullptr;
     if (l.rowptr64) {
         hipLaunchKernelGGL((SpmvPreprocessKernel<int64_t>), dim3(grid), dim3(kThreads), 0, s, p);
         if (l.layout.csc) {
-            if (BuildCsc<int64_t>(l, s) != 0) return 1;
-            return l.staged ? LaunchStagedPreprocess(l, stream) : 0;
+            if (l.staged && LaunchStagedPreprocess(l, stream) != 0) return 1;
+            BuildCsc<int64_t>(l, cscGate, s);
+            return 0;
         }
         if (l.layout.tasks && BuildTasks<int64_t>(l, s) != 0) return 1;
         if (l.staged && LaunchStagedPreprocess(l, stream) != 0) return 1;
@@ -3691,7 +3687,8 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
     } else {
         hipLaunchKernelGGL((SpmvPreprocessKernel<int32_t>), dim3(grid), dim3(kThreads), 0, s, p);
         if (l.layout.csc) {
-            if (BuildCsc<int32_t>(l, s) != 0) return 1;
+            if (l.staged && LaunchStagedPreprocess(l, stream) != 0) return 1;
+            BuildCsc<int32_t>(l, cscGate, s);
             if (l.cband && l.layout.cband) {
                 SpmvWsHeader* h = At<SpmvWsHeader>(l.ws, 0);
                 hipLaunchKernelGGL(CbandRowKernel, dim3(GridFor(l.nnz) < kCbandWgs ? GridFor(l.nnz) : kCbandWgs), dim3(kCheckThreads), 0, s,
@@ -3716,10 +3713,8 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
                                    At<const int32_t>(l.ws, l.layout.csc_block_nnz_offset), nb,
                                    static_cast<const uint32_t*>(&h->staged_flag));
             }
-            if (!l.staged) return 0;
-            if (LaunchStagedPreprocess(l, stream) != 0) return 1;
-            // the banded kernel's 16-bit copies (32-bit offsets and positions only)
-            if (l.nnz <= 0x1FFFFFFFLL && l.val_kind == ValKind::F32) BuildBandedNarrow(l, s);
+            // the banded kernel's rows and 16-bit copies (32-bit offsets and positions only)
+            if (l.staged && l.nnz <= 0x1FFFFFFFLL && l.val_kind == ValKind::F32) BuildBanded(l, s);
             return 0;
         }
         if (l.layout.tasks && BuildTasks<int32_t>(l, s) != 0) return 1;

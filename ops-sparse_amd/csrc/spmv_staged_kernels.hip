@@ -103,11 +103,8 @@ struct StageParams {
     int32_t chunk; // staged slots per 8-byte chunk: runs are padded to a multiple
     int32_t banded_ok;  // bucketed transpose: the one-pass banded kernel exists for this matrix
     // column-bucketed transpose
-    const void* colptr;   // RowT[cols+1], column offsets of the CSC pattern
-    const void* csc_pos;  // RowT[nnz], CSR index of each entry in column order
-    int32_t* inv;         // int32[nnz], column-order place of each CSR entry, then (after
-                          // the sort) csc_row: the row of each entry in column order
-    const int32_t* entry_row;  // int32[nnz], the row of each entry in CSR order
+    void* colptr;         // RowT[cols+2], column offsets
+    uint16_t* bt_col;     // uint16[nnz], bucket order: the column within the bucket (Preprocess only)
     float* prod;          // float[nnz+8], products in bucket order
     Scalars s;
 };
@@ -144,12 +141,13 @@ __device__ __forceinline__ int64_t Norm(const StageParams& q, int64_t i)
 }
 
 // Sort key of an entry: its column (bucket = key >> wshift), or the first
-// column of the bucket S when the column is outside the matrix.
+// column of the bucket S when the column is outside the matrix.  cols is at
+// most kBtMaxBuckets << 16 = 2^27 on both paths, so one unsigned compare
+// rejects every index below base or past the end.
 __device__ __forceinline__ uint32_t KeyOf(const StageParams& q, int32_t rawCol)
 {
-    const int64_t c = static_cast<int64_t>(rawCol) - q.base;
-    if (c < 0 || c >= q.cols) return static_cast<uint32_t>(q.buckets) << q.wshift;
-    return static_cast<uint32_t>(c);
+    const uint32_t c = static_cast<uint32_t>(rawCol) - static_cast<uint32_t>(q.base);
+    return c < static_cast<uint32_t>(q.cols) ? c : static_cast<uint32_t>(q.buckets) << q.wshift;
 }
 
 // ------------------------------- preprocess ---------------------------------
@@ -1118,13 +1116,19 @@ __global__ __launch_bounds__(256) void StageFixupKernel(StageParams q)
 // y = alpha * A^T x + beta * y, fp32 values and compute (BtEligible).  The
 // tiles are the staged path's merge-path tiles; bucket b holds the columns
 // [b*W, (b+1)*W), bucket S the entries outside the rows' range or whose
-// column is outside [0, cols).  Preprocess (pattern only, after the CSC
-// build): per (bucket, tile) counts and their bucket-major scan, each entry's
-// slot in its tile's bucket-ordered runs (st_perm), and, for each slot, its
-// place among its bucket's entries in column order (st_cl, from the CSC
-// pattern).  The bucket-major scan gives bucket b the slots
-// [colptr[b*W], colptr[(b+1)*W]): the same count, and the same start, as its
-// columns' CSC range.
+// column is outside [0, cols).  Preprocess (pattern only): per (bucket, tile)
+// counts and their bucket-major scan, which already decide the path; then,
+// when it is this one, each entry's slot in its tile's bucket-ordered runs
+// (st_perm, BtRankKernel) and, for each slot, its place among its bucket's
+// entries in column order (st_cl) with the column offsets (BtPlaceKernel).
+// The bucket-major scan gives bucket b the slots [colptr[b*W],
+// colptr[(b+1)*W]).  The two kernels are a radix sort by column whose second
+// digit is sorted inside one workgroup per bucket, so the CSC pattern (a
+// sort of all entries, their rows and positions), which the other transpose
+// kernels need, is built only when the decision is another one.  A call that
+// sets up and multiplies once (10.8 M entries of 1 M random columns) takes
+// 208 µs, 803 when the slots and places came from the sorted CSC pattern
+// (sort 305, its inverse 130, slots and places 83, rows 70 µs).
 //  * Pass 1 (BtScatterKernel), one workgroup per tile: the products
 //    a_k * x[row(k)] (values in CSR order, coalesced; each row's x spread
 //    over its entries in LDS, half a tile at a time), placed in LDS at their
@@ -1145,35 +1149,29 @@ constexpr int kBtLongCol = 64;  // columns longer than this are summed by a wave
 constexpr int kBtRunEntries = 64;  // mean run length (entries) below which the bucketed kernels are chosen
 constexpr int kBtMaxLongCols = static_cast<int>(kBtRegionCap) / (kBtLongCol + 1) + 1;
 
-// Bucket of entry k (S: outside the rows' range or a column outside [0, cols)).
-__device__ __forceinline__ uint32_t BtKey(const StageParams& q, int64_t k, int64_t first, int64_t last, int32_t col)
+// Bucket of an entry (S: outside the rows' range or a column outside [0, cols)).
+__device__ __forceinline__ uint32_t BtKey(const StageParams& q, bool inRows, int32_t col)
 {
-    if (k < first || k >= last) return static_cast<uint32_t>(q.buckets);
-    return KeyOf(q, col) >> q.wshift;
+    return inRows ? KeyOf(q, col) >> q.wshift : static_cast<uint32_t>(q.buckets);
 }
 
-// inv[csc_pos[j]] = j.
-template <typename RowT>
-__global__ __launch_bounds__(256) void BtInvertKernel(StageParams q)
-{
-    const int64_t j = blockIdx.x * int64_t{256} + threadIdx.x;
-    if (j >= q.nnz) return;
-    q.inv[static_cast<int64_t>(static_cast<const RowT*>(q.csc_pos)[j])] = static_cast<int32_t>(j);
-}
-
-// counts[s*(T+1) + t] = entries of tile t in bucket s (column T is zero).
+// counts[s*(T+1) + t] = entries of tile t in bucket s (column T is zero);
+// metric[t] = the tile's non-empty runs.
 template <typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
 {
     __shared__ uint32_t hist[kBtMaxBuckets + 1];
+    __shared__ uint32_t runs;
     const int64_t t = blockIdx.x;
     const int nb = q.buckets + 1;
     for (int s = threadIdx.x; s < nb; s += kSortThreads) hist[s] = 0U;
+    if (threadIdx.x == 0) runs = 0U;
     __syncthreads();
     if (t < q.tiles) {
         const int64_t first = Norm<RowT>(q, 0), last = Norm<RowT>(q, q.rows);
         const int64_t e0 = q.tile_nnz[t], e1 = q.tile_nnz[t + 1];
         const int n = static_cast<int>(e1 - e0);
+        const bool inside = e0 >= first && e1 <= last;  // all but the first and last tiles
         uint4 raw[kColGroups];
         LoadTileCols(q, e0, n, raw);  // one round trip
 #pragma unroll
@@ -1183,111 +1181,329 @@ __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if (i + k < n) {
-                    atomicAdd(&hist[BtKey(q, e0 + i + k, first, last, static_cast<int32_t>(WordOf(raw[u], k)))], 1U);
+                    const bool in = inside || (e0 + i + k >= first && e0 + i + k < last);
+                    atomicAdd(&hist[BtKey(q, in, static_cast<int32_t>(WordOf(raw[u], k)))], 1U);
                 }
             }
         }
     }
     __syncthreads();
-    for (int s = threadIdx.x; s < nb; s += kSortThreads) q.counts[s * (q.tiles + 1) + t] = hist[s];
+    uint32_t mine = 0U;
+    for (int s = threadIdx.x; s < nb; s += kSortThreads) {
+        const uint32_t n = hist[s];
+        q.counts[s * (q.tiles + 1) + t] = n;
+        mine += s < q.buckets && n != 0U ? 1U : 0U;
+    }
+    if (mine != 0U) atomicAdd(&runs, mine);
+    __syncthreads();
+    if (threadIdx.x == 0 && t < q.tiles) q.metric[t] = runs;
 }
 
-// Per tile: perm[k] = slot of entry k in the tile's bucket-ordered runs;
-// cl[start(t,b) + (slot - run start)] = the entry's place in bucket b's
-// column-ordered products.  Each entry takes the next place of its bucket's
-// run with an LDS atomic: the order inside a run is free, because pass 1 puts
-// every product at its own slot and pass 2 moves it to its own column-order
-// place before the columns are summed in row order, so results do not depend
-// on it.  Writes the tile's count of non-empty runs (the path metric).
-template <int kItems, typename RowT>
+// Stable places for 64 keys at a time: the counters belong to one wave, so a
+// key's counter after the round minus before is the number of its lanes.
+// Every lane adds 1 to its key's counter and reads it back; LDS operations of
+// one wave complete in order, so the read holds the whole round.  A lane
+// alone with its key takes the count it found; lanes that share a key (rare
+// when there are many more keys than lanes) take places in lane order, one
+// key per turn of the loop, whatever order the hardware added them in.  The
+// kernels that rank are bound by VALU issue (165-185 instructions per 64
+// entries at first, 46 and 51 µs for 10.8 M entries): 32-bit counters, where
+// 16-bit ones would halve the LDS but take five more instructions per access,
+// and whole rounds without lane masks.
+template <bool kMasked>
+__device__ __forceinline__ void CountPlace(uint32_t* ctr, uint32_t key, bool active, uint32_t& found, uint32_t& after)
+{
+    found = after = 0U;
+    if (!kMasked || active) {
+        found = __hip_atomic_fetch_add(ctr + key, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        after = __hip_atomic_load(ctr + key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+template <bool kMasked>
+__device__ __forceinline__ uint32_t StablePlace(uint32_t key, bool active, uint32_t found, uint32_t after)
+{
+    uint64_t shared = __ballot(after - found > 1U);  // every lane of a shared key but one (idle lanes: 0 - 0)
+    while (shared != 0U) {
+        const int lead = __builtin_ctzll(shared);
+        const uint32_t k = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), lead));
+        const bool same = key == k && (!kMasked || active);
+        const uint64_t peers = __ballot(same);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0U));
+        if (same) found = after - static_cast<uint32_t>(__popcll(peers)) + below;
+        shared &= ~peers;
+    }
+    return found;
+}
+
+// The waves' counts of one key -> each wave's first places: `base` plus the
+// counts of the waves before.  Returns the key's total.
+template <int kWaves>
+__device__ __forceinline__ uint32_t WaveBases(uint32_t* table, int keys, int k, uint32_t base)
+{
+    uint32_t run = base;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+        const uint32_t c = table[v * keys + k];
+        table[v * keys + k] = run;
+        run += c;
+    }
+    return run - base;
+}
+
+constexpr int kBtWaves = kSortThreads / kWave;
+constexpr int kBtRounds = CeilDiv(CeilDiv(kWide, kBtWaves), kWave);  // rounds of 64 entries per wave of a tile
+constexpr int kBtBatch = 4;  // rounds whose LDS operations are in flight together
+static_assert(kBtRounds % kBtBatch == 0, "whole batches");
+
+// LDS of BtRankKernel for nb buckets: the waves' counters, the runs' first
+// places in bucket order, their first slots in the tile (uint16) and the
+// tile's columns.
+constexpr unsigned BtRankLdsBytes(int nb)
+{
+    return static_cast<unsigned>(4 * ((kBtWaves + 1) * nb + (nb + 2) / 2) + 2 * kWide);
+}
+
+// Per tile: perm[k] = slot of entry k in the tile's bucket-ordered runs, and
+// each run's columns (within the bucket) to their place in bucket order
+// (bt_col).  Slots follow the entries' order inside a run (each wave ranks
+// its own consecutive stretch of the tile, 64 entries a round), so bucket
+// order is CSR order within every bucket, which BtPlaceKernel keeps.
+template <typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtRankKernel(StageParams q)
 {
     constexpr int kNb = kBtMaxBuckets + 1;
     constexpr int kRunIpt = CeilDiv(kNb, kSortThreads);
-    static_assert(kItems <= kColGroups * 4 * kSortThreads, "a tile's entries fit the column loads");
     using Scan = hipcub::BlockScan<uint32_t, kSortThreads>;
-    __shared__ uint32_t cnt[kNb];       // next slot of each bucket's run (tile-local)
-    __shared__ uint32_t runBase[kNb];   // st_cl slot of each run's first entry minus its tile-local first slot
-    __shared__ uint32_t colBase[kNb];   // CSC index of each bucket's first entry
+    extern __shared__ uint32_t btRankDyn[];
     __shared__ typename Scan::TempStorage scanStorage;
-    __shared__ uint32_t runCount;
-    const int64_t t = blockIdx.x;
-    const int tid = threadIdx.x;
+    if (FlagSet(q.flag) != 1U) return;
+    const int64_t t = ChunkedXcdIndex();  // neighbouring tiles' runs share lines
+    if (t >= q.tiles) return;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int nb = q.buckets + 1;
+    uint32_t* ctr = btRankDyn;  // [kBtWaves][nb]
+    uint32_t* runStart = ctr + kBtWaves * nb;  // [nb]
+    uint16_t* slot0 = reinterpret_cast<uint16_t*>(runStart + nb);  // [nb + 1]
+    uint16_t* staged = slot0 + (nb + 2) / 2 * 2;
     const int64_t e0 = q.tile_nnz[t], e1 = q.tile_nnz[t + 1];
     const int n = static_cast<int>(e1 - e0);
-    const int nb = q.buckets + 1;
     const int64_t first = Norm<RowT>(q, 0), last = Norm<RowT>(q, q.rows);
+
+    // the wave's stretch: columns by coalesced loads, all in flight (zero past the array's end)
+    const int seg = CeilDiv(CeilDiv(n, kBtWaves), kWave) * kWave;
+    const int s0 = wv * seg;
+    const int s1 = s0 + seg < n ? s0 + seg : n;
+    const int64_t cBytes = (q.nnz - e0) * 4;
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int32_t*>(q.col + e0), 0, static_cast<int>(cBytes < 0x7FFFFFFFLL ? cBytes : 0x7FFFFFFFLL),
+        0x00020000);
+    uint32_t key[kBtRounds];
+#pragma unroll
+    for (int r = 0; r < kBtRounds; ++r) {
+        if (r * kWave >= seg) break;  // uniform
+        key[r] = __builtin_amdgcn_raw_buffer_load_b32(rc, (s0 + lane) * 4 + r * kWave * 4, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+
     const uint32_t* startRow = q.start + t * nb;
-    const RowT* colptr = static_cast<const RowT*>(q.colptr);
-    if (tid == 0) runCount = 0U;
-    uint32_t pc[kRunIpt], a[kRunIpt];
-    uint32_t runs = 0U;
+    uint32_t pc[kRunIpt];
 #pragma unroll
     for (int u = 0; u < kRunIpt; ++u) {
         const int sb = tid * kRunIpt + u;
-        a[u] = sb < nb ? startRow[sb] : 0U;
-        pc[u] = sb < nb ? startRow[nb + sb] - a[u] : 0U;
-        if (sb < q.buckets && pc[u] != 0U) ++runs;
-        if (sb < q.buckets) colBase[sb] = static_cast<uint32_t>(colptr[static_cast<int64_t>(sb) << q.wshift]);
+        const uint32_t a = sb < nb ? startRow[sb] : 0U;
+        pc[u] = sb < nb ? startRow[nb + sb] - a : 0U;
+        if (sb < nb) runStart[sb] = a;
     }
+    for (int i = tid; i < kBtWaves * nb; i += kSortThreads) ctr[i] = 0U;
     Scan(scanStorage).ExclusiveSum(pc, pc);
 #pragma unroll
     for (int u = 0; u < kRunIpt; ++u) {
         const int sb = tid * kRunIpt + u;
-        if (sb < nb) {
-            cnt[sb] = pc[u];
-            runBase[sb] = a[u] - pc[u];
-        }
+        if (sb < nb) slot0[sb] = static_cast<uint16_t>(pc[u]);
     }
-    if (runs != 0U) atomicAdd(&runCount, runs);
+    if (tid == 0) slot0[nb] = static_cast<uint16_t>(n);
     __syncthreads();
-    // the tile's column indices and CSC indices (inv) in one round trip of
-    // 16-byte loads, then per entry its slot and place
-    uint4 raw[kColGroups], rinv[kColGroups];
-    LoadTileCols(q, e0, n, raw);
-    {
-        const int64_t iBytes = (q.nnz - e0) * 4;
-        const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(
-            q.inv + e0, 0, static_cast<int>(iBytes < 0x7FFFFFFFLL ? iBytes : 0x7FFFFFFFLL), 0x00020000);
+
+    uint32_t* own = ctr + wv * nb;
+    // entries outside the rows' range go to the last bucket (only the first
+    // and last tiles can have any)
+    const bool inside = e0 >= first && e1 <= last;
 #pragma unroll
-        for (int u = 0; u < kColGroups; ++u) {
-            if (u * 4 * kSortThreads >= n) break;  // uniform
-            const int i = (u * kSortThreads + tid) * 4;
-            rinv[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ri, i * 4, 0, 0));
-        }
-        asm volatile("" ::: "memory");
+    for (int r = 0; r < kBtRounds; ++r) {
+        if (r * kWave >= seg) break;
+        const int i = s0 + r * kWave + lane;
+        key[r] = KeyOf(q, static_cast<int32_t>(key[r]));
+        if (!inside && (e0 + i < first || e0 + i >= last)) key[r] = static_cast<uint32_t>(q.buckets) << q.wshift;
+        if (s0 + (r + 1) * kWave <= s1) atomicAdd(&own[key[r] >> q.wshift], 1U);  // uniform
+        else if (i < s1) atomicAdd(&own[key[r] >> q.wshift], 1U);
     }
+    __syncthreads();
+    for (int k = tid; k < nb; k += kSortThreads) WaveBases<kBtWaves>(ctr, nb, k, slot0[k]);
+    __syncthreads();
+    const uint32_t inMask = (1U << q.wshift) - 1U;
+    uint16_t* perm = q.perm + e0 + s0;
+    const auto batch = [&](int r0, auto masked) {
+        constexpr bool kMasked = decltype(masked)::value;
+        uint32_t found[kBtBatch], after[kBtBatch];
 #pragma unroll
-    for (int u = 0; u < kColGroups; ++u) {
-        if (u * 4 * kSortThreads >= n) break;
-        const int i4 = (u * kSortThreads + tid) * 4;
+        for (int u = 0; u < kBtBatch; ++u) {
+            CountPlace<kMasked>(own, key[r0 + u] >> q.wshift, s0 + (r0 + u) * kWave + lane < s1, found[u], after[u]);
+        }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int i = i4 + k;
-            if (i < n) {
-                const uint32_t b = BtKey(q, e0 + i, first, last, static_cast<int32_t>(WordOf(raw[u], k)));
-                const uint32_t slot = atomicAdd(&cnt[b], 1U);
-                q.perm[e0 + i] = static_cast<uint16_t>(slot);
-                const uint32_t place =
-                    b < static_cast<uint32_t>(q.buckets) ? WordOf(rinv[u], k) - colBase[b] : 0U;
-                q.cl[runBase[b] + slot] = static_cast<uint16_t>(place);
+        for (int u = 0; u < kBtBatch; ++u) {
+            const bool in = s0 + (r0 + u) * kWave + lane < s1;
+            const uint32_t slot = StablePlace<kMasked>(key[r0 + u] >> q.wshift, in, found[u], after[u]);
+            if (!kMasked || in) {
+                perm[(r0 + u) * kWave + lane] = static_cast<uint16_t>(slot);
+                staged[slot] = static_cast<uint16_t>(key[r0 + u] & inMask);
             }
         }
+    };
+#pragma unroll
+    for (int r0 = 0; r0 < kBtRounds; r0 += kBtBatch) {
+        if (s0 + r0 * kWave >= s1) break;  // uniform over the wave
+        if (s0 + (r0 + kBtBatch) * kWave <= s1) batch(r0, std::false_type{});
+        else batch(r0, std::true_type{});
     }
     __syncthreads();
-    if (tid == 0) q.metric[t] = runCount;
+    // the runs out, a power of two of lanes (at least their mean length) each,
+    // four runs' first elements in flight at once (128 lane groups' turns of
+    // three dependent LDS reads otherwise)
+    int lg = 3;
+    while (lg < 6 && (1 << lg) * nb < n) ++lg;
+    const int lanes = 1 << lg, groups = kSortThreads >> lg;
+    constexpr int kRuns = 4;
+    for (int sb = tid >> lg; sb < q.buckets; sb += kRuns * groups) {
+        uint32_t at[kRuns], end[kRuns], dst[kRuns];
+#pragma unroll
+        for (int u = 0; u < kRuns; ++u) {
+            const int run = sb + u * groups < q.buckets ? sb + u * groups : q.buckets;  // slots of bucket S: none kept
+            const uint32_t a = slot0[run];
+            at[u] = a + (tid & (lanes - 1));
+            end[u] = run < q.buckets ? slot0[run + 1] : 0U;
+            dst[u] = runStart[run] - a;
+        }
+        uint16_t v[kRuns];
+#pragma unroll
+        for (int u = 0; u < kRuns; ++u) v[u] = staged[at[u] < end[u] ? at[u] : 0U];
+#pragma unroll
+        for (int u = 0; u < kRuns; ++u) {
+            if (at[u] < end[u]) q.bt_col[dst[u] + at[u]] = v[u];
+            for (uint32_t j = at[u] + lanes; j < end[u]; j += lanes) q.bt_col[dst[u] + j] = staged[j];
+        }
+    }
 }
 
-// csc_row[j] = entry_row[csc_pos[j]] (into the inv array, no longer
-// needed), for the one-pass banded kernel only: launched after the path
-// decision, it does nothing unless that kernel was chosen (a gather of one
-// line per entry, which the other paths would pay for nothing).
-template <typename RowT>
-__global__ __launch_bounds__(256) void BtCscRowKernel(StageParams q)
+// One workgroup per bucket: its slots' places in column order (cl), stable,
+// so that a column's products lie in row order, and its columns' offsets
+// (colptr).  Columns are taken kBtPlaceCols at a time (once, unless the
+// matrix averages under six entries per column); per wave, counters per
+// column of its own consecutive stretch of the bucket's slots.
+constexpr int kBtPlaceCols = 2048;
+constexpr int kBtPlaceRounds = 8;  // rounds of 64 slots in flight per wave
+inline unsigned BtPlaceLdsBytes(int32_t wshift)
 {
-    const int64_t j = blockIdx.x * int64_t{256} + threadIdx.x;
-    if (j >= q.nnz || FlagSet(q.flag) != 2U) return;
-    q.inv[j] = q.entry_row[static_cast<int64_t>(static_cast<const RowT*>(q.csc_pos)[j])];
+    return static_cast<unsigned>(4 * kBtWaves * (wshift >= 11 ? kBtPlaceCols : 1 << wshift));
+}
+
+template <typename RowT>
+__global__ __launch_bounds__(kSortThreads) void BtPlaceKernel(StageParams q)
+{
+    constexpr int kIpt = CeilDiv(kBtPlaceCols, kSortThreads);  // columns per thread
+    using Scan = hipcub::BlockScan<uint32_t, kSortThreads>;
+    extern __shared__ uint32_t btPlaceDyn[];
+    __shared__ typename Scan::TempStorage scanStorage;
+    if (FlagSet(q.flag) != 1U) return;
+    const int64_t b = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int64_t rs = q.start_bm[b * (q.tiles + 1)];
+    const int n = static_cast<int>(static_cast<int64_t>(q.start_bm[(b + 1) * (q.tiles + 1)]) - rs);
+    const int cols = 1 << q.wshift;
+    const int span = cols < kBtPlaceCols ? cols : kBtPlaceCols;
+    const int64_t c0 = b << q.wshift;
+    RowT* colptr = static_cast<RowT*>(q.colptr);
+    uint32_t* own = btPlaceDyn + wv * span;
+    const int seg = CeilDiv(CeilDiv(n, kBtWaves), kWave) * kWave;
+    const int s0 = wv * seg;
+    const int s1 = s0 + seg < n ? s0 + seg : n;
+    const uint16_t* keys = q.bt_col + rs;
+    uint16_t* cl = q.cl + rs;
+    constexpr int kStep = kBtPlaceRounds * kWave;
+    const auto load = [&](int i0, int k0, auto masked, uint32_t (&k)[kBtPlaceRounds]) {
+        constexpr bool kMasked = decltype(masked)::value;
+#pragma unroll
+        for (int u = 0; u < kBtPlaceRounds; ++u) {
+            const int i = i0 + u * kWave + lane;
+            k[u] = !kMasked || i < s1 ? keys[i] - static_cast<uint32_t>(k0) : 0xFFFFFFFFU;
+        }
+    };
+    const auto count = [&](int i0, int k0, auto masked) {
+        constexpr bool kMasked = decltype(masked)::value;
+        uint32_t k[kBtPlaceRounds];
+        load(i0, k0, masked, k);
+#pragma unroll
+        for (int u = 0; u < kBtPlaceRounds; ++u) {
+            if (!kMasked || k[u] < static_cast<uint32_t>(span)) atomicAdd(&own[k[u]], 1U);
+        }
+    };
+    const auto place = [&](int i0, int k0, auto masked) {
+        constexpr bool kMasked = decltype(masked)::value;
+        uint32_t k[kBtPlaceRounds], found[kBtPlaceRounds], after[kBtPlaceRounds];
+        load(i0, k0, masked, k);
+#pragma unroll
+        for (int u = 0; u < kBtPlaceRounds; ++u) {
+            CountPlace<kMasked>(own, k[u], k[u] < static_cast<uint32_t>(span), found[u], after[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kBtPlaceRounds; ++u) {
+            const bool in = k[u] < static_cast<uint32_t>(span);
+            const uint32_t p = StablePlace<kMasked>(k[u], in, found[u], after[u]);
+            if (!kMasked || in) cl[i0 + u * kWave + lane] = static_cast<uint16_t>(p);
+        }
+    };
+    // batches without lane masks: whole ones, when all columns are taken at once
+    const int w1 = cols == span ? s0 + (s1 > s0 ? (s1 - s0) / kStep * kStep : 0) : s0;
+    uint32_t carry = 0U;  // entries of the columns before the current ones
+    for (int k0 = 0; k0 < cols && c0 + k0 < q.cols; k0 += span) {  // uniform
+        for (int i = tid; i < kBtWaves * span; i += kSortThreads) btPlaceDyn[i] = 0U;
+        __syncthreads();
+        for (int i = s0; i < w1; i += kStep) count(i, k0, std::false_type{});  // wave-uniform
+        for (int i = w1; i < s1; i += kStep) count(i, k0, std::true_type{});
+        __syncthreads();
+        // totals of this thread's columns (kIpt consecutive ones), their exclusive scan, the column
+        // offsets and each wave's first places
+        uint32_t len[kIpt];
+        uint32_t sum = 0U;
+#pragma unroll
+        for (int u = 0; u < kIpt; ++u) {
+            const int c = tid * kIpt + u;
+            len[u] = 0U;
+            if (c < span) {
+#pragma unroll
+                for (int v = 0; v < kBtWaves; ++v) len[u] += btPlaceDyn[v * span + c];
+            }
+            sum += len[u];
+        }
+        uint32_t at, total;
+        Scan(scanStorage).ExclusiveSum(sum, at, total);
+        at += carry;
+#pragma unroll
+        for (int u = 0; u < kIpt; ++u) {
+            const int c = tid * kIpt + u;
+            if (c >= span) break;
+            if (c0 + k0 + c < q.cols) colptr[c0 + k0 + c] = static_cast<RowT>(rs + at);
+            WaveBases<kBtWaves>(btPlaceDyn, span, c, at);
+            at += len[u];
+        }
+        carry += total;
+        __syncthreads();
+        for (int i = s0; i < w1; i += kStep) place(i, k0, std::false_type{});
+        for (int i = w1; i < s1; i += kStep) place(i, k0, std::true_type{});
+        __syncthreads();
+    }
+    if (b + 1 == q.buckets && tid < 2) colptr[q.cols + tid] = static_cast<RowT>(rs + n);  // the end, and its pad entry
 }
 
 // The path decision (header flag): 1, the column-bucketed kernels, when the
@@ -1302,7 +1518,6 @@ __global__ __launch_bounds__(256) void BtCscRowKernel(StageParams q)
 // (banded kernel -> bucketed kernels, µs per SpMV): 1 M entries 22 -> 34,
 // 2 M 40 -> 27-30, 4 M 78 (CSC kernels) -> 38.
 constexpr int64_t kBtWideNnz = int64_t{1} << 21;
-template <typename RowT>
 __global__ __launch_bounds__(kDecideThreads) void BtDecideKernel(StageParams q)
 {
     __shared__ int ok;
@@ -1313,12 +1528,8 @@ __global__ __launch_bounds__(kDecideThreads) void BtDecideKernel(StageParams q)
                                                      static_cast<unsigned long long>(q.buckets));
     if (threadIdx.x == 0) ok = 1;
     __syncthreads();
-    const RowT* colptr = static_cast<const RowT*>(q.colptr);
-    const int64_t w = int64_t{1} << q.wshift;
     for (int64_t b = threadIdx.x; b < q.buckets; b += kDecideThreads) {
-        const int64_t c0 = b * w;
-        const int64_t c1 = c0 + w < q.cols ? c0 + w : q.cols;
-        if (static_cast<int64_t>(colptr[c1]) - static_cast<int64_t>(colptr[c0]) > kBtRegionCap) ok = 0;
+        if (q.start_bm[(b + 1) * (q.tiles + 1)] - q.start_bm[b * (q.tiles + 1)] > kBtRegionCap) ok = 0;
     }
     __syncthreads();
     if (threadIdx.x == 0) *q.flag = scattered ? (ok != 0 ? 1U : 0U) : (q.banded_ok != 0 ? 2U : 0U);
@@ -1773,9 +1984,7 @@ StageParams MakeStageParams(const SpmvLaunch& l)
     q.banded_ok = !l.rowptr64 && l.nnz <= 0x1FFFFFFFLL ? 1 : 0;
     q.chunk = L.st_value_bytes > 0 ? static_cast<int32_t>(StageChunkSlots(static_cast<uint32_t>(L.st_value_bytes))) : 1;
     q.colptr = At<void>(l.ws, L.colptr_offset);
-    q.csc_pos = At<void>(l.ws, L.csc_pos_offset);
-    q.inv = At<int32_t>(l.ws, L.key_b_offset);  // free once the CSC build is done
-    q.entry_row = At<const int32_t>(l.ws, L.entry_row_offset);
+    q.bt_col = At<uint16_t>(l.ws, L.key_a_offset);
     q.prod = At<float>(l.ws, L.prod_offset);
     q.s.device = l.device_scalars;
     q.s.alpha_re = l.alpha_re;
@@ -1783,6 +1992,36 @@ StageParams MakeStageParams(const SpmvLaunch& l)
     q.s.alpha_ptr = l.alpha_ptr;
     q.s.beta_ptr = l.beta_ptr;
     return q;
+}
+
+// Dynamic LDS beyond the 64 KiB that older parts allow (pass A's 128 KiB, the
+// transpose's rank and place kernels'); gfx950 has 160 KiB per workgroup.  The attribute is set once per kernel, and a runtime that does
+// not need it may decline it (the launch reports real failures).
+void AllowLds(const void* kernel, unsigned bytes)
+{
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    (void)hipGetLastError();
+}
+
+template <typename XT>
+void AllowGatherLds()
+{
+    static const bool once = [] {
+        AllowLds(reinterpret_cast<const void*>(&StageGatherKernel<XT>), static_cast<unsigned>(kStageSegmentBytes));
+        return true;
+    }();
+    (void)once;
+}
+
+template <typename RowT>
+void AllowRankLds()
+{
+    static const bool once = [] {
+        AllowLds(reinterpret_cast<const void*>(&BtRankKernel<RowT>), BtRankLdsBytes(kBtMaxBuckets + 1));
+        AllowLds(reinterpret_cast<const void*>(&BtPlaceKernel<RowT>), BtPlaceLdsBytes(16));
+        return true;
+    }();
+    (void)once;
 }
 
 unsigned XcdGrid(int64_t n) { return static_cast<unsigned>((n + kXcds - 1) / kXcds * kXcds); }
@@ -1826,7 +2065,6 @@ int BtPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
     const int64_t T = L.st_tiles;
     hipLaunchKernelGGL((StageTileSplitKernel<RowT>), dim3(static_cast<unsigned>((T + 1 + 255) / 256)), dim3(256), 0,
                        s, q);
-    hipLaunchKernelGGL((BtInvertKernel<RowT>), dim3(static_cast<unsigned>((l.nnz + 255) / 256)), dim3(256), 0, s, q);
     hipLaunchKernelGGL((BtCountKernel<RowT>), dim3(static_cast<unsigned>(T + 1)), dim3(kSortThreads), 0, s, q);
     const int64_t cells = static_cast<int64_t>(L.st_buckets + 1) * (T + 1);
     void* temp = reinterpret_cast<void*>(
@@ -1836,12 +2074,15 @@ int BtPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
         hipSuccess) {
         return 1;
     }
+    hipLaunchKernelGGL(BtDecideKernel, dim3(1), dim3(kDecideThreads), 0, s, q);
     hipLaunchKernelGGL(StageTransposeKernel,
                        dim3(static_cast<unsigned>((T + 1 + 31) / 32), static_cast<unsigned>((L.st_buckets + 1 + 31) / 32)),
                        dim3(32, 8), 0, s, q);
-    hipLaunchKernelGGL((BtRankKernel<kWide, RowT>), dim3(static_cast<unsigned>(T)), dim3(kSortThreads), 0, s, q);
-    hipLaunchKernelGGL((BtDecideKernel<RowT>), dim3(1), dim3(kDecideThreads), 0, s, q);
-    hipLaunchKernelGGL((BtCscRowKernel<RowT>), dim3(static_cast<unsigned>((l.nnz + 255) / 256)), dim3(256), 0, s, q);
+    AllowRankLds<RowT>();
+    hipLaunchKernelGGL((BtRankKernel<RowT>), dim3(XcdGrid(T)), dim3(kSortThreads), BtRankLdsBytes(L.st_buckets + 1), s,
+                       q);
+    hipLaunchKernelGGL((BtPlaceKernel<RowT>), dim3(static_cast<unsigned>(L.st_buckets)), dim3(kSortThreads),
+                       BtPlaceLdsBytes(L.st_wshift), s, q);
     return 0;
 }
 
@@ -1892,22 +2133,6 @@ int LaunchStagedRowT(const SpmvLaunch& l, hipStream_t s)
             return 0;
         default: return 1;
     }
-}
-
-// Pass A's dynamic LDS (128 KiB) is beyond the 64 KiB that older parts
-// allow; gfx950 has 160 KiB per workgroup.  The attribute is set once, and a
-// runtime that does not need it may decline it (the launch reports real
-// failures).
-template <typename XT>
-void AllowGatherLds()
-{
-    static const bool once = [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&StageGatherKernel<XT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kStageSegmentBytes));
-        (void)hipGetLastError();
-        return true;
-    }();
-    (void)once;
 }
 
 }  // namespace

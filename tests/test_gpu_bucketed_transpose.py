@@ -327,3 +327,76 @@ def test_mixed_row_lengths_meet_the_middle_of_every_tile(dev, seed):
     assert_close(w.to("cpu"), y)
     y2, _ = run(w)
     assert torch.equal(y.view(torch.int32), y2.view(torch.int32))
+
+
+# rows, cols, mean: columns per bucket W and buckets S around the limits of the slot and place kernels
+PLACE_CASES = [
+    (600_000, 1 << 23, 4.0),  # W = 65536 (16 passes of 4096 columns), hyper-sparse columns
+    (1 << 20, (1 << 21) + 5, 4.0),  # W = 8192: two passes, the last bucket 5 columns wide
+    (1 << 20, (1 << 20) + 4095, 6.5),  # W = 2048, a last bucket of 2047 columns
+    (262_147, 8192, 8.5),  # W = 64, columns of about 270 entries
+    (1 << 21, 1_800_001, 14.0),  # over 1400 buckets: the slot kernel's LDS beyond 64 KiB
+]
+
+
+@pytest.mark.parametrize("rows,cols,mean", PLACE_CASES)
+@pytest.mark.parametrize("x_offset", [0, 1])
+def test_columns_are_summed_in_row_order(dev, rows, cols, mean, x_offset):
+    """Slots and places follow the entries' order: with alpha = 1 and beta = 0 every column of at most 64
+    entries is the sequential fp32 sum of its products in row order, bit for bit (longer ones are summed
+    by a wave).  x_offset = 1 binds an x that is only 4-byte aligned after Preprocess: the bucketed
+    kernels keep the matrix, which has no CSC pattern to fall back to."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows + cols)
+    lengths = torch.poisson(torch.full((rows,), mean, device=dev), generator=g).to(torch.int64)
+    row_ptr, col = wl.csr_from_lengths(lengths, cols, g, dev, distinct=False)
+    vals = torch.rand(col.numel(), generator=g, device=dev) * 2 - 1
+    xs = torch.rand(rows + 1, generator=g, device=dev) * 2 - 1
+    y = torch.full((cols,), float("nan"), device=dev)
+    plan = CsrSpMV(rows, cols, row_ptr.to(torch.int32), col, vals, xs[:rows], y, 1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    x = xs[x_offset:x_offset + rows]
+    plan._lib.aclsparseDnVecSetValues(plan.x.d, ctypes.c_void_p(x.data_ptr()))
+    plan.run()
+    torch.cuda.synchronize()
+    flag, buckets, _ = header(plan)
+    assert flag == 1 and buckets == -(-cols // bucket_width(cols, col.numel()))
+    row = np.repeat(np.arange(rows), np.diff(row_ptr.cpu().numpy()))
+    c, got = col.cpu().numpy(), y.cpu().numpy()
+    prod = vals.cpu().numpy() * x.cpu().numpy()[row]
+    want = np.zeros(cols, np.float32)
+    np.add.at(want, c, prod)
+    count = np.bincount(c, minlength=cols)
+    short = count <= 64
+    np.testing.assert_array_equal(got[short].view(np.uint32), (want[short] + 0.0).view(np.uint32))
+    scale = np.bincount(c, weights=np.abs(prod), minlength=cols)
+    exact = np.bincount(c, weights=prod.astype(np.float64), minlength=cols)
+    assert np.all(np.abs(got - exact) <= 1e-5 * scale)
+
+
+# entry counts around the CSC sort's tile (16384) and wave (1024) edges; columns of one, two, three and four digits
+@pytest.mark.parametrize("nnz", [1, 63, 1024, 16383, 16384, 16385, 49_153])
+@pytest.mark.parametrize("cols", [1, 255, 256, 70_000, 20_000_000])
+@pytest.mark.parametrize("i64", [False, True])
+def test_csc_sort_edges(dev, nnz, cols, i64):
+    """Transposes below the bucketed path's size: the CSC kernels on the pattern the column sort leaves, with
+    entries outside the columns ignored, against fp64 sums."""
+    rng = np.random.default_rng(nnz * 7 + cols)
+    rows = max(1, nnz // 3)
+    row_ptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, rows - 1)), [nnz]])
+    col = rng.integers(0, cols, nnz).astype(np.int32)
+    col[::11] = np.where(np.arange(col[::11].size) % 2 == 0, cols, -1)  # outside the matrix
+    val = rng.uniform(-1, 1, nnz).astype(np.float32)
+    x = rng.uniform(-1, 1, rows).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    y = torch.full((cols,), 0.5, device=dev)
+    plan = CsrSpMV(rows, cols, d(row_ptr.astype(np.int64 if i64 else np.int32)), d(col), d(val), d(x), y, 2.0, -1.0,
+                   op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    ok = (col >= 0) & (col < cols)
+    prod = val.astype(np.float64) * x[np.repeat(np.arange(rows), np.diff(row_ptr))]
+    want = 2.0 * np.bincount(col[ok], weights=prod[ok], minlength=cols) - 0.5
+    scale = 2.0 * np.bincount(col[ok], weights=np.abs(prod[ok]), minlength=cols) + 0.5
+    assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * scale)
