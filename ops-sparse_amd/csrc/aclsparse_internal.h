@@ -434,7 +434,8 @@ inline bool StageEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t v
 }
 
 // ---------------------------------------------------------------------------
-// Column-bucketed transpose (fp32 values and compute, unit strides).  The
+// Column-bucketed transpose (fp32, fp16 or bf16 values, fp32 compute, unit
+// strides; the products are fp32 whatever the values' type).  The
 // CSC column pass gathers each product from a CSR-ordered array as large as
 // the matrix: one MALL line per 4-byte product.  Instead, Preprocess cuts the
 // matrix into the same merge-path tiles and buckets every entry by its
@@ -462,7 +463,7 @@ inline int32_t BtBucketShift(uint64_t cols, uint64_t nnz)
 
 inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valueBytes)
 {
-    if (valueBytes != 4U || rows == 0U || cols == 0U) return false;
+    if (valueBytes == 0U || rows == 0U || cols == 0U) return false;
     if (nnz < static_cast<uint64_t>(kBtMinNnz) || nnz > 0x7FFFFFFFULL) return false;
     const uint64_t w = uint64_t{1} << BtBucketShift(cols, nnz);
     return (cols + w - 1) / w <= static_cast<uint64_t>(kBtMaxBuckets);

@@ -102,6 +102,7 @@ struct StageParams {
     int64_t part;  // pass A: bucket-ordered slots per workgroup
     int32_t chunk; // staged slots per 8-byte chunk: runs are padded to a multiple
     int32_t banded_ok;  // bucketed transpose: the one-pass banded kernel exists for this matrix
+    int32_t fp32_values;
     // column-bucketed transpose
     void* colptr;         // RowT[cols+2], column offsets
     uint16_t* bt_col;     // uint16[nnz], bucket order: the column within the bucket (Preprocess only)
@@ -393,15 +394,20 @@ __global__ __launch_bounds__(kThr) void StageRankKernel(StageParams q)
     }
 }
 
-// Sum of the tiles' metrics, by a workgroup of kDecideThreads.
+// Sum of the tiles' metrics, by a workgroup of kDecideThreads; a metric's
+// bits from kSplit on (0: none) are summed into the sum's high word.
 constexpr int kDecideThreads = 1024;
+template <int kSplit>
 __device__ __forceinline__ unsigned long long SumMetric(const StageParams& q)
 {
     using Reduce = hipcub::BlockReduce<unsigned long long, kDecideThreads>;
     __shared__ typename Reduce::TempStorage storage;
     __shared__ unsigned long long total;
     unsigned long long sum = 0ULL;
-    for (int64_t t = threadIdx.x; t < q.tiles; t += kDecideThreads) sum += q.metric[t];
+    for (int64_t t = threadIdx.x; t < q.tiles; t += kDecideThreads) {
+        const unsigned long long m = q.metric[t];
+        sum += kSplit == 0 ? m : (m & ((1ULL << kSplit) - 1ULL)) | (m >> kSplit << 32);
+    }
     sum = Reduce(storage).Sum(sum);
     if (threadIdx.x == 0) total = sum;
     __syncthreads();
@@ -412,7 +418,7 @@ __device__ __forceinline__ unsigned long long SumMetric(const StageParams& q)
 // nnz / kStageLinesPerEntryDen.
 __global__ __launch_bounds__(kDecideThreads) void StageDecideKernel(StageParams q)
 {
-    const unsigned long long lines = SumMetric(q);
+    const unsigned long long lines = SumMetric<0>(q);
     if (threadIdx.x != 0) return;
     *q.flag = lines * static_cast<unsigned long long>(kStageLinesPerEntryDen) >
                       static_cast<unsigned long long>(q.nnz)
@@ -1113,7 +1119,8 @@ __global__ __launch_bounds__(256) void StageFixupKernel(StageParams q)
 
 // ----------------------- column-bucketed transpose ---------------------------
 //
-// y = alpha * A^T x + beta * y, fp32 values and compute (BtEligible).  The
+// y = alpha * A^T x + beta * y, fp32, fp16 or bf16 values, fp32 compute and
+// products (BtEligible).  The
 // tiles are the staged path's merge-path tiles; bucket b holds the columns
 // [b*W, (b+1)*W), bucket S the entries outside the rows' range or whose
 // column is outside [0, cols).  Preprocess (pattern only): per (bucket, tile)
@@ -1156,7 +1163,11 @@ __device__ __forceinline__ uint32_t BtKey(const StageParams& q, bool inRows, int
 }
 
 // counts[s*(T+1) + t] = entries of tile t in bucket s (column T is zero);
-// metric[t] = the tile's non-empty runs.
+// metric[t] = the tile's non-empty runs (low kBtRunBits bits) and, above them,
+// its entries when its rows average more than kBtLongRows of them.
+constexpr int kBtRunBits = 12;
+constexpr int kBtLongRows = 256;
+static_assert(kBtMaxBuckets < 1 << kBtRunBits && kWide < 1 << (32 - kBtRunBits), "metric fields");
 template <typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
 {
@@ -1196,7 +1207,11 @@ __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
     }
     if (mine != 0U) atomicAdd(&runs, mine);
     __syncthreads();
-    if (threadIdx.x == 0 && t < q.tiles) q.metric[t] = runs;
+    if (threadIdx.x == 0 && t < q.tiles) {
+        const int64_t entries = q.tile_nnz[t + 1] - q.tile_nnz[t];
+        const int64_t rows = q.tile_row[t + 1] - q.tile_row[t];
+        q.metric[t] = runs | (entries > kBtLongRows * rows ? static_cast<uint32_t>(entries) << kBtRunBits : 0U);
+    }
 }
 
 // Stable places for 64 keys at a time: the counters belong to one wave, so a
@@ -1516,15 +1531,23 @@ __global__ __launch_bounds__(kSortThreads) void BtPlaceKernel(StageParams q)
 // average (a random pattern with few, wide buckets has long runs too; a
 // banded one touches a few buckets per tile).  Measured on random patterns
 // (banded kernel -> bucketed kernels, µs per SpMV): 1 M entries 22 -> 34,
-// 2 M 40 -> 27-30, 4 M 78 (CSC kernels) -> 38.
+// 2 M 40 -> 27-30, 4 M 78 (CSC kernels) -> 38.  16-bit values have no banded
+// kernel, and the CSC kernels they otherwise take read neighbouring columns'
+// products of a long row from the same lines: their count to kBtWideNnz leaves
+// out the tiles of long rows, one and a half times (bf16, CSC -> bucketed kernels: Poisson rows of
+// 8-40 entries 2.2 M 36-41 -> 22-32, 3 M 50-55 -> 23-32, 5 M 86-91 -> 32-42;
+// rows of 1 to 200 000 entries, a third of them in long rows, 2.2 M 24-30 ->
+// 29-30, 3 M 29-35 -> 29-32, 5 M 44-49 -> 37-39).
 constexpr int64_t kBtWideNnz = int64_t{1} << 21;
 __global__ __launch_bounds__(kDecideThreads) void BtDecideKernel(StageParams q)
 {
     __shared__ int ok;
-    const unsigned long long runs = SumMetric(q);
+    const unsigned long long sums = SumMetric<kBtRunBits>(q);
+    const unsigned long long runs = sums & 0xFFFFFFFFULL;
+    const int64_t wide = q.nnz - (q.fp32_values != 0 ? 0 : static_cast<int64_t>(sums >> 32) * 3 / 2);
     const bool scattered =
         runs * static_cast<unsigned long long>(kBtRunEntries) > static_cast<unsigned long long>(q.nnz) ||
-        (q.nnz >= kBtWideNnz && 2ULL * runs >= static_cast<unsigned long long>(q.tiles) *
+        (wide >= kBtWideNnz && 2ULL * runs >= static_cast<unsigned long long>(q.tiles) *
                                                      static_cast<unsigned long long>(q.buckets));
     if (threadIdx.x == 0) ok = 1;
     __syncthreads();
@@ -1554,9 +1577,11 @@ constexpr unsigned BtScatterLdsBytes(int64_t nb)
 // workgroups of 81 KB.  Eight waves per SIMD spill 25-30 VGPRs.
 constexpr int kBtPreRows = 4;
 
-template <int kItems, typename RowT>
+template <int kItems, typename RowT, ValKind V>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6))) void BtScatterKernel(StageParams q)
 {
+    using SV = StageVal<V>;
+    using Raw = typename SV::Raw;
     constexpr int kTileItems = kItems;
     constexpr int kMaxLong = Tile<kItems>::kMaxLong;
     constexpr int kGroupSlots = Tile<kItems>::kGroupSlots;
@@ -1615,10 +1640,10 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
     const __amdgpu_buffer_rsrc_t rn = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<RowT*>(static_cast<const RowT*>(q.norm) + r0), 0,
         static_cast<int>(nBytes < 0x7FFFFFFFLL ? nBytes : 0x7FFFFFFFLL), 0x00020000);
-    const int64_t xBytes = (q.rows - r0) * 4;
+    const Raw* x = static_cast<const Raw*>(q.x);
+    const int64_t xBytes = (q.rows - r0) * static_cast<int64_t>(sizeof(Raw));
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(static_cast<const float*>(q.x) + r0), 0,
-        static_cast<int>(xBytes < 0x7FFFFFFFLL ? xBytes : 0x7FFFFFFFLL), 0x00020000);
+        const_cast<Raw*>(x + r0), 0, static_cast<int>(xBytes < 0x7FFFFFFFLL ? xBytes : 0x7FFFFFFFLL), 0x00020000);
     int64_t rowOff[kBtPreRows];
     float xRow[kBtPreRows];
 #pragma unroll
@@ -1635,23 +1660,32 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
         } else {
             rowOff[u] = static_cast<int32_t>(__builtin_amdgcn_raw_buffer_load_b32(rn, i * 4, 0, 0));
         }
-        xRow[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, i * 4, 0, 0));
+        if constexpr (sizeof(Raw) == 4) {
+            xRow[u] = SV::ToF(__builtin_amdgcn_raw_buffer_load_b32(rx, i * 4, 0, 0));
+        } else {
+            xRow[u] = SV::ToF(__builtin_amdgcn_raw_buffer_load_b16(rx, i * 2, 0, 0));
+        }
     }
     const int64_t g0 = e0 >> 2;
     const int a0 = static_cast<int>(e0 - g0 * 4);  // entry e0's place in its group
     const int ng = (a0 + E + 3) >> 2;              // groups of 4 entries touching the tile
-    const int64_t vBytes = (q.nnz - g0 * 4) * 4;
+    // (16-bit values: bytes rounded up to a dword, inside the array's 16-byte block)
+    const int64_t vBytes = ((q.nnz - g0 * 4) * static_cast<int64_t>(sizeof(Raw)) + 3) & ~int64_t{3};
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(static_cast<const float*>(q.val) + g0 * 4), 0,
+        const_cast<Raw*>(static_cast<const Raw*>(q.val) + g0 * 4), 0,
         static_cast<int>(vBytes < 0x7FFFFFFFLL ? vBytes : 0x7FFFFFFFLL), 0x00020000);
     const int64_t pBytes = (q.nnz + 8 - g0 * 4) * 2;
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
         q.perm + g0 * 4, 0, static_cast<int>(pBytes < 0x7FFFFFFFLL ? pBytes : 0x7FFFFFFFLL), 0x00020000);
-    uint4 gv[kGroupSlots];
+    typename SV::Group raw[kGroupSlots];
 #pragma unroll
     for (int u = 0; u < kGroupSlots; ++u) {
         const int gi = tid + u * kTileThreads;
-        gv[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rv, gi * 16, 0, 0));
+        if constexpr (sizeof(Raw) == 4) {
+            raw[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rv, gi * 16, 0, 0));
+        } else {
+            raw[u] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rv, gi * 8, 0, 0));
+        }
     }
     asm volatile("" ::: "memory");
 
@@ -1708,7 +1742,13 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
     //    half's products into registers.  The tile's two edge groups also
     //    hold entries of the neighbouring tiles, which are skipped below.
     const int gs = ng / 2, em = gs * 4;
-    // each group's products replace its values in gv (the same registers)
+    // each group's products replace its values in gv (the same registers; 16-bit values are widened here)
+    uint4 gv[kGroupSlots];
+#pragma unroll
+    for (int u = 0; u < kGroupSlots; ++u) {
+        gv[u] = make_uint4(__float_as_uint(SV::ToF(SV::Get(raw[u], 0))), __float_as_uint(SV::ToF(SV::Get(raw[u], 1))),
+                           __float_as_uint(SV::ToF(SV::Get(raw[u], 2))), __float_as_uint(SV::ToF(SV::Get(raw[u], 3))));
+    }
 #pragma unroll
     for (int ph = 0; ph < 2; ++ph) {
         const int lo = ph == 0 ? 0 : em, hi = ph == 0 ? em : ng * 4;
@@ -1724,7 +1764,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
             float xv = 0.0f;
 #pragma unroll
             for (int h = 0; h < kBtPreRows; ++h) xv = u == h ? xRow[h] : xv;
-            if (u >= kBtPreRows) xv = static_cast<const float*>(q.x)[r0 + loc];
+            if (u >= kBtPreRows) xv = SV::ToF(x[r0 + loc]);
             for (int k = a; k < b; ++k) xs[k - lo] = xv;
         }
         __syncthreads();
@@ -1734,7 +1774,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
             int a = rel[loc], b = rel[loc + 1];
             a = a > lo ? a : lo;
             b = b < hi ? b : hi;
-            const float xv = static_cast<const float*>(q.x)[r0 + loc];
+            const float xv = SV::ToF(x[r0 + loc]);
             for (int k = a + lane; k < b; k += kWave) xs[k - lo] = xv;
         }
         __syncthreads();
@@ -1825,11 +1865,11 @@ struct BtBucketLoads {
     float py[kBtColPre];
 };
 
-template <typename RowT>
+template <typename RowT, OutKind O>
 __device__ __forceinline__ void BtLoadBucket(const StageParams& q, int64_t b, bool betaNz, int tid, BtBucketLoads& L)
 {
     const RowT* colptr = static_cast<const RowT*>(q.colptr);
-    const float* y = static_cast<const float*>(q.y);
+    const typename OutOf<O>::T* y = static_cast<const typename OutOf<O>::T*>(q.y);
     const int64_t c0 = b << q.wshift;
     const int64_t c1 = c0 + (int64_t{1} << q.wshift) < q.cols ? c0 + (int64_t{1} << q.wshift) : q.cols;
 #pragma unroll
@@ -1837,7 +1877,7 @@ __device__ __forceinline__ void BtLoadBucket(const StageParams& q, int64_t b, bo
         const int64_t c = c0 + tid + u * kBtColThreads;
         L.pa[u] = static_cast<int64_t>(colptr[c < c1 ? c : c1]);
         L.pe[u] = static_cast<int64_t>(colptr[c < c1 ? c + 1 : c1]);
-        L.py[u] = betaNz && c < c1 ? y[c] : 0.0f;
+        L.py[u] = betaNz && c < c1 ? OutToAcc<O, AccKind::F32>(y[c]) : 0.0f;
     }
     L.rs = static_cast<int64_t>(colptr[c0]);
     L.n = static_cast<int>(static_cast<int64_t>(colptr[c1]) - L.rs);
@@ -1860,7 +1900,7 @@ __device__ __forceinline__ void BtLoadBucket(const StageParams& q, int64_t b, bo
     }
 }
 
-template <typename RowT>
+template <typename RowT, OutKind O>
 __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
 {
     __shared__ float buf[kBtRegionCap];
@@ -1876,9 +1916,9 @@ __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
     float alpha, beta;
     LoadScalars<AccKind::F32>(q.s, alpha, beta);
     const bool betaNz = beta != 0.0f;  // y is not read when beta == 0, wherever beta lives
-    float* y = static_cast<float*>(q.y);
+    typename OutOf<O>::T* y = static_cast<typename OutOf<O>::T*>(q.y);
     BtBucketLoads cur;
-    BtLoadBucket<RowT>(q, b, betaNz, tid, cur);
+    BtLoadBucket<RowT, O>(q, b, betaNz, tid, cur);
     for (; b < q.buckets; b += gridDim.x) {
         const int64_t c0 = b << q.wshift;
         const int64_t c1 = c0 + (int64_t{1} << q.wshift) < q.cols ? c0 + (int64_t{1} << q.wshift) : q.cols;
@@ -1906,7 +1946,7 @@ __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
             pe[u] = cur.pe[u];
             py[u] = cur.py[u];
         }
-        if (b + gridDim.x < q.buckets) BtLoadBucket<RowT>(q, b + gridDim.x, betaNz, tid, cur);  // uniform
+        if (b + gridDim.x < q.buckets) BtLoadBucket<RowT, O>(q, b + gridDim.x, betaNz, tid, cur);  // uniform
         asm volatile("" ::: "memory");
         auto column = [&](int64_t c, int64_t ca, int64_t ce, float old) {
             const int a = static_cast<int>(ca - rs);
@@ -1917,7 +1957,7 @@ __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
             }
             float sum = 0.0f;
             for (int k = a; k < e; ++k) sum += buf[k];
-            StoreRowOld<OutKind::F32, AccKind::F32>(y, c, sum, alpha, beta, betaNz, old);
+            StoreRowOld<O, AccKind::F32>(y, c, sum, alpha, beta, betaNz, old);
         };
 #pragma unroll
         for (int u = 0; u < kBtColPre; ++u) {
@@ -1925,7 +1965,8 @@ __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
             if (c < c1) column(c, pa[u], pe[u], py[u]);
         }
         for (int64_t c = c0 + tid + kBtColPre * kBtColThreads; c < c1; c += kBtColThreads) {
-            column(c, static_cast<int64_t>(colptr[c]), static_cast<int64_t>(colptr[c + 1]), betaNz ? y[c] : 0.0f);
+            column(c, static_cast<int64_t>(colptr[c]), static_cast<int64_t>(colptr[c + 1]),
+                   betaNz ? OutToAcc<O, AccKind::F32>(y[c]) : 0.0f);
         }
         __syncthreads();
         const int nLong = longCount;
@@ -1936,7 +1977,7 @@ __global__ __launch_bounds__(kBtColThreads) void BtColumnKernel(StageParams q)
             float part = 0.0f;
             for (int k = a + lane; k < e; k += kWave) part += buf[k];
             const float sum = WaveSum(part);
-            if (lane == 0) StoreRow<OutKind::F32, AccKind::F32>(y, c, sum, alpha, beta, betaNz);
+            if (lane == 0) StoreRow<O, AccKind::F32>(y, c, sum, alpha, beta, betaNz);
         }
         __syncthreads();  // the region is free for the next bucket
     }
@@ -1979,9 +2020,10 @@ StageParams MakeStageParams(const SpmvLaunch& l)
     q.part = L.st_part_size;
     q.rp16 = l.narrow && L.narrow ? At<uint16_t>(l.ws, L.nr_offset) : nullptr;
     q.tile_items = L.st_tile_items;
-    // the one-pass banded transpose: 32-bit row offsets and positions whose
-    // byte offsets fit a buffer resource (LaunchBandedTranspose)
-    q.banded_ok = !l.rowptr64 && l.nnz <= 0x1FFFFFFFLL ? 1 : 0;
+    // the one-pass banded transpose: fp32 values, 32-bit row offsets and
+    // positions whose byte offsets fit a buffer resource (LaunchBandedTranspose)
+    q.fp32_values = l.val_kind == ValKind::F32 ? 1 : 0;
+    q.banded_ok = l.val_kind == ValKind::F32 && !l.rowptr64 && l.nnz <= 0x1FFFFFFFLL ? 1 : 0;
     q.chunk = L.st_value_bytes > 0 ? static_cast<int32_t>(StageChunkSlots(static_cast<uint32_t>(L.st_value_bytes))) : 1;
     q.colptr = At<void>(l.ws, L.colptr_offset);
     q.bt_col = At<uint16_t>(l.ws, L.key_a_offset);
@@ -2086,14 +2128,31 @@ int BtPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
     return 0;
 }
 
-template <typename RowT>
+template <typename RowT, ValKind V, OutKind O>
 void BtComputeTyped(const SpmvLaunch& l, hipStream_t s)
 {
     const StageParams q = MakeStageParams(l);
-    hipLaunchKernelGGL((BtScatterKernel<kWide, RowT>), dim3(XcdGrid(l.layout.st_tiles)), dim3(kTileThreads),
+    hipLaunchKernelGGL((BtScatterKernel<kWide, RowT, V>), dim3(XcdGrid(l.layout.st_tiles)), dim3(kTileThreads),
                        BtScatterLdsBytes(l.layout.st_buckets + 1), s, q);
     const int64_t colGrid = l.layout.st_buckets < kBtColGrid ? l.layout.st_buckets : kBtColGrid;
-    hipLaunchKernelGGL((BtColumnKernel<RowT>), dim3(static_cast<unsigned>(colGrid)), dim3(kBtColThreads), 0, s, q);
+    hipLaunchKernelGGL((BtColumnKernel<RowT, O>), dim3(static_cast<unsigned>(colGrid)), dim3(kBtColThreads), 0, s, q);
+}
+
+template <typename RowT>
+int LaunchBtRowT(const SpmvLaunch& l, hipStream_t s)
+{
+    switch (l.val_kind) {
+        case ValKind::F32: BtComputeTyped<RowT, ValKind::F32, OutKind::F32>(l, s); return 0;
+        case ValKind::F16:
+            if (l.out_kind == OutKind::F16) BtComputeTyped<RowT, ValKind::F16, OutKind::F16>(l, s);
+            else BtComputeTyped<RowT, ValKind::F16, OutKind::F32>(l, s);
+            return 0;
+        case ValKind::BF16:
+            if (l.out_kind == OutKind::BF16) BtComputeTyped<RowT, ValKind::BF16, OutKind::BF16>(l, s);
+            else BtComputeTyped<RowT, ValKind::BF16, OutKind::F32>(l, s);
+            return 0;
+        default: return 1;
+    }
 }
 
 template <typename RowT, ValKind V, OutKind O>
@@ -2162,10 +2221,7 @@ int LaunchStagedCompute(const SpmvLaunch& l, void* stream)
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (!l.layout.staged) return 1;
     if (l.op != ACL_SPARSE_OP_NON_TRANSPOSE) {
-        if (l.val_kind != ValKind::F32 || l.out_kind != OutKind::F32) return 1;
-        if (l.rowptr64) BtComputeTyped<int64_t>(l, s);
-        else BtComputeTyped<int32_t>(l, s);
-        return 0;
+        return l.rowptr64 ? LaunchBtRowT<int64_t>(l, s) : LaunchBtRowT<int32_t>(l, s);
     }
     if (l.layout.st_value_bytes == 4) AllowGatherLds<uint32_t>();
     else AllowGatherLds<uint16_t>();

@@ -400,3 +400,56 @@ def test_csc_sort_edges(dev, nnz, cols, i64):
     want = 2.0 * np.bincount(col[ok], weights=prod[ok], minlength=cols) - 0.5
     scale = 2.0 * np.bincount(col[ok], weights=np.abs(prod[ok]), minlength=cols) + 0.5
     assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * scale)
+
+
+@pytest.mark.parametrize("vdt,odt", [(torch.float16, torch.float16), (torch.float16, torch.float32),
+                                     (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("i64", [False, True])
+@pytest.mark.parametrize("rows,cols,mean", [(1 << 20, (1 << 20) + 4095, 6.5), (300_001, 1 << 19, 9.3)])
+def test_16_bit_values(dev, vdt, odt, i64, rows, cols, mean):
+    """fp16 and bf16 values: fp32 products summed in row order and rounded once to y's type, bit for bit for
+    columns of at most 64 entries (x two bytes off a 4-byte boundary, odd entry counts); beta != 0 within one
+    rounding of the same sums."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows + cols)
+    lengths = torch.poisson(torch.full((rows,), mean, device=dev), generator=g).to(torch.int64)
+    lengths[-1] += 1 - int(lengths.sum()) % 2
+    row_ptr, col = wl.csr_from_lengths(lengths, cols, g, dev, distinct=False)
+    assert col.numel() % 2 == 1
+    vals = torch.randn(col.numel(), generator=g, device=dev).to(vdt)
+    x = (torch.rand(rows + 1, generator=g, device=dev) * 2 - 1).to(vdt)[1:]
+    rp = row_ptr.to(torch.int64 if i64 else torch.int32)
+    y = torch.full((cols,), float("nan"), device=dev).to(odt)
+    plan = CsrSpMV(rows, cols, rp, col, vals, x, y, 1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    assert header(plan)[0] == 1
+    row = np.repeat(np.arange(rows), np.diff(row_ptr.cpu().numpy()))
+    c = col.cpu().numpy()
+    prod = vals.float().cpu().numpy() * x.float().cpu().numpy()[row]
+    acc = np.zeros(cols, np.float32)
+    np.add.at(acc, c, prod)
+    want = torch.from_numpy(acc + 0.0).to(odt)
+    short = torch.from_numpy(np.bincount(c, minlength=cols) <= 64)
+    bits = torch.int32 if odt == torch.float32 else torch.int16
+    assert torch.equal(y.cpu()[short].view(bits), want[short].view(bits))
+    y0 = (torch.rand(cols, generator=g, device=dev) * 2 - 1).to(odt)
+    y2 = y0.clone()
+    plan2 = CsrSpMV(rows, cols, rp, col, vals, x, y2, 0.5, -1.0, op=Operation.TRANSPOSE)
+    plan2.preprocess()
+    plan2.run()
+    torch.cuda.synchronize()
+    exact = 0.5 * np.bincount(c, weights=prod.astype(np.float64), minlength=cols) - y0.cpu().double().numpy()
+    scale = 0.5 * np.bincount(c, weights=np.abs(prod), minlength=cols) + np.abs(y0.cpu().double().numpy())
+    eps = {torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8, torch.float32: 0.0}[odt]
+    assert np.all(np.abs(y2.cpu().double().numpy() - exact) <= eps * np.abs(exact) + 1e-5 * scale + 1e-7)
+
+
+def test_banded_16_bit_transpose_keeps_the_csc_kernels(dev):
+    """The one-pass banded kernel is fp32's: a 16-bit Laplacian stays on the CSC kernels."""
+    w = banded_workload(dev, n=1100)
+    w.values, w.x, w.y0, w.out_dtype = w.values.half(), w.x.half(), w.y0.half(), torch.float16
+    y, plan = run(w)
+    assert header(plan)[0] == 0
+    assert_close(w.to("cpu"), y)
