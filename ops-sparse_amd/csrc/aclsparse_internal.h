@@ -471,15 +471,12 @@ inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valu
 
 // Sort of the entries by column for the CSC build (spmv_csc_sort.hip): a
 // stable radix sort in digits of at most kSortDigitBits bits over tiles of
-// kSortTile entries; its temporary storage holds a count per digit and tile
-// and a total per digit.
+// kSortTile entries, whose temporary storage holds a count per digit and tile
+// and a total per digit; below kSortMinNnz entries hipCUB's.
 constexpr int64_t kSortTile = 16384;
 constexpr int kSortDigitBits = 8;
-inline size_t CscSortTempBytes(int64_t nnz)
-{
-    const size_t tiles = static_cast<size_t>((nnz + kSortTile - 1) / kSortTile);
-    return (tiles + 1) * (size_t{1} << kSortDigitBits) * sizeof(uint32_t);
-}
+constexpr int64_t kSortMinNnz = int64_t{1} << 17;
+size_t CscSortTempBytes(int64_t nnz);
 struct CscSort {
     const int32_t* col;
     int64_t col_stride;
@@ -489,10 +486,11 @@ struct CscSort {
     bool rowptr64;
     int32_t *key, *val;   // results: the columns (cols for entries outside the matrix) in order, their CSR positions
     int32_t *key_tmp, *val_tmp;
-    void* temp;           // CscSortTempBytes
-    const uint32_t* gate; // non-null: a device word; nothing is written when it reads 1
+    void* temp;           // CscSortTempBytes (+ 256: re-aligned to 256 bytes at use)
+    size_t temp_bytes;
+    const uint32_t* gate; // non-null (kSortMinNnz entries at least): a device word; nothing is written when it reads 1
 };
-void LaunchCscSort(const CscSort& c, void* stream);
+int LaunchCscSort(const CscSort& c, void* stream);
 
 // Entries per group of the transpose's compact row table (one wave of 4 entries per lane).
 constexpr int64_t kRowGroup = 256;

@@ -12,11 +12,17 @@
 // path decision (taken on the device) does not need the CSC pattern skips the
 // sort without the host knowing.
 //
+// Below kSortMinNnz entries a tile or a few leave the chip idle and hipCUB's
+// sort of so few pairs is faster (a transposed call with its set-up: 30 000
+// entries 77 µs on hipCUB, 98 on the tiles; 100 000: 96 and 102; 500 000: 181
+// and 119), so those sizes keep it.
+//
 // Bound: HBM traffic, 12 bytes per entry in the first pass (the column twice,
 // one pair written less the position read) and 20 in the others.
 // Reference counterpart: sparse/spmv/arch35/spmv_kernel.cpp:861-879 orders its
 // deterministic transpose by column.
 #include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>
 
 #include <cstdint>
 
@@ -263,6 +269,27 @@ __global__ __launch_bounds__(kSortThreads) void SortScatterKernel(SortParams q)
     }
 }
 
+// Keys and positions of a small matrix, for hipCUB's sort (key_out, val_out).
+template <typename RowT>
+__global__ __launch_bounds__(kSortThreads) void SortKeysKernel(SortParams q)
+{
+    int64_t first, last;
+    RowRange<RowT, true>(q, first, last);
+    const int64_t k = static_cast<int64_t>(blockIdx.x) * kSortThreads + threadIdx.x;
+    if (k >= q.nnz) return;
+    q.key_out[k] = static_cast<int32_t>(KeyAt<RowT, true>(q, k, first, last));
+    q.val_out[k] = static_cast<int32_t>(k);
+}
+
+// (size query when temp is null)
+hipError_t SmallSort(void* temp, size_t& bytes, const SortParams& q, int32_t* key, int32_t* val, int bits,
+                     hipStream_t s)
+{
+    return hipcub::DeviceRadixSort::SortPairs(temp, bytes, static_cast<const int32_t*>(q.key_out), key,
+                                              static_cast<const int32_t*>(q.val_out), val, static_cast<int>(q.nnz), 0,
+                                              bits, s);
+}
+
 template <typename RowT, bool kFirst>
 void Pass(const SortParams& q, hipStream_t s)
 {
@@ -274,9 +301,24 @@ void Pass(const SortParams& q, hipStream_t s)
 
 }  // namespace
 
-void LaunchCscSort(const CscSort& c, void* stream)
+size_t CscSortTempBytes(int64_t nnz)
 {
-    if (c.nnz <= 0) return;
+    if (nnz >= kSortMinNnz) {
+        const size_t tiles = static_cast<size_t>((nnz + kSortTile - 1) / kSortTile);
+        return (tiles + 1) * kDigits * sizeof(uint32_t);
+    }
+    size_t bytes = 0;
+    SortParams q{};
+    q.nnz = nnz;
+    if (SmallSort(nullptr, bytes, q, nullptr, nullptr, 31, nullptr) != hipSuccess) {
+        bytes = static_cast<size_t>(nnz) * 16 + (1 << 20);  // no device to ask: a generous bound
+    }
+    return bytes;
+}
+
+int LaunchCscSort(const CscSort& c, void* stream)
+{
+    if (c.nnz <= 0) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     SortParams q{};
     q.col = c.col;
@@ -292,6 +334,16 @@ void LaunchCscSort(const CscSort& c, void* stream)
     q.gate = c.gate;
     int bits = 1;  // keys are 0 .. cols
     while (bits < 31 && (int64_t{1} << bits) <= c.cols) ++bits;
+    if (c.nnz < kSortMinNnz) {
+        q.key_out = c.key_tmp;
+        q.val_out = c.val_tmp;
+        const dim3 grid(static_cast<unsigned>((c.nnz + kSortThreads - 1) / kSortThreads));
+        if (c.rowptr64) hipLaunchKernelGGL(SortKeysKernel<int64_t>, grid, dim3(kSortThreads), 0, s, q);
+        else hipLaunchKernelGGL(SortKeysKernel<int32_t>, grid, dim3(kSortThreads), 0, s, q);
+        void* temp = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(c.temp) + 255) & ~uintptr_t{255});
+        size_t bytes = c.temp_bytes;
+        return SmallSort(temp, bytes, q, c.key, c.val, bits, s) == hipSuccess ? 0 : 1;
+    }
     const int passes = (bits + kSortDigitBits - 1) / kSortDigitBits;
     for (int p = 0; p < passes; ++p) {
         const int w = bits / passes + (p < bits % passes ? 1 : 0);
@@ -306,6 +358,7 @@ void LaunchCscSort(const CscSort& c, void* stream)
         else Pass<int32_t, true>(q, s);
         q.shift += w;
     }
+    return 0;
 }
 
 }  // namespace aclsp

@@ -340,9 +340,15 @@ constexpr int kWaveRows = static_cast<int>(kMaxRowsPerBlock);
 // eight were slower.  Without Preprocess the power-law c3 takes 2.08 ms
 // against 2.04 ms with four.
 constexpr int kFlatWaves = 1;
-// Block workgroups of the stream kernel when the staged path may take the
-// matrix instead (multiple of the XCD count).
-constexpr int64_t kStagedFallbackWgs = 2048;
+// Most block workgroups (of one wave) of a stream kernel launched while the
+// path choice is not on the host, multiples of the XCD count: every wave slot
+// of the chip when the staged or bucketed kernels may take the matrix instead
+// (2048 made the kernel slow where it did run: a first product of 3 M random
+// entries 28 µs longer, 7.2 M 46; 32768 made the launches that only exit cost
+// 8 µs each), and four times that when the choice is only between the row
+// kernels (7.2 M random entries, a call with its set-up: 133 -> 123 µs).
+constexpr int64_t kFallbackWgs = 32768;
+constexpr int64_t kStagedFallbackWgs = 8192;
 
 static_assert(kLaneItems == 8, "the reductions are written for 8 slots per lane");
 static_assert(kWaveRows <= 2 * kWave - 1, "two rows per lane");
@@ -2511,8 +2517,9 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
                 // the flags of paths whose kernels are not launched here.
                 p.skip_flag = &At<SpmvWsHeader>(l.ws, 0)->staged_flag;
                 p.run_mask = 1U | (l.staged ? 0U : 2U) | (narrow ? 0U : (1U << kNarrowFlag) | (1U << kEntryFlag));
-                if (blockWgs > kStagedFallbackWgs) {
-                    blockWgs = kStagedFallbackWgs;
+                const int64_t cap = l.staged ? kStagedFallbackWgs : kFallbackWgs;
+                if (blockWgs > cap) {
+                    blockWgs = cap;
                     p.block_stride = blockWgs * kFlatWaves;
                 }
             }
@@ -2585,8 +2592,7 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
 
 // Grid of a stream kernel without task waves: one wave per row block, or,
 // when the launch may exit on the path flag, at most kStagedFallbackWgs
-// workgroups whose waves loop over the blocks (22 000 workgroups that only
-// read the flag took 5.7 µs a launch).
+// workgroups whose waves loop over the blocks.
 unsigned FlatGrid(RowBlockParams& c)
 {
     int64_t wgs = ((c.num_blocks + kFlatWaves - 1) / kFlatWaves + kXcds - 1) / kXcds * kXcds;
@@ -3212,13 +3218,24 @@ __global__ __launch_bounds__(kCheckThreads) void NarrowColKernel(NarrowParams q)
     CheckBlocks(entry ? q.num_eblocks : q.num_blocks, q.bad, [&](int64_t b, int lane) {
         const int64_t rb = static_cast<int64_t>(blocks[b]) + q.base;
         const int64_t k1 = static_cast<int64_t>(bn[b + 1]);
-        bool bad = false;
-        for (int64_t k = static_cast<int64_t>(bn[b]) + lane; k < k1; k += kWave) {
-            const int64_t d = static_cast<int64_t>(q.col[k]) - rb;
-            bad |= d < -32768 || d > 32767;
-            q.nc[k] = static_cast<int16_t>(d);
+        // a chunk of the block at a time, its loads in flight together, until
+        // one has a misfit (a row of 200 000 scattered entries, one load and
+        // test after the other to its end, took 0.9 ms)
+        constexpr int kPer = kWaveChunk / kWave;
+        for (int64_t k0 = static_cast<int64_t>(bn[b]) + lane; k0 - lane < k1; k0 += kWaveChunk) {  // wave-uniform
+            int32_t c[kPer];
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) c[u] = q.col[k0 + u * kWave < k1 ? k0 + u * kWave : k1 - 1];
+            bool bad = false;
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int64_t d = static_cast<int64_t>(c[u]) - rb;
+                bad |= d < -32768 || d > 32767;
+                if (k0 + u * kWave < k1) q.nc[k0 + u * kWave] = static_cast<int16_t>(d);
+            }
+            if (__ballot(bad) != 0) return true;
         }
-        return bad;
+        return false;
     });
 }
 
@@ -3464,7 +3481,7 @@ __global__ void CbandDecideKernel(const uint32_t* far, const uint32_t* narrowBad
 // The CSC pattern and its row-block partition; with gate, unless *gate reads
 // 1 when they run.
 template <typename RowT>
-void BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
+int BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
 {
     const int64_t nnz = l.nnz;
     CscSort c{};
@@ -3484,8 +3501,9 @@ void BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
     c.val = c.rowptr64 ? b : a;
     c.val_tmp = c.rowptr64 ? a : b;
     c.temp = At<void>(l.ws, l.layout.sort_offset);
+    c.temp_bytes = l.layout.sort_bytes;
     c.gate = gate;
-    LaunchCscSort(c, s);
+    if (LaunchCscSort(c, s) != 0) return 1;
     const int64_t finishWaves = (nnz + kFinishSpan - 1) / kFinishSpan;
     hipLaunchKernelGGL((CscFinishKernel<RowT>),
                        dim3(static_cast<unsigned>(finishWaves < kFinishWgs ? finishWaves : kFinishWgs)),
@@ -3513,6 +3531,7 @@ void BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
     const int64_t n = (l.cols > pp.num_blocks ? l.cols : pp.num_blocks) + 1;
     hipLaunchKernelGGL((SpmvPreprocessKernel<RowT>), dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, s, pp);
+    return 0;
 }
 
 }  // namespace
@@ -3677,7 +3696,7 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
         hipLaunchKernelGGL((SpmvPreprocessKernel<int64_t>), dim3(grid), dim3(kThreads), 0, s, p);
         if (l.layout.csc) {
             if (l.staged && LaunchStagedPreprocess(l, stream) != 0) return 1;
-            BuildCsc<int64_t>(l, cscGate, s);
+            if (BuildCsc<int64_t>(l, cscGate, s) != 0) return 1;
             return 0;
         }
         if (l.layout.tasks && BuildTasks<int64_t>(l, s) != 0) return 1;
@@ -3688,7 +3707,7 @@ int LaunchSpmvPreprocess(const SpmvLaunch& l, void* stream)
         hipLaunchKernelGGL((SpmvPreprocessKernel<int32_t>), dim3(grid), dim3(kThreads), 0, s, p);
         if (l.layout.csc) {
             if (l.staged && LaunchStagedPreprocess(l, stream) != 0) return 1;
-            BuildCsc<int32_t>(l, cscGate, s);
+            if (BuildCsc<int32_t>(l, cscGate, s) != 0) return 1;
             if (l.cband && l.layout.cband) {
                 SpmvWsHeader* h = At<SpmvWsHeader>(l.ws, 0);
                 hipLaunchKernelGGL(CbandRowKernel, dim3(GridFor(l.nnz) < kCbandWgs ? GridFor(l.nnz) : kCbandWgs), dim3(kCheckThreads), 0, s,

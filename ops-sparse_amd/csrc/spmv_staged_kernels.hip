@@ -1166,7 +1166,7 @@ __device__ __forceinline__ uint32_t BtKey(const StageParams& q, bool inRows, int
 // metric[t] = the tile's non-empty runs (low kBtRunBits bits) and, above them,
 // its entries when its rows average more than kBtLongRows of them.
 constexpr int kBtRunBits = 12;
-constexpr int kBtLongRows = 256;
+constexpr int kBtLongRows = 64;
 static_assert(kBtMaxBuckets < 1 << kBtRunBits && kWide < 1 << (32 - kBtRunBits), "metric fields");
 template <typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
