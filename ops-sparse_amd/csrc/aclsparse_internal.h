@@ -179,7 +179,10 @@ struct SpmvWsHeader {
     // (some block of more than 127 rows, or whose rows run past its window);
     // complex64 transposes: nonzero when some entry's offsets exceed 16 bits
     uint32_t entry_bad;
-    uint32_t reserved[6];
+    // matrices below kSmallNnz entries: nonzero when some row has more than
+    // SmallRowLimit entries (the row-block code then takes the matrix)
+    uint32_t long_rows;
+    uint32_t reserved[5];
 };
 static_assert(sizeof(SpmvWsHeader) <= kWsHeaderBytes, "header must fit 192 bytes");
 
@@ -303,6 +306,18 @@ struct SpmvLayout {
 #define SPMV_LONG_CHUNKS 4
 #endif
 constexpr int64_t kLongChunks = SPMV_LONG_CHUNKS;  // blocks with more chunks than this are split into tasks
+
+// Small matrices (fp32 compute, opA = N): below kSmallNnz entries, and unless
+// Preprocess finds a row of more than SmallRowLimit entries, the row kernel
+// gives each row 2^SmallLanes lanes of four entries a turn.
+constexpr int64_t kSmallNnz = int64_t{1} << 19;
+inline int32_t SmallLanes(int64_t rows, int64_t nnz)
+{
+    int32_t lg = 0;  // a turn covers one and a half mean rows
+    while (lg < 6 && (int64_t{4} << lg) * 2 * rows < 3 * nnz) ++lg;
+    return lg;
+}
+inline int64_t SmallRowLimit(int64_t rows, int64_t nnz) { return int64_t{16} << SmallLanes(rows, nnz); }
 
 // Exclusive-scan temporary storage of the task table (implemented in spmv_kernels.hip).
 size_t TaskScanTempBytes(int64_t n);

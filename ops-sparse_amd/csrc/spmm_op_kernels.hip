@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 #include <utility>
 
 #include "aclsparse_internal.h"
@@ -136,6 +137,7 @@ struct MmParams {
     int32_t b_vec;       // rows of op(B) can be read J elements at a time
     int32_t c_row;       // C(i, j) = c[i*ldc + j]; else c[j*ldc + i]
     int32_t c_vec;
+    int32_t lds_rows;    // LDS kernels: rows per wave
     int32_t has_b;       // k > 0: op(B) has rows to read
     int32_t b_ubuf;      // fp32 rows of op(B) read as 16-byte buffer loads from any 4-byte
                          // boundary (widths not a multiple of 4, or rows not 16-byte aligned);
@@ -226,8 +228,10 @@ __device__ __forceinline__ void SpmmLoad(const MmParams& p, const typename Elem<
     }
 }
 
-// Adds a batch's products into the sums, in entry order.
-template <bool kKahan, int J>
+// Adds a batch's products into the sums, in entry order (kHalf: fp16 values
+// and op(B), whose products are exact in fp32, so that one fused
+// multiply-add rounds as the multiply and the add do).
+template <bool kKahan, int J, bool kHalf>
 __device__ __forceinline__ void SpmmAccum(const int32_t cc[kU], const float vv[kU], const float bv[kU][J],
                                           float acc[J], float comp[J])
 {
@@ -236,6 +240,11 @@ __device__ __forceinline__ void SpmmAccum(const int32_t cc[kU], const float vv[k
         const bool take = cc[q] >= 0;  // skipped entries leave the sums untouched
 #pragma unroll
         for (int t = 0; t < J; ++t) {
+            if constexpr (kHalf && !kKahan) {
+                const float s2 = __builtin_fmaf(vv[q], bv[q][t], acc[t]);
+                acc[t] = take ? s2 : acc[t];
+                continue;
+            }
             const float prod = vv[q] * bv[q][t];
             if constexpr (kKahan) {
                 const float y = prod - comp[t];
@@ -295,10 +304,10 @@ __device__ __forceinline__ void SpmmStore(const MmParams& p, typename Elem<kHalf
                                                static_cast<int>((row * p.ldc + j0) * 4), 0, 0);
     } else if (p.c_row) {
         T* crow = c + row * p.ldc;
-        if (p.c_vec && j0 + J <= p.n && !kHalf) {
+        if (p.c_vec && j0 + J <= p.n) {
             Vec<T, J> wv;
 #pragma unroll
-            for (int q = 0; q < J; ++q) wv.v[q] = out[q];
+            for (int q = 0; q < J; ++q) Elem<kHalf>::Store(wv.v, q, out[q]);
             *reinterpret_cast<Vec<T, J>*>(crow + j0) = wv;
         } else {
 #pragma unroll
@@ -436,7 +445,7 @@ void SpmmOpKernel(MmParams p)
                     cc[q] = q < cnt ? cq : -1;
                 }
                 SpmmLoad<kHalf, J>(p, b, fast ? jf : j0, fast, strided, cc, bv);
-                SpmmAccum<kKahan, J>(cc, vv, bv, acc, comp);
+                SpmmAccum<kKahan, J, kHalf>(cc, vv, bv, acc, comp);
             }
         } else
         for (int64_t e0 = rs; e0 < re; e0 += g) {
@@ -455,7 +464,7 @@ void SpmmOpKernel(MmParams p)
                 if constexpr (kWave) SpmmFetchWave(myc, myv, u0, cnt, cc, vv);
                 else SpmmFetch(myc, myv, gbase, g, u0, cnt, cc, vv);
                 SpmmLoad<kHalf, J>(p, b, fast ? jf : j0, fast, strided, cc, bv);
-                SpmmAccum<kKahan, J>(cc, vv, bv, acc, comp);
+                SpmmAccum<kKahan, J, kHalf>(cc, vv, bv, acc, comp);
             }
         }
         if (live) SpmmStore<kHalf, J>(p, c, row, j0, acc, alpha, beta, betaZero, old);
@@ -470,12 +479,13 @@ void SpmmOpKernel(MmParams p)
 constexpr int kLdsBytes = 64 * 1024;
 constexpr int kLdsWideBytes = 128 * 1024;  // J = 4 tiles without compensation
 constexpr int kLdsThreads = 1024;  // 16 waves share one staged tile
-constexpr int kLdsRowsPerWave = 4;
+constexpr int kLdsMaxRows = 4;  // rows per wave (MmParams::lds_rows: 1, 2 or 4)
 
-template <typename RowT, bool kHalf, bool kKahan, int J>
+template <typename RowT, bool kKahan, int J>
 __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))) void SpmmOpLdsKernel(MmParams p)
 {
-    using T = typename Elem<kHalf>::T;
+    using T = float;
+    constexpr bool kHalf = false;
     extern __shared__ float sB[];
     constexpr int TW = kMmWave * J;
     const RowT* rp = static_cast<const RowT*>(p.rp);
@@ -495,19 +505,19 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int r = idx / TW, cj = idx - r * TW;
             const int64_t j = jt + cj;
-            sB[idx] = j < p.n ? Elem<kHalf>::Load(b, static_cast<int64_t>(r) * p.ldb + j) : 0.0f;
+            sB[idx] = j < p.n ? b[static_cast<int64_t>(r) * p.ldb + j] : 0.0f;
         }
     } else {
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int cj = idx / k, r = idx - cj * k;
             const int64_t j = jt + cj;
-            sB[r * TW + cj] = j < p.n ? Elem<kHalf>::Load(b, j * p.ldb + r) : 0.0f;
+            sB[r * TW + cj] = j < p.n ? b[j * p.ldb + r] : 0.0f;
         }
     }
     __syncthreads();
     const int64_t j0 = jt + lane * J;
-    const int64_t row0 = (chunk * (kLdsThreads / kMmWave) + wv) * kLdsRowsPerWave;
-    for (int rr = 0; rr < kLdsRowsPerWave; ++rr) {
+    const int64_t row0 = (chunk * (kLdsThreads / kMmWave) + wv) * p.lds_rows;
+    for (int rr = 0; rr < p.lds_rows; ++rr) {
         const int64_t row = row0 + rr;
         if (row >= p.m) break;
         // the row's entries are read 64 at a time, one per lane, and handed out
@@ -562,7 +572,7 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))
                         }
                     }
                 } else {
-                    SpmmAccum<kKahan, J>(cc, vv, bv, acc, comp);
+                    SpmmAccum<kKahan, J, kHalf>(cc, vv, bv, acc, comp);
                 }
             }
         }
@@ -570,17 +580,25 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))
     }
 }
 
-// Stages op(B)[0:k, jt:jt+TW] in LDS as fp32 (row r at sB[r*TW]; columns past
-// n read as 0).  Full tiles of a row-major op(B) whose rows start on a
-// 4-element boundary move 4 elements per load, four loads in flight per
-// thread; other tiles element by element.
-template <bool kHalf, int TW>
-__device__ __forceinline__ void StageBTile(const MmParams& p, const typename Elem<kHalf>::T* b, float* sB, int64_t jt,
+// Stages op(B)[0:k, jt:jt+TW] in LDS (row r at sB[r*TW]; columns past n read
+// as 0) as fp32, or as fp16 when L is uint16_t.  Tiles of a
+// row-major op(B) whose rows start on a 4-element boundary, and whose columns
+// inside it are a multiple of 4, move 4 elements per load, four loads in
+// flight per thread; other tiles element by element.
+template <bool kHalf, int TW, typename L>
+__device__ __forceinline__ void StageBTile(const MmParams& p, const typename Elem<kHalf>::T* b, L* sB, int64_t jt,
                                           int k)
 {
     using T = typename Elem<kHalf>::T;
-    if (p.b_contig && p.b_vec && jt + TW <= p.n) {
+    constexpr bool kRaw = std::is_same<T, L>::value;  // LDS holds op(B)'s own type
+    const auto load = [&](int64_t i) {
+        if constexpr (kRaw) return b[i];
+        else return Elem<kHalf>::Load(b, i);
+    };
+    const int64_t left = p.n - jt;  // columns of the tile inside op(B)
+    if (p.b_contig && p.b_vec && (left >= TW || left % 4 == 0)) {
         constexpr int kQ = TW / 4;  // 4-element groups per staged row
+        const int inside = left >= TW ? kQ : static_cast<int>(left / 4);
         const int total = k * kQ;
         for (int i0 = static_cast<int>(threadIdx.x); i0 < total; i0 += 4 * kLdsThreads) {
             Vec<T, 4> w[4];
@@ -588,20 +606,21 @@ __device__ __forceinline__ void StageBTile(const MmParams& p, const typename Ele
             for (int u = 0; u < 4; ++u) {
                 const int idx = i0 + u * kLdsThreads;
                 const int r = idx < total ? idx / kQ : 0, q = idx < total ? idx % kQ : 0;
-                w[u] = *reinterpret_cast<const Vec<T, 4>*>(b + static_cast<int64_t>(r) * p.ldb + jt + 4 * q);
+                w[u] = *reinterpret_cast<const Vec<T, 4>*>(b + static_cast<int64_t>(r) * p.ldb + jt +
+                                                           4 * (q < inside ? q : 0));
+                if (q >= inside) w[u] = Vec<T, 4>{};
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int idx = i0 + u * kLdsThreads;
                 if (idx < total) {
-                    float4 f;
-                    if constexpr (kHalf) {
-                        f = make_float4(Half2Float(w[u].v[0]), Half2Float(w[u].v[1]), Half2Float(w[u].v[2]),
-                                        Half2Float(w[u].v[3]));
-                    } else {
-                        f = make_float4(w[u].v[0], w[u].v[1], w[u].v[2], w[u].v[3]);
+                    Vec<L, 4> f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (kRaw) f.v[e] = w[u].v[e];
+                        else f.v[e] = Half2Float(w[u].v[e]);
                     }
-                    *reinterpret_cast<float4*>(&sB[(idx / kQ) * TW + 4 * (idx % kQ)]) = f;
+                    *reinterpret_cast<Vec<L, 4>*>(&sB[(idx / kQ) * TW + 4 * (idx % kQ)]) = f;
                 }
             }
         }
@@ -609,13 +628,13 @@ __device__ __forceinline__ void StageBTile(const MmParams& p, const typename Ele
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int r = idx / TW, cj = idx - r * TW;
             const int64_t j = jt + cj;
-            sB[idx] = j < p.n ? Elem<kHalf>::Load(b, static_cast<int64_t>(r) * p.ldb + j) : 0.0f;
+            sB[idx] = j < p.n ? load(static_cast<int64_t>(r) * p.ldb + j) : L{0};
         }
     } else {
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int cj = idx / k, r = idx - cj * k;
             const int64_t j = jt + cj;
-            sB[r * TW + cj] = j < p.n ? Elem<kHalf>::Load(b, j * p.ldb + r) : 0.0f;
+            sB[r * TW + cj] = j < p.n ? load(j * p.ldb + r) : L{0};
         }
     }
 }
@@ -630,9 +649,13 @@ __device__ __forceinline__ int RowBcast(int v)
 
 // Entry Q of a batch of 16 held by lanes 0..15 of every 16-lane row (byte
 // offset of its op(B) row in LDS, with the sign bit set for a skipped entry,
-// and its value): its products with the lane's J columns added in order.
-template <int J, bool kAll, int Q>
-__device__ __forceinline__ void BcastEntry(const char* sB, uint32_t laneOff, int off, float v, float acc[J])
+// and its value): its products with the lane's J columns added in order.  The
+// product of two fp16 values is exact in fp32 (22 significant bits, exponents
+// well inside), so for them one fused multiply-add rounds exactly as the
+// multiply and the add do: half the arithmetic, and op(B) stays fp16 in LDS
+// (v_fma_mix_f32 reads the half where it lies).
+template <int J, bool kAll, int Q, typename L>
+__device__ __forceinline__ void BcastEntry(const L* sB, uint32_t laneOff, int off, float v, float acc[J])
 {
     bool take = true;
     int o;
@@ -643,17 +666,19 @@ __device__ __forceinline__ void BcastEntry(const char* sB, uint32_t laneOff, int
         take = o >= 0;
         o &= 0x7FFFFFFF;  // a skipped entry reads row 0
     }
-    const Vec<float, J> w = *reinterpret_cast<const Vec<float, J>*>(sB + (o + laneOff));
+    const Vec<L, J> w = *reinterpret_cast<const Vec<L, J>*>(reinterpret_cast<const char*>(sB) + (o + laneOff));
     const float vq = __int_as_float(RowBcast<Q>(__float_as_int(v)));
 #pragma unroll
     for (int t = 0; t < J; ++t) {
-        const float s2 = acc[t] + vq * w.v[t];
+        float s2;
+        if constexpr (sizeof(L) == 2) s2 = __builtin_fmaf(Half2Float(w.v[t]), vq, acc[t]);
+        else s2 = acc[t] + vq * w.v[t];
         acc[t] = take ? s2 : acc[t];
     }
 }
 
-template <int J, bool kAll, int... Q>
-__device__ __forceinline__ void BcastBatch(std::integer_sequence<int, Q...>, const char* sB, uint32_t laneOff, int off,
+template <int J, bool kAll, typename L, int... Q>
+__device__ __forceinline__ void BcastBatch(std::integer_sequence<int, Q...>, const L* sB, uint32_t laneOff, int off,
                                            float v, float acc[J])
 {
     (BcastEntry<J, kAll, Q>(sB, laneOff, off, v, acc), ...);
@@ -661,8 +686,8 @@ __device__ __forceinline__ void BcastBatch(std::integer_sequence<int, Q...>, con
 
 // Entries first..15 of a batch whose columns are all in range (a row's last
 // batch holds its entries in the top slots): wave-uniform branches, no selects.
-template <int J, int Q>
-__device__ __forceinline__ void BcastFrom(int first, const char* sB, uint32_t laneOff, int off, float v, float acc[J])
+template <int J, int Q, typename L>
+__device__ __forceinline__ void BcastFrom(int first, const L* sB, uint32_t laneOff, int off, float v, float acc[J])
 {
     if (first <= Q) BcastEntry<J, true, Q>(sB, laneOff, off, v, acc);
     if constexpr (Q < 15) BcastFrom<J, Q + 1>(first, sB, laneOff, off, v, acc);
@@ -675,13 +700,16 @@ __device__ __forceinline__ void BcastFrom(int first, const char* sB, uint32_t la
 // Per entry and lane: one address add, one LDS read of J columns, J
 // multiplies and J adds.  Same tiles, rows and sums as SpmmOpLdsKernel.
 template <typename RowT, bool kHalf, int J>
-__global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(J >= 4 ? 4 : 8))) void SpmmOpLdsBcastKernel(MmParams p)
+__global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(J >= 4 && !kHalf ? 4 : 8)))
+void SpmmOpLdsBcastKernel(MmParams p)
 {
     using T = typename Elem<kHalf>::T;
-    extern __shared__ float sB[];
+    extern __shared__ float sBRaw[];
+    T* sB = reinterpret_cast<T*>(sBRaw);
+    constexpr int kEsz = static_cast<int>(sizeof(T));
     constexpr int TW = kMmWave * J;
     constexpr int kBatch = 16;
-    constexpr int kWindow = J >= 4 ? 5 : 4;  // batches loaded together (J = 4: rows of up to 80 entries in one)
+    constexpr int kWindow = J >= 4 && !kHalf ? 5 : 4;  // batches loaded together (J = 4: rows of up to 80 entries in one)
     const T* val = static_cast<const T*>(p.val);
     const T* b = static_cast<const T*>(p.b);
     T* c = static_cast<T*>(p.c);
@@ -695,9 +723,8 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(J >
     const int64_t chunk = static_cast<int64_t>(blockIdx.x) / p.tiles;
     const int64_t jt = tile * TW;
     const int k = static_cast<int>(p.k);
-    const int64_t row0 = (chunk * (kLdsThreads / kMmWave) + wv) * kLdsRowsPerWave;
-    const int nRows = static_cast<int>(p.m - row0 < kLdsRowsPerWave ? (p.m - row0 > 0 ? p.m - row0 : 0)
-                                                                     : kLdsRowsPerWave);
+    const int64_t row0 = (chunk * (kLdsThreads / kMmWave) + wv) * p.lds_rows;
+    const int nRows = static_cast<int>(p.m - row0 < p.lds_rows ? (p.m - row0 > 0 ? p.m - row0 : 0) : p.lds_rows);
     // A window of kWindow batches: lane sub of every 16-lane row holds slot
     // sub of each batch; a batch's entries fill its slots first..15.
     struct Window {
@@ -717,14 +744,13 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(J >
                 ci = p.col[e] - p.base;
                 x = Elem<kHalf>::Load(val, e);
             }
-            w.off[q] = ci >= 0 && ci < k ? ci * (TW * 4) : static_cast<int>(0x80000000U);
+            w.off[q] = ci >= 0 && ci < k ? ci * (TW * kEsz) : static_cast<int>(0x80000000U);
             w.v[q] = x;
         }
     };
     StageBTile<kHalf, TW>(p, b, sB, jt, k);
     __syncthreads();
-    const char* sBytes = reinterpret_cast<const char*>(sB);
-    const uint32_t laneOff = static_cast<uint32_t>(lane * J * 4);
+    const uint32_t laneOff = static_cast<uint32_t>(lane * J * kEsz);
     const int64_t j0 = jt + lane * J;
     for (int rr = 0; rr < nRows; ++rr) {
         const int64_t row = row0 + rr;
@@ -745,13 +771,13 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(J >
                 if (cur.first[q] == kBatch) break;  // wave-uniform: no entries left
                 if (__ballot(cur.off[q] < 0 && sub >= cur.first[q]) == 0) {  // every entry of the batch taken
                     if (cur.first[q] == 0) {
-                        BcastBatch<J, true>(std::make_integer_sequence<int, kBatch>{}, sBytes, laneOff, cur.off[q],
+                        BcastBatch<J, true>(std::make_integer_sequence<int, kBatch>{}, sB, laneOff, cur.off[q],
                                             cur.v[q], acc);
                     } else {
-                        BcastFrom<J, 0>(cur.first[q], sBytes, laneOff, cur.off[q], cur.v[q], acc);
+                        BcastFrom<J, 0>(cur.first[q], sB, laneOff, cur.off[q], cur.v[q], acc);
                     }
                 } else {
-                    BcastBatch<J, false>(std::make_integer_sequence<int, kBatch>{}, sBytes, laneOff, cur.off[q],
+                    BcastBatch<J, false>(std::make_integer_sequence<int, kBatch>{}, sB, laneOff, cur.off[q],
                                          cur.v[q], acc);
                 }
             }
@@ -813,39 +839,83 @@ void Dispatch(const MmParams& p, int J, bool kahan, unsigned grid, hipStream_t s
 #undef SPMM_NARROW
 }
 
+// Dynamic LDS beyond 64 KiB: gfx950 allows 160 KiB per workgroup; the
+// attribute is set once, and a runtime that does not need it may decline it
+// (the launch reports real failures).
+template <typename RowT, bool kHalf>
+void AllowWideLds()
+{
+    static const bool once = [] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&SpmmOpLdsBcastKernel<RowT, kHalf, 4>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsWideBytes));
+        (void)hipGetLastError();
+        return true;
+    }();
+    (void)once;
+}
+
 template <typename RowT, bool kHalf>
 void DispatchLds(const MmParams& p, int J, bool kahan, unsigned grid, unsigned lds, hipStream_t s)
 {
 #define SPMM_LDS(JJ, KK) \
-    hipLaunchKernelGGL((SpmmOpLdsKernel<RowT, kHalf, KK, JJ>), dim3(grid), dim3(kLdsThreads), lds, s, p)
+    hipLaunchKernelGGL((SpmmOpLdsKernel<RowT, KK, JJ>), dim3(grid), dim3(kLdsThreads), lds, s, p)
 #define SPMM_BCAST(JJ) \
     hipLaunchKernelGGL((SpmmOpLdsBcastKernel<RowT, kHalf, JJ>), dim3(grid), dim3(kLdsThreads), lds, s, p)
-    if (kahan && !kHalf) {
-        if (J == 4) SPMM_LDS(4, true);
-        else if (J == 2) SPMM_LDS(2, true);
-        else SPMM_LDS(1, true);
-    } else if (lds > static_cast<unsigned>(kLdsBytes)) {  // J = 4 over up to 128 KiB: one workgroup per CU
-        // gfx950 allows 160 KiB per workgroup; the attribute is set once, and
-        // a runtime that does not need it may decline it (the launch reports
-        // real failures)
-        static const bool once = [] {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&SpmmOpLdsBcastKernel<RowT, kHalf, 4>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsWideBytes));
-            (void)hipGetLastError();
-            return true;
-        }();
-        (void)once;
+    if constexpr (kHalf) {  // fp16 tiles: J = 4 for every k (up to 128 KiB)
+        AllowWideLds<RowT, true>();
         SPMM_BCAST(4);
     } else {
-        if (J == 4) SPMM_LDS(4, false);  // (the broadcast kernel spills at J = 4 and eight waves per SIMD)
-        else if (J == 2) SPMM_BCAST(2);
-        else SPMM_BCAST(1);
+        if (kahan) {
+            if (J == 4) SPMM_LDS(4, true);
+            else if (J == 2) SPMM_LDS(2, true);
+            else SPMM_LDS(1, true);
+        } else if (lds > static_cast<unsigned>(kLdsBytes)) {  // J = 4 over up to 128 KiB: one workgroup per CU
+            AllowWideLds<RowT, false>();
+            SPMM_BCAST(4);
+        } else {
+            if (J == 4) SPMM_LDS(4, false);  // (the broadcast kernel spills at J = 4 and eight waves per SIMD)
+            else if (J == 2) SPMM_BCAST(2);
+            else SPMM_BCAST(1);
+        }
     }
 #undef SPMM_LDS
 #undef SPMM_BCAST
 }
 
 bool AlignedTo(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
+
+// Rows per wave of the LDS kernels.  Four, unless that makes fewer than two
+// workgroups per CU; then by their cost in CU cycles: a workgroup stages its
+// tile (about 2000 + 8 cycles per row of op(B)) and works 16 rows at a time
+// (4 waves per SIMD, 4 cycles per instruction and entry), the workgroups go
+// over the chip in rounds of one per CU, and staging hides behind another
+// workgroup when two fit a CU.  Fewer rows make more, smaller workgroups:
+// fuller last rounds, more staging.  Half-dense m x k x n, µs, 4 rows ->
+// chosen: fp16 2048 x 128 x 2048 24.8 -> 23.1 (2 rows), 3983 x 179 x 1196
+// 65 -> 56 (2), 700 x 40 x 300 12.1 -> 10.1 (1); fp32 700 x 40 x 300 26 -> 10
+// (1), 1500 x 100 x 1000 23.5 -> 13.9 (1).  With more workgroups fewer rows
+// only add staging: fp32 4096 x 32 x 2048 41.5 (4 rows), 49.4 (1).
+constexpr int64_t kCus = 256;
+int LdsRows(int64_t m, int64_t nnz, int64_t k, int64_t tiles, int J, bool half, int64_t lds)
+{
+    const int64_t row = 16 * (half ? J + 3 : 2 * J + 2) * (nnz / m + 1);
+    const int64_t stage = 2000 + 8 * k;
+    const int64_t perRound = lds <= 80 * 1024 ? 0 : stage;
+    int best = kLdsMaxRows;
+    int64_t bestCost = INT64_MAX;
+    const int64_t perMax = int64_t{kLdsThreads / kMmWave} * kLdsMaxRows;
+    if ((m + perMax - 1) / perMax * tiles >= 2 * kCus) return kLdsMaxRows;
+    for (int r = 1; r <= kLdsMaxRows; r *= 2) {
+        const int64_t perBlock = int64_t{kLdsThreads / kMmWave} * r;
+        const int64_t blocks = (m + perBlock - 1) / perBlock * tiles;
+        const int64_t cost = (blocks + kCus - 1) / kCus * (r * row + perRound) + stage;
+        if (cost < bestCost) {
+            best = r;
+            bestCost = cost;
+        }
+    }
+    return best;
+}
 
 }  // namespace
 
@@ -885,17 +955,19 @@ int LaunchSpmmOp(const SpmmLaunch& l, void* stream)
     const bool kahan = l.high_precision != 0;
     // small k: op(B) column tiles staged in LDS (n of at least one wave's width)
     if (l.k > 0 && l.n >= kMmWave && l.k * kMmWave * 4 <= kLdsBytes) {
-        const int J = l.k * kMmWave * 4 * 4 <= (kahan ? kLdsBytes : kLdsWideBytes) ? 4
-                      : l.k * kMmWave * 4 * 2 <= kLdsBytes                      ? 2
-                                                                                : 1;
+        const int J = l.fp16                                                        ? 4
+                      : l.k * kMmWave * 4 * 4 <= (kahan ? kLdsBytes : kLdsWideBytes) ? 4
+                      : l.k * kMmWave * 4 * 2 <= kLdsBytes                           ? 2
+                                                                                     : 1;
         const int64_t tw = int64_t{kMmWave} * J;
         p.tiles = (l.n + tw - 1) / tw;
         p.c_vec = l.c_row_major && l.ldc % J == 0 && AlignedTo(l.c, J * esz) ? 1 : 0;
         p.b_vec = l.ldb % 4 == 0 && AlignedTo(l.b, 4 * esz) ? 1 : 0;  // staging 4 elements per load
-        const int64_t rowsPerBlock = int64_t{kLdsThreads / kMmWave} * kLdsRowsPerWave;
+        p.lds_rows = LdsRows(l.m, l.nnz, l.k, p.tiles, J, l.fp16 != 0, l.k * tw * static_cast<int64_t>(esz));
+        const int64_t rowsPerBlock = int64_t{kLdsThreads / kMmWave} * p.lds_rows;
         const int64_t blocks = (l.m + rowsPerBlock - 1) / rowsPerBlock * p.tiles;
         if (blocks <= 0x7FFFFFFF) {
-            const unsigned lds = static_cast<unsigned>(l.k * tw * 4);
+            const unsigned lds = static_cast<unsigned>(l.k * tw * static_cast<int64_t>(esz));
             if (l.rowptr64) {
                 if (l.fp16) DispatchLds<int64_t, true>(p, J, false, static_cast<unsigned>(blocks), lds, s);
                 else DispatchLds<int64_t, false>(p, J, kahan, static_cast<unsigned>(blocks), lds, s);

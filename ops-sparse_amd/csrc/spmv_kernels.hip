@@ -134,6 +134,8 @@ struct RowBlockParams {
     // Stream kernel: when > 0, the grid is capped and each wave loops over
     // the blocks tile, tile + block_stride, ... (block_stride = all block waves)
     int64_t block_stride;
+    int32_t lane_lg;            // small matrices (SmallRows): log2 of the lanes per row
+    const uint32_t* long_rows;  // and the header word that says whether some row is too long for it
 };
 
 // Loads the block's row offsets relative to its first non-zero into LDS.
@@ -1198,16 +1200,90 @@ __device__ __forceinline__ void FixupLongBlock(const RowBlockParams& p, const St
 // is reduced by many waves at once.  Each task stores the partial sums of its
 // chunk-crossing rows; the block's last task to arrive combines them.
 //
+// Small matrices: the rows of a matrix whose launch leaves most of the chip's
+// wave slots idle, 2^lane_lg lanes per row, four entries per lane and turn.  A
+// wave then waits for three dependent round trips (row offsets; columns and
+// values; x) and runs about 150 instructions, where a row block's wave waits
+// for four and runs through some 2000 of straight-line code that every CU
+// has to fetch first.  Where Preprocess found a row of more than four turns
+// (long_rows, read beside the first row offsets) SmallRows returns false and
+// the row-block code takes the matrix.  4096 rows of 41 entries, fp32:
+// SMALL_A -> SMALL_B µs a product; SMALL_C.
+template <typename RowT, ValKind V, OutKind O, bool kBeta>
+__device__ __forceinline__ bool SmallRows(const RowBlockParams& p)
+{
+    using ValT = typename ValOf<V>::T;
+    using OutT = typename OutOf<O>::T;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int g = 1 << p.lane_lg;
+    const int sub = lane & (g - 1);
+    const int64_t rpw = kWave >> p.lane_lg;
+    const RowT* norm = static_cast<const RowT*>(p.rp);
+    OutT* y = static_cast<OutT*>(p.y);
+    const __amdgpu_buffer_rsrc_t rc = Rsrc(p.col, p.nnz * 4);
+    const __amdgpu_buffer_rsrc_t rv = Rsrc(p.val, p.nnz * static_cast<int64_t>(sizeof(ValT)));
+    const __amdgpu_buffer_rsrc_t rx = Rsrc(p.x, p.cols * static_cast<int64_t>(sizeof(ValT)));
+    const uint32_t longRows = ConstLoad<uint32_t>(p.long_rows, 0);
+    float alpha, beta;
+    LoadScalars<AccKind::F32>(p.s, alpha, beta);
+    for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * rpw; r0 < p.rows; r0 += static_cast<int64_t>(gridDim.x) * rpw) {
+        const int64_t row = r0 + (lane >> p.lane_lg);
+        const bool valid = row < p.rows;
+        const int64_t rr = valid ? row : p.rows;
+        const int32_t a = static_cast<int32_t>(norm[rr]);
+        const int32_t b = static_cast<int32_t>(norm[valid ? row + 1 : p.rows]);
+        if (longRows != 0U) return false;  // uniform
+        float old = 0.0f;
+        if constexpr (kBeta) {
+            if (beta != 0.0f && valid && sub == 0) old = OutToAcc<O, AccKind::F32>(y[row]);
+        }
+        float sum = 0.0f;
+        for (int32_t k0 = a + sub; __ballot(k0 < b) != 0; k0 += 4 * g) {
+            int32_t c[4];
+            float v[4], xv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int32_t k = k0 + u * g;
+                c[u] = __builtin_amdgcn_raw_buffer_load_b32(rc, k < b ? k * 4 : -16, 0, 0);
+                if constexpr (sizeof(ValT) == 4) {
+                    v[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, k < b ? k * 4 : -16, 0, 0));
+                } else {
+                    v[u] = ToAcc<V, AccKind::F32>(__builtin_amdgcn_raw_buffer_load_b16(rv, k < b ? k * 2 : -16, 0, 0));
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                uint32_t off = static_cast<uint32_t>(c[u] - p.base) * static_cast<uint32_t>(sizeof(ValT));
+                off = k0 + u * g < b ? off : 0xFFFFFFF0U;  // past the row: no request, reads 0
+                if constexpr (sizeof(ValT) == 4) {
+                    xv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, static_cast<int>(off), 0, 0));
+                } else {
+                    xv[u] = ToAcc<V, AccKind::F32>(__builtin_amdgcn_raw_buffer_load_b16(rx, static_cast<int>(off), 0, 0));
+                }
+            }
+            sum += (v[0] * xv[0] + v[1] * xv[1]) + (v[2] * xv[2] + v[3] * xv[3]);
+        }
+        for (int m = g / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, kWave);
+        if (valid && sub == 0) {
+            StoreRowOld<O, AccKind::F32>(y, row, sum, alpha, beta, kBeta && beta != 0.0f, old);
+        }
+    }
+    return longRows == 0U;  // (waves without rows too)
+}
+
 // kGated: the launch made when another path may have taken the matrix (the
 // decision is on the device only): the kernel exits unless p.skip_flag reads
 // a value whose bit is set in p.run_mask, and a capped grid loops over the
 // blocks (block_stride).  Ungated launches carry neither (one block per wave,
 // no flag load).  kNarrow: column indices from the narrow copy p.ncol.
 template <typename RowT, ValKind V, OutKind O, bool kBeta, bool kGated = false, bool kNarrow = false,
-          bool kEntry = false>
+          bool kEntry = false, bool kSmall = false>
 __global__ __launch_bounds__(kWave* kFlatWaves) __attribute__((amdgpu_waves_per_eu(6)))
 void SpmvStreamFlatKernel(RowBlockParams p)
 {
+    if constexpr (kSmall) {
+        if (SmallRows<RowT, V, O, kBeta>(p)) return;
+    }
     using ValT = typename ValOf<V>::T;
     using OutT = typename OutOf<O>::T;
     using L = StreamLoad<RowT, V, O>;
@@ -2553,7 +2629,26 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
                                            stream_, q);
                     }
                 }
-            } else if (betaNz) {
+                return 0;
+            }
+            if constexpr (!kInt8) {
+                if (l.layout.tasks && p.rows > 0 && l.nnz < kSmallNnz) {
+                    p.lane_lg = SmallLanes(l.rows, l.nnz);
+                    p.long_rows = &At<SpmvWsHeader>(l.ws, 0)->long_rows;
+                    const int64_t rpw = kWave >> p.lane_lg;
+                    const int64_t rowWgs = ((l.rows + rpw - 1) / rpw + kXcds - 1) / kXcds * kXcds;
+                    const unsigned gs = static_cast<unsigned>(rowWgs > g ? (rowWgs < 8192 ? rowWgs : 8192) : g);
+                    if (betaNz) {
+                        hipLaunchKernelGGL((SpmvStreamFlatKernel<RowT, V, O, true, false, false, false, true>), dim3(gs),
+                                           wg, 0, stream_, p);
+                    } else {
+                        hipLaunchKernelGGL((SpmvStreamFlatKernel<RowT, V, O, false, false, false, false, true>),
+                                           dim3(gs), wg, 0, stream_, p);
+                    }
+                    return 0;
+                }
+            }
+            if (betaNz) {
                 hipLaunchKernelGGL((SpmvStreamFlatKernel<RowT, V, O, true>), dim3(g), wg, 0, stream_, p);
             } else {
                 hipLaunchKernelGGL((SpmvStreamFlatKernel<RowT, V, O, false>), dim3(g), wg, 0, stream_, p);
@@ -3060,10 +3155,21 @@ int DispatchTypes(const SpmvLaunch& l, hipStream_t s)
 
 // Task table of the long blocks: counts[b] = chunks of block b when it has
 // more than kLongChunks, else 0 (counts[B] = 0); arrival counters cleared.
+// For small matrices (rows > 0) also *longRows = 1 when a row has more than
+// limit entries.
 template <typename RowT>
 __global__ __launch_bounds__(kThreads) void TaskCountKernel(const RowT* blockNnz, int64_t numBlocks, int32_t* counts,
-                                                            uint32_t* cnt)
+                                                            uint32_t* cnt, const RowT* norm, int64_t rows,
+                                                            int64_t limit, uint32_t* longRows)
 {
+    bool isLong = false;
+    for (int64_t r = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; r < rows;
+         r += static_cast<int64_t>(gridDim.x) * kThreads) {
+        isLong |= static_cast<int64_t>(norm[r + 1]) - static_cast<int64_t>(norm[r]) > limit;
+    }
+    if (__ballot(isLong) != 0 && (threadIdx.x & (kWave - 1)) == 0) {
+        __hip_atomic_fetch_or(longRows, 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     for (int64_t b = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; b <= numBlocks;
          b += static_cast<int64_t>(gridDim.x) * kThreads) {
         int32_t n = 0;
@@ -3088,15 +3194,20 @@ __global__ __launch_bounds__(kThreads) void TaskFillKernel(const int32_t* taskSt
     }
 }
 
+constexpr int kTaskCountWgs = 1024;
+
 template <typename RowT>
 int BuildTasks(const SpmvLaunch& l, hipStream_t s)
 {
     const int64_t nb = l.layout.num_blocks;
     int32_t* counts = At<int32_t>(l.ws, l.layout.task_head_offset);  // temporary: max_tasks >= nb + 1
     int32_t* start = At<int32_t>(l.ws, l.layout.task_start_offset);
-    hipLaunchKernelGGL((TaskCountKernel<RowT>), dim3(GridFor(nb + 1)), dim3(kThreads), 0, s,
-                       At<const RowT>(l.ws, l.layout.block_nnz_offset), nb, counts,
-                       At<uint32_t>(l.ws, l.layout.task_cnt_offset));
+    const int64_t rows = l.nnz < kSmallNnz ? l.rows : 0;  // small matrices: their rows are looked at too
+    const int grid = GridFor(rows > nb + 1 ? rows : nb + 1);
+    hipLaunchKernelGGL((TaskCountKernel<RowT>), dim3(grid < kTaskCountWgs ? grid : kTaskCountWgs), dim3(kThreads), 0,
+                       s, At<const RowT>(l.ws, l.layout.block_nnz_offset), nb, counts,
+                       At<uint32_t>(l.ws, l.layout.task_cnt_offset), At<const RowT>(l.ws, l.layout.rowptr_offset),
+                       rows, SmallRowLimit(l.rows, l.nnz), &At<SpmvWsHeader>(l.ws, 0)->long_rows);
     void* temp = reinterpret_cast<void*>(
         (reinterpret_cast<uintptr_t>(At<uint8_t>(l.ws, l.layout.task_scan_offset)) + 255) & ~uintptr_t{255});
     size_t tempBytes = l.layout.task_scan_bytes;

@@ -438,3 +438,18 @@ def test_bench_laplacian_block_full_size_bit_exact(dev):
     want = oracle.spmm_f32(w.rows, w.cols, n, w.row_ptr.numpy(), w.col_ind.numpy(), w.values.numpy(), 0, b.ravel(), n,
                            1, c0.ravel(), n, 1, 1.5, 0.5)
     np.testing.assert_array_equal(dc.cpu().numpy().ravel().view(np.uint32), want.view(np.uint32))
+
+
+# rows around the LDS kernels' 16, 32 and 64 rows per workgroup, which the launch picks by how full the chip is;
+# k up to their limit of 256; last column tiles of 44 (whole 4-column groups), 1 and 255 columns
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m", [1, 16, 17, 65, 1030, 2300])
+@pytest.mark.parametrize("k,n", [(33, 300), (128, 257), (256, 511), (200, 1024)])
+def test_lds_rows_and_tiles(dev, half, m, k, n):
+    rp, col, val = _rand_csr(m, k, 0.3, m + k, bad_cols=m % 2 == 1, long_rows=True)
+    rng = np.random.default_rng(n)
+    b, c = rng.uniform(-1, 1, k * n), rng.uniform(-1, 1, m * n)
+    for order_b, op_b, pad in ((Order.ROW, Operation.NON_TRANSPOSE, 0), (Order.COL, Operation.NON_TRANSPOSE, 3)):
+        got, want, _ = _run_plan(dev, m, k, n, rp, col, val, b, c, op_b, order_b, Order.ROW, SpMMOpAlg.ALG1, half, 1.25,
+                                 0.5, ldb_pad=pad, ldc_pad=4 * pad)
+        np.testing.assert_array_equal(got, want)

@@ -1019,3 +1019,49 @@ def test_complex_graph_capture_on_chosen_paths(op, dev):
         with torch.cuda.stream(s):
             plan.run()
         torch.cuda.synchronize()
+
+
+# below 2^19 entries each row gets 1 to 64 lanes of four entries a turn, unless some row exceeds four turns
+# (limit = 16 lanes' entries): rows exactly at the limit, one entry past it in the last row, and ragged tails
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("i64,base", [(False, 0), (True, 1)])
+@pytest.mark.parametrize("rows,mean", [(65, 1), (1001, 2), (4099, 5), (3001, 21), (2050, 85), (67, 400)])
+@pytest.mark.parametrize("past", [0, 1])
+def test_small_matrices(dev, dtype, i64, base, rows, mean, past):
+    rng = np.random.default_rng(rows + mean)
+    lens = rng.poisson(mean, rows)
+    lens[::13] = 0
+    lg = 0
+    for _ in range(3):  # the lanes follow from the entry count, which the long row changes
+        lg = next((g for g in range(7) if (4 << g) * 2 * rows >= 3 * int(lens.sum())), 6)
+        lens[-1] = (16 << lg) + past
+        lens[rows // 2] = 16 << lg
+        lens = np.minimum(lens, 16 << lg) if not past else np.concatenate([np.minimum(lens[:-1], 16 << lg), lens[-1:]])
+    cols = max(8, int(lens.max()) // 2)
+    nnz = int(lens.sum())
+    assert nnz < 1 << 19
+    rp = np.concatenate([[0], np.cumsum(lens)]) + base
+    col = rng.integers(0, cols, nnz).astype(np.int32) + base
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(d)  # noqa: E731
+    vals, x = t(rng.uniform(-1, 1, nnz), dtype), t(rng.uniform(-1, 1, cols), dtype)
+    for alpha, beta in ((1.0, 0.0), (-0.5, 2.0)):
+        y0 = t(rng.uniform(-1, 1, rows), dtype) if beta else torch.full((rows,), float("nan"), device=dev).to(dtype)
+        y = y0.clone()
+        plan = CsrSpMV(rows, cols, t(rp, torch.int64 if i64 else torch.int32), t(col, torch.int32), vals, x, y, alpha,
+                       beta, base=base)
+        plan.preprocess()
+        plan.run()
+        torch.cuda.synchronize()
+        long_rows = int(np.frombuffer(plan.workspace[:192].cpu().numpy().tobytes(), dtype=np.uint32)[42])
+        assert long_rows == past
+        v, xs = vals.double().cpu().numpy(), x.double().cpu().numpy()
+        r = np.repeat(np.arange(rows), lens)
+        prod = v * xs[col - base]
+        want = alpha * np.bincount(r, weights=prod, minlength=rows)
+        scale = abs(alpha) * np.bincount(r, weights=np.abs(prod), minlength=rows)
+        if beta:
+            yd = y0.double().cpu().numpy()
+            want, scale = want + beta * yd, scale + abs(beta * yd)
+        eps = {torch.float32: 0.0, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+        err = np.abs(y.double().cpu().numpy() - want)
+        assert np.all(err <= eps * np.abs(want) + 1e-5 * scale + (1e-7 if eps else 0.0))
