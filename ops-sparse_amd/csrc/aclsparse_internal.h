@@ -319,6 +319,22 @@ inline int32_t SmallLanes(int64_t rows, int64_t nnz)
 }
 inline int64_t SmallRowLimit(int64_t rows, int64_t nnz) { return int64_t{16} << SmallLanes(rows, nnz); }
 
+// fn(n) for a fn whose value depends on n alone, or the value of this call
+// site's last call on this thread when n is the same: every product works the
+// layout out again, and asking hipCUB for its temporary storage takes longer
+// than the rest of it.
+template <typename F>
+inline size_t LastResult(int64_t n, F fn)
+{
+    static thread_local int64_t lastN = -1;
+    static thread_local size_t last = 0;
+    if (n != lastN) {
+        last = fn(n);
+        lastN = n;
+    }
+    return last;
+}
+
 // Exclusive-scan temporary storage of the task table (implemented in spmv_kernels.hip).
 size_t TaskScanTempBytes(int64_t n);
 

@@ -307,13 +307,15 @@ size_t CscSortTempBytes(int64_t nnz)
         const size_t tiles = static_cast<size_t>((nnz + kSortTile - 1) / kSortTile);
         return (tiles + 1) * kDigits * sizeof(uint32_t);
     }
-    size_t bytes = 0;
-    SortParams q{};
-    q.nnz = nnz;
-    if (SmallSort(nullptr, bytes, q, nullptr, nullptr, 31, nullptr) != hipSuccess) {
-        bytes = static_cast<size_t>(nnz) * 16 + (1 << 20);  // no device to ask: a generous bound
-    }
-    return bytes;
+    return LastResult(nnz, [](int64_t n) {
+        size_t bytes = 0;
+        SortParams q{};
+        q.nnz = n;
+        if (SmallSort(nullptr, bytes, q, nullptr, nullptr, 31, nullptr) != hipSuccess) {
+            bytes = static_cast<size_t>(n) * 16 + (1 << 20);  // no device to ask: a generous bound
+        }
+        return bytes;
+    });
 }
 
 int LaunchCscSort(const CscSort& c, void* stream)

@@ -3649,12 +3649,14 @@ int BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
 
 size_t TaskScanTempBytes(int64_t n)
 {
-    size_t bytes = 0;
-    if (hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, static_cast<int32_t*>(nullptr),
-                                         static_cast<int32_t*>(nullptr), static_cast<int>(n)) != hipSuccess) {
-        bytes = static_cast<size_t>(n) * 16 + (64 << 10);  // no device to ask: a generous bound
-    }
-    return bytes;
+    return LastResult(n, [](int64_t count) {
+        size_t bytes = 0;
+        if (hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, static_cast<int32_t*>(nullptr),
+                                             static_cast<int32_t*>(nullptr), static_cast<int>(count)) != hipSuccess) {
+            bytes = static_cast<size_t>(count) * 16 + (64 << 10);  // no device to ask: a generous bound
+        }
+        return bytes;
+    });
 }
 
 int LaunchSpmvOpStreamFixed(const SpmvLaunch& l, float* z, void* stream)

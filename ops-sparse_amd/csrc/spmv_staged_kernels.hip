@@ -2198,12 +2198,14 @@ int LaunchStagedRowT(const SpmvLaunch& l, hipStream_t s)
 
 size_t StageScanTempBytes(int64_t n)
 {
-    size_t bytes = 0;
-    if (hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, static_cast<uint32_t*>(nullptr),
-                                         static_cast<uint32_t*>(nullptr), static_cast<int>(n)) != hipSuccess) {
-        bytes = static_cast<size_t>(n) * 8 + (1 << 20);
-    }
-    return bytes;
+    return LastResult(n, [](int64_t count) {
+        size_t bytes = 0;
+        if (hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, static_cast<uint32_t*>(nullptr),
+                                             static_cast<uint32_t*>(nullptr), static_cast<int>(count)) != hipSuccess) {
+            bytes = static_cast<size_t>(count) * 8 + (1 << 20);
+        }
+        return bytes;
+    });
 }
 
 int LaunchStagedPreprocess(const SpmvLaunch& l, void* stream)

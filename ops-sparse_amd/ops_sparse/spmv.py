@@ -80,22 +80,22 @@ class HostScalar:
 
     def __init__(self, value, compute_type):
         value = complex(value)
+        self._obj = self._convert(value, compute_type)
+        #: address of the scalar for the C calls (it keeps the scalar alive)
+        self.ptr = ctypes.cast(ctypes.pointer(self._obj), ctypes.c_void_p)
+
+    @staticmethod
+    def _convert(value, compute_type):
         if compute_type == DataType.COMPLEX64:
-            self._obj = _lib.Complex(value.real, value.imag)
-            return
+            return _lib.Complex(value.real, value.imag)
         if value.imag != 0.0:
             kind = "int32 SpMV" if compute_type == DataType.INT32 else "real SpMV compute type"
             raise ValueError(f"{kind} cannot use a complex scalar, but got imaginary part {value.imag}")
         if compute_type == DataType.INT32:
             if not -2.0**31 <= value.real <= float(_INT32_MAX):
                 raise ValueError(f"int32 SpMV scalar {value.real} is out of the int32 range")
-            self._obj = ctypes.c_int32(int(value.real))
-        else:
-            self._obj = ctypes.c_float(value.real)
-
-    @property
-    def ptr(self):
-        return ctypes.cast(ctypes.pointer(self._obj), ctypes.c_void_p)
+            return ctypes.c_int32(int(value.real))
+        return ctypes.c_float(value.real)
 
 
 class Handle:
@@ -214,9 +214,11 @@ class CsrSpMV:
             int(self.compute_type), int(self.alg), ctypes.c_void_p(self.workspace.data_ptr())))
 
     def run(self):
-        check("aclsparseSpMV", self._lib.aclsparseSpMV(
-            self.handle.h, int(self.op), self.alpha.ptr, self.mat.d, self.x.d, self.beta.ptr, self.y.d,
-            int(self.compute_type), int(self.alg), ctypes.c_void_p(self.workspace.data_ptr())))
+        status = self._lib.aclsparseSpMV(
+            self.handle.h, self.op, self.alpha.ptr, self.mat.d, self.x.d, self.beta.ptr, self.y.d,
+            self.compute_type, self.alg, self.workspace.data_ptr())
+        if status:
+            check("aclsparseSpMV", status)
 
 
 def _validate_npu_args(row_ptr, col_ind, values, x, y, trans, base):
