@@ -309,8 +309,13 @@ constexpr int64_t kLongChunks = SPMV_LONG_CHUNKS;  // blocks with more chunks th
 
 // Small matrices (fp32 compute, opA = N): below kSmallNnz entries, and unless
 // Preprocess finds a row of more than SmallRowLimit entries, the row kernel
-// gives each row 2^SmallLanes lanes of four entries a turn.
-constexpr int64_t kSmallNnz = int64_t{1} << 19;
+// gives each row 2^SmallLanes lanes of four entries a turn.  The line is that
+// of the 16-bit column copy, whose kernels give the same bits as the row
+// blocks: above it the first product after Preprocess, every later one and
+// one without Preprocess have to agree.  (By speed alone it would lie at
+// about 4 M entries: random rows of 24-40, 3.5 M entries 21-25 -> 18-21 µs, 7 M
+// 39-42 -> 34-43, 14 M 73-115 -> 79-131.)
+constexpr int64_t kSmallNnz = int64_t{1} << 20;
 inline int32_t SmallLanes(int64_t rows, int64_t nnz)
 {
     int32_t lg = 0;  // a turn covers one and a half mean rows
@@ -405,6 +410,7 @@ inline bool NarrowTypes(aclDataType valueType, aclDataType computeType)
 
 // Narrow columns are built for matrices of at least this many entries.
 constexpr int64_t kNarrowMinNnz = int64_t{1} << 20;
+static_assert(kSmallNnz <= kNarrowMinNnz, "matrices with a path choice keep the row blocks");
 constexpr int32_t kNarrowFlag = 3;  // staged_flag value of the narrow-column row kernel
 // staged_flag value of the banded one-pass transpose on 16-bit copies of its
 // two per-entry streams (each entry's row as an offset from its CSC block's

@@ -1021,7 +1021,7 @@ def test_complex_graph_capture_on_chosen_paths(op, dev):
         torch.cuda.synchronize()
 
 
-# below 2^19 entries each row gets 1 to 64 lanes of four entries a turn, unless some row exceeds four turns
+# below 2^20 entries each row gets 1 to 64 lanes of four entries a turn, unless some row exceeds four turns
 # (limit = 16 lanes' entries): rows exactly at the limit, one entry past it in the last row, and ragged tails
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("i64,base", [(False, 0), (True, 1)])
@@ -1039,7 +1039,7 @@ def test_small_matrices(dev, dtype, i64, base, rows, mean, past):
         lens = np.minimum(lens, 16 << lg) if not past else np.concatenate([np.minimum(lens[:-1], 16 << lg), lens[-1:]])
     cols = max(8, int(lens.max()) // 2)
     nnz = int(lens.sum())
-    assert nnz < 1 << 19
+    assert nnz < 1 << 20
     rp = np.concatenate([[0], np.cumsum(lens)]) + base
     col = rng.integers(0, cols, nnz).astype(np.int32) + base
     t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(d)  # noqa: E731
