@@ -217,7 +217,8 @@ struct SpmvLayout {
     int64_t items_per_block = 0;
     int64_t num_blocks = 0;
     uint32_t rowptr_bytes = 4;
-    // Transpose by columns (CSC pattern built by Preprocess): column offsets
+    // Transpose by columns (CSC pattern built by Preprocess unless it chose
+    // the column-bucketed kernels, which need only colptr): column offsets
     // colptr[cols+1] (RowT), the row of every entry in CSR order
     // entry_row[nnz] (int32) and, in column order, each entry's position in
     // the CSR arrays csc_pos[nnz] (RowT), plus the sort's temporary arrays
@@ -479,7 +480,7 @@ inline bool StageEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t v
 // column (W columns per bucket, W chosen so that a bucket's entries fit one
 // workgroup's LDS); pass 1 writes each tile's products as runs into bucket
 // order, pass 2 loads one bucket's products into LDS, places them in column
-// order (each entry's place, from the CSC pattern, is a Preprocess table) and
+// order (each entry's place is a Preprocess table, counted per bucket) and
 // sums every column in row order.  It reuses the staged sections: st_perm is
 // each entry's slot in its tile's bucket-ordered runs, st_cl each slot's
 // place within its bucket's column-ordered products.

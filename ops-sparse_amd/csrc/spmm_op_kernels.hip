@@ -472,9 +472,9 @@ void SpmmOpKernel(MmParams p)
 }
 
 // Small k (k * 64 * J fp32 values fit the workgroup's 64 KiB of LDS): the
-// workgroup stages the column tile op(B)[0:k, tile] in LDS once (fp16 widened
-// to fp32, exactly) and its four waves then take their rows' products from
-// LDS; op(B) is read from L2 once per workgroup instead of once per entry.
+// workgroup stages the column tile op(B)[0:k, tile] in LDS once (fp32 only:
+// fp16 takes SpmmOpLdsBcastKernel on fp16 tiles) and its waves then take their
+// rows' products from LDS; op(B) is read from L2 once per workgroup instead of once per entry.
 // One row per wave at a time, its entries shared by cross-lane reads.
 constexpr int kLdsBytes = 64 * 1024;
 constexpr int kLdsWideBytes = 128 * 1024;  // J = 4 tiles without compensation

@@ -22,8 +22,8 @@
 //    (and real A with complex y) run on the same row blocks and chunk loads
 //    with an int64 / complex accumulator (SpmvStreamGenKernel); strided or
 //    unaligned operands use the general LDS-scan kernel (SpmvRowBlockKernel).
-//  * Transpose: Preprocess builds a CSC pattern (radix sort of (column,
-//    position) pairs); each SpMV streams the products a_k*x_row(k) in CSR
+//  * Transpose (other than on the column-bucketed kernels): Preprocess builds
+//    a CSC pattern (radix sort of (column, position) pairs); each SpMV streams the products a_k*x_row(k) in CSR
 //    order and then sums every column's products in a fixed order
 //    (deterministic, the reference's CSR_ALG2 semantics,
 //    sparse/spmv/arch35/spmv_kernel.cpp:861-879).  Transposes beyond the
