@@ -351,6 +351,9 @@ constexpr int kFlatWaves = 1;
 // kernels (7.2 M random entries, a call with its set-up: 133 -> 123 µs).
 constexpr int64_t kFallbackWgs = 32768;
 constexpr int64_t kStagedFallbackWgs = 8192;
+// Workgroups (of one wave) beyond which a lanes-per-row launch does not grow:
+// every wave slot of the chip.
+constexpr int64_t kSmallWgs = 8192;
 
 static_assert(kLaneItems == 8, "the reductions are written for 8 slots per lane");
 static_assert(kWaveRows <= 2 * kWave - 1, "two rows per lane");
@@ -2638,7 +2641,9 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
                     p.long_rows = &At<SpmvWsHeader>(l.ws, 0)->long_rows;
                     const int64_t rpw = kWave >> p.lane_lg;
                     const int64_t rowWgs = ((l.rows + rpw - 1) / rpw + kXcds - 1) / kXcds * kXcds;
-                    const unsigned gs = static_cast<unsigned>(rowWgs > g ? (rowWgs < 8192 ? rowWgs : 8192) : g);
+                    // never below g: the row-block code behind SmallRows takes one block per wave
+                    const int64_t capped = rowWgs < kSmallWgs ? rowWgs : kSmallWgs;
+                    const unsigned gs = capped > g ? static_cast<unsigned>(capped) : g;
                     if (betaNz) {
                         hipLaunchKernelGGL((SpmvStreamFlatKernel<RowT, V, O, true, false, false, false, true>), dim3(gs),
                                            wg, 0, stream_, p);

@@ -1025,7 +1025,7 @@ def test_complex_graph_capture_on_chosen_paths(op, dev):
 # (limit = 16 lanes' entries): rows exactly at the limit, one entry past it in the last row, and ragged tails
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("i64,base", [(False, 0), (True, 1)])
-@pytest.mark.parametrize("rows,mean", [(65, 1), (1001, 2), (4099, 5), (3001, 21), (2050, 85), (67, 400)])
+@pytest.mark.parametrize("rows,mean", [(65, 1), (1001, 2), (4099, 5), (777, 9), (3001, 21), (1500, 40), (2050, 85), (67, 400)])
 @pytest.mark.parametrize("past", [0, 1])
 def test_small_matrices(dev, dtype, i64, base, rows, mean, past):
     rng = np.random.default_rng(rows + mean)
@@ -1065,3 +1065,71 @@ def test_small_matrices(dev, dtype, i64, base, rows, mean, past):
         eps = {torch.float32: 0.0, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
         err = np.abs(y.double().cpu().numpy() - want)
         assert np.all(err <= eps * np.abs(want) + 1e-5 * scale + (1e-7 if eps else 0.0))
+
+
+# Below 2^20 entries with few of them per row (one lane per row): more rows than the capped launch has lanes, so that
+# its waves loop, and more row blocks than it has workgroups when one row past the limit of 16 entries leaves the
+# matrix to the row blocks.  A sum of at most 17 products is within 17 * 2^-24 < 1e-5 of its terms' magnitudes.
+@pytest.mark.parametrize("dtype,i64", [(torch.float32, False), (torch.float32, True), (torch.float16, False),
+                                       (torch.bfloat16, True)])
+@pytest.mark.parametrize("rows,nnz", [(800_000, 600_000), (1_000_000, 900_000), (2_000_000, 500_000),
+                                      (2_097_152, (1 << 20) - 1), (6_000_000, 1000)])
+@pytest.mark.parametrize("past", [0, 1])
+@pytest.mark.parametrize("prep", [False, True])
+def test_small_matrices_of_many_rows(dev, dtype, i64, rows, nnz, past, prep):
+    rng = np.random.default_rng(rows + nnz + past)
+    cols = 4096
+    at = np.sort(rng.choice(rows * 2, nnz - 33, replace=False)) // 2  # at most two entries per row
+    at = np.concatenate([at[at != rows // 3], np.full(16 + past, rows // 3), [rows - 1]])
+    at = np.sort(np.concatenate([at, np.arange(nnz - len(at)) * 7]))
+    lens = np.bincount(at, minlength=rows)
+    assert lens.sum() == nnz and lens.max() == 16 + past and lens[-1] > 0
+    rp = np.concatenate([[0], np.cumsum(lens)])
+    col = rng.integers(0, cols, nnz).astype(np.int32)
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(d)  # noqa: E731
+    vals, x = t(rng.uniform(-1, 1, nnz), dtype), t(rng.uniform(-1, 1, cols), dtype)
+    y = torch.full((rows,), float("nan"), device=dev).to(dtype)
+    plan = CsrSpMV(rows, cols, t(rp, torch.int64 if i64 else torch.int32), t(col, torch.int32), vals, x, y, 1.5, 0.0)
+    if prep:
+        plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    prod = 1.5 * vals.double().cpu().numpy() * x.double().cpu().numpy()[col]
+    want = np.bincount(at, weights=prod, minlength=rows)
+    scale = np.bincount(at, weights=np.abs(prod), minlength=rows)
+    eps = {torch.float32: 0.0, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+    err = np.abs(y.double().cpu().numpy() - want)
+    assert np.all(err <= eps * np.abs(want) + 1e-5 * scale + (1e-7 if eps else 0.0))
+
+
+# the line of the lanes-per-row kernel: the last entry count below it and the first at it, whose products have the
+# same bits without Preprocess, first after it and later.  Sums of about 35 products, as above.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("nnz", [(1 << 20) - 1, 1 << 20])
+def test_small_matrices_line(dev, dtype, nnz):
+    rng = np.random.default_rng(nnz)
+    rows = cols = 30_011
+    at = np.sort(rng.integers(0, rows, nnz))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(at, minlength=rows))])
+    col = rng.integers(0, cols, nnz).astype(np.int32)
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(d)  # noqa: E731
+    vals, x = t(rng.uniform(-1, 1, nnz), dtype), t(rng.uniform(-1, 1, cols), dtype)
+    out = []
+    for prep in (False, True):
+        y = torch.full((rows,), float("nan"), device=dev).to(dtype)
+        plan = CsrSpMV(rows, cols, t(rp, torch.int32), t(col, torch.int32), vals, x, y, 1.0, 0.0)
+        if prep:
+            plan.preprocess()
+        for _ in range(3 if prep else 1):
+            plan.run()
+            torch.cuda.synchronize()
+            out.append(y.clone())
+            y.fill_(float("nan"))
+    prod = vals.double().cpu().numpy() * x.double().cpu().numpy()[col]
+    want = np.bincount(at, weights=prod, minlength=rows)
+    scale = np.bincount(at, weights=np.abs(prod), minlength=rows)
+    eps = {torch.float32: 0.0, torch.float16: 2.0**-11}[dtype]
+    err = np.abs(out[0].double().cpu().numpy() - want)
+    assert np.all(err <= eps * np.abs(want) + 1e-5 * scale + (1e-7 if eps else 0.0))
+    for o in out[1:]:
+        assert torch.equal(o, out[0])
