@@ -134,8 +134,9 @@ struct RowBlockParams {
     // Stream kernel: when > 0, the grid is capped and each wave loops over
     // the blocks tile, tile + block_stride, ... (block_stride = all block waves)
     int64_t block_stride;
-    int32_t lane_lg;            // small matrices (SmallRows): log2 of the lanes per row
-    const uint32_t* long_rows;  // and the header word that says whether some row is too long for it
+    int32_t lane_lg;            // small matrices (SmallRows): log2 of the lanes per row,
+    const uint32_t* long_rows;  // the header word that says whether some row is too long for it
+    int64_t block_wgs;          // and the row blocks' workgroups (the launch may have more)
 };
 
 // Loads the block's row offsets relative to its first non-zero into LDS.
@@ -1210,7 +1211,7 @@ __device__ __forceinline__ void FixupLongBlock(const RowBlockParams& p, const St
 // for four and runs through some 2000 of straight-line code that every CU
 // has to fetch first.  Where Preprocess found a row of more than four turns
 // (long_rows, read beside the first row offsets) SmallRows returns false and
-// the row-block code takes the matrix.  Kernel time, row blocks -> lanes per
+// the row-block code takes the matrix, 0.1-0.5 µs later than without the look.  Kernel time, row blocks -> lanes per
 // row: 4096 rows of 41 entries, fp32, 9.8 -> 3.3 µs; 40 000 rows of 5 4.4 ->
 // 3.2; a product of 30 000 rows of 27 14.2 -> 6.0 µs.
 template <typename RowT, ValKind V, OutKind O, bool kBeta>
@@ -1358,7 +1359,12 @@ void SpmvStreamFlatKernel(RowBlockParams p)
     // Block worker: one block per wave, or (block_stride > 0, capped grid)
     // blocks tile, tile + block_stride, ...
     const int64_t wg = static_cast<int64_t>(blockIdx.x) - p.task_wgs;
-    const int64_t per = (static_cast<int64_t>(gridDim.x) - p.task_wgs) / kXcds;
+    const int64_t wgs = kSmall ? p.block_wgs : static_cast<int64_t>(gridDim.x) - p.task_wgs;
+    // (a lanes-per-row launch has more workgroups: spread by those, its blocks
+    // went to the first XCDs only, and 200 000 rows of 4 with one long row
+    // took 11.6 µs, now 7.6)
+    if (kSmall && wg >= wgs) return;
+    const int64_t per = wgs / kXcds;
     auto block = [&](int64_t tile) {
         Stage cur = OpenTileFlat<RowT>(p, tile);
         if constexpr (kEntry) {
@@ -2639,6 +2645,7 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
                 if (l.layout.tasks && p.rows > 0 && l.nnz < kSmallNnz) {
                     p.lane_lg = SmallLanes(l.rows, l.nnz);
                     p.long_rows = &At<SpmvWsHeader>(l.ws, 0)->long_rows;
+                    p.block_wgs = blockWgs;
                     const int64_t rpw = kWave >> p.lane_lg;
                     const int64_t rowWgs = ((l.rows + rpw - 1) / rpw + kXcds - 1) / kXcds * kXcds;
                     // never below g: the row-block code behind SmallRows takes one block per wave
