@@ -179,7 +179,7 @@ struct SpmvWsHeader {
     // (some block of more than 127 rows, or whose rows run past its window);
     // complex64 transposes: nonzero when some entry's offsets exceed 16 bits
     uint32_t entry_bad;
-    // matrices below kSmallNnz entries: nonzero when some row has more than
+    // small matrices (SmallMatrix): nonzero when some row has more than
     // SmallRowLimit entries (the row-block code then takes the matrix)
     uint32_t long_rows;
     uint32_t reserved[5];
@@ -308,15 +308,21 @@ struct SpmvLayout {
 #endif
 constexpr int64_t kLongChunks = SPMV_LONG_CHUNKS;  // blocks with more chunks than this are split into tasks
 
-// Small matrices (fp32 compute, opA = N): below kSmallNnz entries, and unless
-// Preprocess finds a row of more than SmallRowLimit entries, the row kernel
+// Small matrices (fp32 compute, opA = N): below kSmallNnz entries in at most
+// kSmallRows rows, and unless Preprocess finds a row of more than SmallRowLimit entries, the row kernel
 // gives each row 2^SmallLanes lanes of four entries a turn.  The line is that
 // of the 16-bit column copy, whose kernels give the same bits as the row
 // blocks: above it the first product after Preprocess, every later one and
 // one without Preprocess have to agree.  (By speed alone it would lie at
 // about 4 M entries: random rows of 24-40, 3.5 M entries 21-25 -> 18-21 µs, 7 M
-// 39-42 -> 34-43, 14 M 73-115 -> 79-131.)
+// 39-42 -> 34-43, 14 M 73-115 -> 79-131.)  Preprocess looks at every row's
+// length, which costs up to 1.5 µs at kSmallRows rows, for 2 µs saved in every
+// product; past it the look is a pass over memory (5 M rows: Preprocess 24 ->
+// 30 µs, a product 27 -> 23; 50 M: 186 -> 273 and 255 -> 250), and the row
+// blocks take the matrix.
 constexpr int64_t kSmallNnz = int64_t{1} << 20;
+constexpr int64_t kSmallRows = int64_t{1} << 20;
+inline bool SmallMatrix(int64_t rows, int64_t nnz) { return nnz < kSmallNnz && rows > 0 && rows <= kSmallRows; }
 inline int32_t SmallLanes(int64_t rows, int64_t nnz)
 {
     int32_t lg = 0;  // a turn covers one and a half mean rows

@@ -2642,7 +2642,7 @@ int LaunchRowBlock(const SpmvLaunch& l, hipStream_t stream)
                 return 0;
             }
             if constexpr (!kInt8) {
-                if (l.layout.tasks && p.rows > 0 && l.nnz < kSmallNnz) {
+                if (l.layout.tasks && SmallMatrix(l.rows, l.nnz)) {
                     p.lane_lg = SmallLanes(l.rows, l.nnz);
                     p.long_rows = &At<SpmvWsHeader>(l.ws, 0)->long_rows;
                     p.block_wgs = blockWgs;
@@ -3207,7 +3207,7 @@ __global__ __launch_bounds__(kThreads) void TaskFillKernel(const int32_t* taskSt
     }
 }
 
-constexpr int kTaskCountWgs = 1024;
+constexpr int kTaskCountWgs = 4096;  // kSmallRows rows in one turn
 
 template <typename RowT>
 int BuildTasks(const SpmvLaunch& l, hipStream_t s)
@@ -3215,7 +3215,7 @@ int BuildTasks(const SpmvLaunch& l, hipStream_t s)
     const int64_t nb = l.layout.num_blocks;
     int32_t* counts = At<int32_t>(l.ws, l.layout.task_head_offset);  // temporary: max_tasks >= nb + 1
     int32_t* start = At<int32_t>(l.ws, l.layout.task_start_offset);
-    const int64_t rows = l.nnz < kSmallNnz ? l.rows : 0;  // small matrices: their rows are looked at too
+    const int64_t rows = SmallMatrix(l.rows, l.nnz) ? l.rows : 0;  // small matrices: their rows are looked at too
     const int grid = GridFor(rows > nb + 1 ? rows : nb + 1);
     hipLaunchKernelGGL((TaskCountKernel<RowT>), dim3(grid < kTaskCountWgs ? grid : kTaskCountWgs), dim3(kThreads), 0,
                        s, At<const RowT>(l.ws, l.layout.block_nnz_offset), nb, counts,

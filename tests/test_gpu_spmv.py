@@ -1073,6 +1073,7 @@ def test_small_matrices(dev, dtype, i64, base, rows, mean, past):
 @pytest.mark.parametrize("dtype,i64", [(torch.float32, False), (torch.float32, True), (torch.float16, False),
                                        (torch.bfloat16, True)])
 @pytest.mark.parametrize("rows,nnz", [(800_000, 600_000), (1_000_000, 900_000), (2_000_000, 500_000),
+                                      (1 << 20, 700_000), ((1 << 20) + 1, 700_000),
                                       (2_097_152, (1 << 20) - 1), (6_000_000, 1000)])
 @pytest.mark.parametrize("past", [0, 1])
 @pytest.mark.parametrize("prep", [False, True])
