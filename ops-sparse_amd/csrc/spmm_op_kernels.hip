@@ -517,9 +517,8 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))
     __syncthreads();
     const int64_t j0 = jt + lane * J;
     const int64_t row0 = (chunk * (kLdsThreads / kMmWave) + wv) * p.lds_rows;
-    for (int rr = 0; rr < p.lds_rows; ++rr) {
-        const int64_t row = row0 + rr;
-        if (row >= p.m) break;
+    const int64_t row1 = row0 + p.lds_rows < p.m ? row0 + p.lds_rows : p.m;
+    for (int64_t row = row0; row < row1; ++row) {
         // the row's entries are read 64 at a time, one per lane, and handed out
         // through scalar registers; their tiles of op(B) come from LDS
         const int64_t rs = static_cast<int64_t>(rp[row]) - p.base;
@@ -580,61 +579,58 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(8))
     }
 }
 
-// Stages op(B)[0:k, jt:jt+TW] in LDS (row r at sB[r*TW]; columns past n read
-// as 0) as fp32, or as fp16 when L is uint16_t.  Tiles of a
-// row-major op(B) whose rows start on a 4-element boundary, and whose columns
-// inside it are a multiple of 4, move 4 elements per load, four loads in
-// flight per thread; other tiles element by element.
-template <bool kHalf, int TW, typename L>
-__device__ __forceinline__ void StageBTile(const MmParams& p, const typename Elem<kHalf>::T* b, L* sB, int64_t jt,
-                                          int k)
+// Stages op(B)[0:k, jt:jt+TW] in LDS in its own type (row r at sB[r*TW];
+// columns past n read as 0).  Tiles of a row-major op(B) whose rows start on a
+// 4-element boundary, and whose columns inside it are a multiple of 4, move 4
+// elements per load, four loads in flight per thread (kFull: all TW columns
+// are inside op(B)); other tiles element by element.
+template <typename T, int TW, bool kFull>
+__device__ __forceinline__ void StageBVec(const MmParams& p, const T* b, T* sB, int64_t jt, int k, int inside)
 {
-    using T = typename Elem<kHalf>::T;
-    constexpr bool kRaw = std::is_same<T, L>::value;  // LDS holds op(B)'s own type
-    const auto load = [&](int64_t i) {
-        if constexpr (kRaw) return b[i];
-        else return Elem<kHalf>::Load(b, i);
-    };
-    const int64_t left = p.n - jt;  // columns of the tile inside op(B)
-    if (p.b_contig && p.b_vec && (left >= TW || left % 4 == 0)) {
-        constexpr int kQ = TW / 4;  // 4-element groups per staged row
-        const int inside = left >= TW ? kQ : static_cast<int>(left / 4);
-        const int total = k * kQ;
-        for (int i0 = static_cast<int>(threadIdx.x); i0 < total; i0 += 4 * kLdsThreads) {
-            Vec<T, 4> w[4];
+    constexpr int kQ = TW / 4;  // 4-element groups per staged row; `inside` of them inside op(B)
+    const int total = k * kQ;
+    for (int i0 = static_cast<int>(threadIdx.x); i0 < total; i0 += 4 * kLdsThreads) {
+        Vec<T, 4> w[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = i0 + u * kLdsThreads;
-                const int r = idx < total ? idx / kQ : 0, q = idx < total ? idx % kQ : 0;
-                w[u] = *reinterpret_cast<const Vec<T, 4>*>(b + static_cast<int64_t>(r) * p.ldb + jt +
-                                                           4 * (q < inside ? q : 0));
-                if (q >= inside) w[u] = Vec<T, 4>{};
-            }
+        for (int u = 0; u < 4; ++u) {
+            const int idx = i0 + u * kLdsThreads;
+            const int r = idx < total ? idx / kQ : 0, q = idx < total ? idx % kQ : 0;
+            w[u] = *reinterpret_cast<const Vec<T, 4>*>(b + static_cast<int64_t>(r) * p.ldb + jt +
+                                                       4 * (kFull || q < inside ? q : 0));
+        }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = i0 + u * kLdsThreads;
-                if (idx < total) {
-                    Vec<L, 4> f;
+        for (int u = 0; u < 4; ++u) {
+            const int idx = i0 + u * kLdsThreads;
+            const int q = idx % kQ;
+            if (idx < total) {
+                Vec<T, 4> f;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if constexpr (kRaw) f.v[e] = w[u].v[e];
-                        else f.v[e] = Half2Float(w[u].v[e]);
-                    }
-                    *reinterpret_cast<Vec<L, 4>*>(&sB[(idx / kQ) * TW + 4 * (idx % kQ)]) = f;
-                }
+                for (int e = 0; e < 4; ++e) f.v[e] = kFull || q < inside ? w[u].v[e] : T{0};
+                *reinterpret_cast<Vec<T, 4>*>(&sB[(idx / kQ) * TW + 4 * q]) = f;
             }
         }
+    }
+}
+
+template <typename T, int TW>
+__device__ __forceinline__ void StageBTile(const MmParams& p, const T* b, T* sB, int64_t jt, int k)
+{
+    const int64_t left = p.n - jt;  // columns of the tile inside op(B)
+    if (p.b_contig && p.b_vec && left >= TW) {
+        StageBVec<T, TW, true>(p, b, sB, jt, k, TW / 4);
+    } else if (p.b_contig && p.b_vec && left % 4 == 0) {
+        StageBVec<T, TW, false>(p, b, sB, jt, k, static_cast<int>(left / 4));
     } else if (p.b_contig) {
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int r = idx / TW, cj = idx - r * TW;
             const int64_t j = jt + cj;
-            sB[idx] = j < p.n ? load(static_cast<int64_t>(r) * p.ldb + j) : L{0};
+            sB[idx] = j < p.n ? b[static_cast<int64_t>(r) * p.ldb + j] : T{0};
         }
     } else {
         for (int idx = static_cast<int>(threadIdx.x); idx < k * TW; idx += kLdsThreads) {
             const int cj = idx / k, r = idx - cj * k;
             const int64_t j = jt + cj;
-            sB[r * TW + cj] = j < p.n ? load(j * p.ldb + r) : L{0};
+            sB[r * TW + cj] = j < p.n ? b[j * p.ldb + r] : T{0};
         }
     }
 }
@@ -748,7 +744,7 @@ void SpmmOpLdsBcastKernel(MmParams p)
             w.v[q] = x;
         }
     };
-    StageBTile<kHalf, TW>(p, b, sB, jt, k);
+    StageBTile<T, TW>(p, b, sB, jt, k);
     __syncthreads();
     const uint32_t laneOff = static_cast<uint32_t>(lane * J * kEsz);
     const int64_t j0 = jt + lane * J;
