@@ -880,35 +880,51 @@ void DispatchLds(const MmParams& p, int J, bool kahan, unsigned grid, unsigned l
 
 bool AlignedTo(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
 
-// Rows per wave of the LDS kernels.  Four, unless that makes fewer than two
-// workgroups per CU; then by their cost in CU cycles: a workgroup stages its
-// tile (about 2000 + 8 cycles per row of op(B)) and works 16 rows at a time
-// (4 waves per SIMD, 4 cycles per instruction and entry), the workgroups go
-// over the chip in rounds of one per CU, and staging hides behind another
-// workgroup when two fit a CU.  Fewer rows make more, smaller workgroups:
-// fuller last rounds, more staging.  Half-dense m x k x n, µs, 4 rows ->
-// chosen: fp16 2048 x 128 x 2048 24.8 -> 23.1 (2 rows), 3983 x 179 x 1196
-// 65 -> 56 (2), 700 x 40 x 300 12.1 -> 10.1 (1); fp32 700 x 40 x 300 26 -> 10
-// (1), 1500 x 100 x 1000 23.5 -> 13.9 (1).  With more workgroups fewer rows
-// only add staging: fp32 4096 x 32 x 2048 41.5 (4 rows), 49.4 (1).
-constexpr int64_t kCus = 256;
-int LdsRows(int64_t m, int64_t nnz, int64_t k, int64_t tiles, int J, bool half, int64_t lds)
+// What an LDS kernel's workgroup costs, in CU cycles (fitted to 4000 shapes
+// per kernel: 200-65536 rows, k 16-256, n 64-2048, 2-50% full, fp32, fp16 and
+// compensated fp32, at 1, 2 and 4 rows per wave; the shape chosen by it is
+// within 1% of the fastest on average).
+struct LdsRate {
+    int64_t group;  // per workgroup, or per two that share a CU: launch, first loads
+    int64_t bytes;  // tile bytes staged per cycle (half when read element by element)
+    int64_t entry;  // per turn of 16 rows and entry of the mean row
+    int64_t turn;   // per turn: row offsets, result
+    int64_t alone;  // sixteenths: a workgroup alone on its CU against one of two
+};
+
+LdsRate LdsRateOf(int J, bool half, bool kahan, bool wide)
 {
-    const int64_t row = 16 * (half ? J + 3 : 2 * J + 2) * (nnz / m + 1);
-    const int64_t stage = 2000 + 8 * k;
-    const int64_t perRound = lds <= 80 * 1024 ? 0 : stage;
+    if (half) return {1280, 43, 16 * (J + 3), 1090, 21};
+    if (kahan) return {2970, 150, 52 * (J + 1), 690, 17};
+    if (J == 4 && !wide) return {1150, 26, 520, 820, 18};  // SpmmOpLdsKernel
+    return {3300, 40, 16 * (2 * J + 2), 1550, 19};
+}
+
+constexpr int64_t kCus = 256;
+constexpr int64_t kLdsPerCu = 160 * 1024;
+
+// A workgroup stages its tile, then its 16 waves take r turns of a row each.
+// The workgroups go over the CUs evenly, two at a time where two tiles fit a
+// CU's LDS.  Fewer rows make more, smaller workgroups: fuller last rounds,
+// more staging.
+int64_t LdsCost(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t tiles, int r, bool byElement)
+{
+    const int64_t perBlock = int64_t{kLdsThreads / kMmWave} * r;
+    const int64_t perCu = ((m + perBlock - 1) / perBlock * tiles + kCus - 1) / kCus;
+    const int64_t pairs = 2 * lds <= kLdsPerCu ? perCu / 2 : 0;
+    const int64_t work = lds / c.bytes * (byElement ? 2 : 1) + r * (c.entry * nnz / m + c.turn);
+    return pairs * (2 * work + c.group) + (perCu - 2 * pairs) * (work * c.alone / 16 + c.group);
+}
+
+// Rows per wave of the LDS kernels: the cheapest of 4, 2 and 1.  µs at 4 rows
+// -> chosen: half-dense fp16 2048 x 128 x 2048 24.8 -> 23.1 (2 rows), fp32
+// 700 x 40 x 300 26 -> 10 (1); with few entries per row fewer rows only add
+// staging: fp32 6000 x 160 x 300, 2% full, 12.1 (4), 13.8 (2), 17.8 (1).
+int LdsRows(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t tiles, bool byElement)
+{
     int best = kLdsMaxRows;
-    int64_t bestCost = INT64_MAX;
-    const int64_t perMax = int64_t{kLdsThreads / kMmWave} * kLdsMaxRows;
-    if ((m + perMax - 1) / perMax * tiles >= 2 * kCus) return kLdsMaxRows;
-    for (int r = 1; r <= kLdsMaxRows; r *= 2) {
-        const int64_t perBlock = int64_t{kLdsThreads / kMmWave} * r;
-        const int64_t blocks = (m + perBlock - 1) / perBlock * tiles;
-        const int64_t cost = (blocks + kCus - 1) / kCus * (r * row + perRound) + stage;
-        if (cost < bestCost) {
-            best = r;
-            bestCost = cost;
-        }
+    for (int r = kLdsMaxRows / 2; r >= 1; r /= 2) {
+        if (LdsCost(c, m, nnz, lds, tiles, r, byElement) < LdsCost(c, m, nnz, lds, tiles, best, byElement)) best = r;
     }
     return best;
 }
@@ -959,11 +975,14 @@ int LaunchSpmmOp(const SpmmLaunch& l, void* stream)
         p.tiles = (l.n + tw - 1) / tw;
         p.c_vec = l.c_row_major && l.ldc % J == 0 && AlignedTo(l.c, J * esz) ? 1 : 0;
         p.b_vec = l.ldb % 4 == 0 && AlignedTo(l.b, 4 * esz) ? 1 : 0;  // staging 4 elements per load
-        p.lds_rows = LdsRows(l.m, l.nnz, l.k, p.tiles, J, l.fp16 != 0, l.k * tw * static_cast<int64_t>(esz));
+        const int64_t ldsBytes = l.k * tw * static_cast<int64_t>(esz);
+        const bool byElement = l.fp16 && (!p.b_contig || !p.b_vec || l.n % 4 != 0);
+        p.lds_rows = LdsRows(LdsRateOf(J, l.fp16 != 0, kahan && !l.fp16, ldsBytes > kLdsBytes), l.m, l.nnz, ldsBytes,
+                             p.tiles, byElement);
         const int64_t rowsPerBlock = int64_t{kLdsThreads / kMmWave} * p.lds_rows;
         const int64_t blocks = (l.m + rowsPerBlock - 1) / rowsPerBlock * p.tiles;
         if (blocks <= 0x7FFFFFFF) {
-            const unsigned lds = static_cast<unsigned>(l.k * tw * static_cast<int64_t>(esz));
+            const unsigned lds = static_cast<unsigned>(ldsBytes);
             if (l.rowptr64) {
                 if (l.fp16) DispatchLds<int64_t, true>(p, J, false, static_cast<unsigned>(blocks), lds, s);
                 else DispatchLds<int64_t, false>(p, J, kahan, static_cast<unsigned>(blocks), lds, s);
