@@ -857,9 +857,15 @@ void DispatchLds(const MmParams& p, int J, bool kahan, unsigned grid, unsigned l
     hipLaunchKernelGGL((SpmmOpLdsKernel<RowT, KK, JJ>), dim3(grid), dim3(kLdsThreads), lds, s, p)
 #define SPMM_BCAST(JJ) \
     hipLaunchKernelGGL((SpmmOpLdsBcastKernel<RowT, kHalf, JJ>), dim3(grid), dim3(kLdsThreads), lds, s, p)
-    if constexpr (kHalf) {  // fp16 tiles: J = 4 for every k (up to 128 KiB)
-        AllowWideLds<RowT, true>();
-        SPMM_BCAST(4);
+    if constexpr (kHalf) {
+        if (J == 4) {  // up to 128 KiB
+            AllowWideLds<RowT, true>();
+            SPMM_BCAST(4);
+        } else if (J == 2) {
+            SPMM_BCAST(2);
+        } else {
+            SPMM_BCAST(1);
+        }
     } else {
         if (kahan) {
             if (J == 4) SPMM_LDS(4, true);
@@ -916,15 +922,33 @@ int64_t LdsCost(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t t
     return pairs * (2 * work + c.group) + (perCu - 2 * pairs) * (work * c.alone / 16 + c.group);
 }
 
-// Rows per wave of the LDS kernels: the cheapest of 4, 2 and 1.  µs at 4 rows
-// -> chosen: half-dense fp16 2048 x 128 x 2048 24.8 -> 23.1 (2 rows), fp32
-// 700 x 40 x 300 26 -> 10 (1); with few entries per row fewer rows only add
-// staging: fp32 6000 x 160 x 300, 2% full, 12.1 (4), 13.8 (2), 17.8 (1).
-int LdsRows(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t tiles, bool byElement)
+// Columns per lane and rows per wave of the LDS kernels: the cheapest of 4, 2
+// and 1 rows and, for fp16 (fp32 tiles are as wide as LDS allows), of 4, 2 and
+// 1 columns: a tile wider than op(B) stages and multiplies columns that are
+// not there.  µs at 4 rows -> chosen: half-dense fp16 2048 x 128 x 2048 24.8 ->
+// 23.1 (2 rows), fp32 700 x 40 x 300 26 -> 10 (1); with few entries per row
+// fewer rows only add staging: fp32 6000 x 160 x 300, 2% full, 12.1 (4), 13.8
+// (2), 17.8 (1).  fp16 65536 x 256 half-dense at 4, 2 and 1 columns per lane:
+// n = 64 168, 93 and 77 µs.
+struct LdsShape {
+    int j, rows;
+};
+
+LdsShape LdsChoose(const SpmmLaunch& l, bool kahan, int fp32J, bool byElement)
 {
-    int best = kLdsMaxRows;
-    for (int r = kLdsMaxRows / 2; r >= 1; r /= 2) {
-        if (LdsCost(c, m, nnz, lds, tiles, r, byElement) < LdsCost(c, m, nnz, lds, tiles, best, byElement)) best = r;
+    LdsShape best{};
+    int64_t bestCost = 0;
+    for (int j = l.fp16 ? 4 : fp32J; j >= (l.fp16 ? 1 : fp32J); j /= 2) {
+        const int64_t tw = int64_t{kMmWave} * j;
+        const int64_t lds = l.k * tw * (l.fp16 ? 2 : 4);
+        const LdsRate c = LdsRateOf(j, l.fp16 != 0, kahan && !l.fp16, lds > kLdsBytes);
+        for (int r = kLdsMaxRows; r >= 1; r /= 2) {
+            const int64_t cost = LdsCost(c, l.m, l.nnz, lds, (l.n + tw - 1) / tw, r, byElement);
+            if (best.j == 0 || cost < bestCost) {
+                best = {j, r};
+                bestCost = cost;
+            }
+        }
     }
     return best;
 }
@@ -967,18 +991,18 @@ int LaunchSpmmOp(const SpmmLaunch& l, void* stream)
     const bool kahan = l.high_precision != 0;
     // small k: op(B) column tiles staged in LDS (n of at least one wave's width)
     if (l.k > 0 && l.n >= kMmWave && l.k * kMmWave * 4 <= kLdsBytes) {
-        const int J = l.fp16                                                        ? 4
-                      : l.k * kMmWave * 4 * 4 <= (kahan ? kLdsBytes : kLdsWideBytes) ? 4
-                      : l.k * kMmWave * 4 * 2 <= kLdsBytes                           ? 2
-                                                                                     : 1;
+        const int fp32J = l.k * kMmWave * 4 * 4 <= (kahan ? kLdsBytes : kLdsWideBytes) ? 4
+                          : l.k * kMmWave * 4 * 2 <= kLdsBytes                          ? 2
+                                                                                        : 1;
+        p.b_vec = l.ldb % 4 == 0 && AlignedTo(l.b, 4 * esz) ? 1 : 0;  // staging 4 elements per load
+        const bool byElement = l.fp16 && (!p.b_contig || !p.b_vec || l.n % 4 != 0);
+        const LdsShape shape = LdsChoose(l, kahan, fp32J, byElement);
+        const int J = shape.j;
         const int64_t tw = int64_t{kMmWave} * J;
+        const int64_t ldsBytes = l.k * tw * static_cast<int64_t>(esz);
         p.tiles = (l.n + tw - 1) / tw;
         p.c_vec = l.c_row_major && l.ldc % J == 0 && AlignedTo(l.c, J * esz) ? 1 : 0;
-        p.b_vec = l.ldb % 4 == 0 && AlignedTo(l.b, 4 * esz) ? 1 : 0;  // staging 4 elements per load
-        const int64_t ldsBytes = l.k * tw * static_cast<int64_t>(esz);
-        const bool byElement = l.fp16 && (!p.b_contig || !p.b_vec || l.n % 4 != 0);
-        p.lds_rows = LdsRows(LdsRateOf(J, l.fp16 != 0, kahan && !l.fp16, ldsBytes > kLdsBytes), l.m, l.nnz, ldsBytes,
-                             p.tiles, byElement);
+        p.lds_rows = shape.rows;
         const int64_t rowsPerBlock = int64_t{kLdsThreads / kMmWave} * p.lds_rows;
         const int64_t blocks = (l.m + rowsPerBlock - 1) / rowsPerBlock * p.tiles;
         if (blocks <= 0x7FFFFFFF) {

@@ -453,3 +453,18 @@ def test_lds_rows_and_tiles(dev, half, m, k, n):
         got, want, _ = _run_plan(dev, m, k, n, rp, col, val, b, c, op_b, order_b, Order.ROW, SpMMOpAlg.ALG1, half, 1.25,
                                  0.5, ldb_pad=pad, ldc_pad=4 * pad)
         np.testing.assert_array_equal(got, want)
+
+
+# fp16 tiles of 64, 128 and 256 columns (1, 2 and 4 per lane) with 1, 2 and 4 rows per wave, as the launch picks them
+# for these shapes at about 20 entries a row; whole and cut last tiles, op(B) read by 4 elements and one by one
+@pytest.mark.parametrize("m,k,n", [(700, 130, 64), (9000, 130, 64), (20000, 256, 130), (3000, 256, 65), (9000, 130, 72),
+                                   (20000, 256, 65), (3000, 130, 130), (9000, 7, 192), (20000, 130, 130)])
+def test_fp16_tile_widths(dev, m, k, n):
+    rp, col, val = _rand_csr(m, k, min(1.0, 20 / k), m + n, bad_cols=n == 65)
+    rng = np.random.default_rng(k)
+    b, c = rng.uniform(-1, 1, k * n), rng.uniform(-1, 1, m * n)
+    for order_b, op_b, order_c, pad in ((Order.ROW, Operation.NON_TRANSPOSE, Order.ROW, 0),
+                                        (Order.ROW, Operation.TRANSPOSE, Order.COL, 1)):
+        got, want, _ = _run_plan(dev, m, k, n, rp, col, val, b, c, op_b, order_b, order_c, SpMMOpAlg.ALG1, True, 1.25,
+                                 -0.5, ldb_pad=pad, ldc_pad=pad)
+        np.testing.assert_array_equal(got, want)
