@@ -1164,19 +1164,19 @@ __device__ __forceinline__ uint32_t BtKey(const StageParams& q, bool inRows, int
 
 // counts[s*(T+1) + t] = entries of tile t in bucket s (column T is zero);
 // metric[t] = the tile's non-empty runs (low kBtRunBits bits) and, above them,
-// its entries when its rows average more than kBtLongRows of them.
+// for 16-bit values, its entries in rows of more than kBtLongRow (BtDecideKernel).
 constexpr int kBtRunBits = 12;
-constexpr int kBtLongRows = 64;
+constexpr int64_t kBtLongRow = 512;
 static_assert(kBtMaxBuckets < 1 << kBtRunBits && kWide < 1 << (32 - kBtRunBits), "metric fields");
 template <typename RowT>
 __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
 {
     __shared__ uint32_t hist[kBtMaxBuckets + 1];
-    __shared__ uint32_t runs;
+    __shared__ uint32_t runs, longEntries;
     const int64_t t = blockIdx.x;
     const int nb = q.buckets + 1;
     for (int s = threadIdx.x; s < nb; s += kSortThreads) hist[s] = 0U;
-    if (threadIdx.x == 0) runs = 0U;
+    if (threadIdx.x == 0) runs = longEntries = 0U;
     __syncthreads();
     if (t < q.tiles) {
         const int64_t first = Norm<RowT>(q, 0), last = Norm<RowT>(q, q.rows);
@@ -1197,6 +1197,14 @@ __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
                 }
             }
         }
+        if (q.fp32_values == 0) {  // the tile's rows: the last one may go on in the next tile
+            const int64_t r1 = q.tile_row[t + 1] < q.rows ? q.tile_row[t + 1] : q.rows - 1;
+            for (int64_t r = q.tile_row[t] + threadIdx.x; r <= r1; r += kSortThreads) {
+                const int64_t a = Norm<RowT>(q, r), b = Norm<RowT>(q, r + 1);
+                const int64_t in = (b < e1 ? b : e1) - (a > e0 ? a : e0);
+                if (b - a > kBtLongRow && in > 0) atomicAdd(&longEntries, static_cast<uint32_t>(in));
+            }
+        }
     }
     __syncthreads();
     uint32_t mine = 0U;
@@ -1207,11 +1215,7 @@ __global__ __launch_bounds__(kSortThreads) void BtCountKernel(StageParams q)
     }
     if (mine != 0U) atomicAdd(&runs, mine);
     __syncthreads();
-    if (threadIdx.x == 0 && t < q.tiles) {
-        const int64_t entries = q.tile_nnz[t + 1] - q.tile_nnz[t];
-        const int64_t rows = q.tile_row[t + 1] - q.tile_row[t];
-        q.metric[t] = runs | (entries > kBtLongRows * rows ? static_cast<uint32_t>(entries) << kBtRunBits : 0U);
-    }
+    if (threadIdx.x == 0 && t < q.tiles) q.metric[t] = runs | longEntries << kBtRunBits;
 }
 
 // Stable places for 64 keys at a time: the counters belong to one wave, so a
@@ -1533,22 +1537,32 @@ __global__ __launch_bounds__(kSortThreads) void BtPlaceKernel(StageParams q)
 // (banded kernel -> bucketed kernels, µs per SpMV): 1 M entries 22 -> 34,
 // 2 M 40 -> 27-30, 4 M 78 (CSC kernels) -> 38.  16-bit values have no banded
 // kernel, and the CSC kernels they otherwise take read neighbouring columns'
-// products of a long row from the same lines: their count to kBtWideNnz leaves
-// out the tiles of long rows, one and a half times (bf16, CSC -> bucketed kernels: Poisson rows of
-// 8-40 entries 2.2 M 36-41 -> 22-32, 3 M 50-55 -> 23-32, 5 M 86-91 -> 32-42;
-// rows of 1 to 200 000 entries, a third of them in long rows, 2.2 M 24-30 ->
-// 29-30, 3 M 29-35 -> 29-32, 5 M 44-49 -> 37-39).
+// products of a long row from the same lines, while the bucketed kernels pay
+// for rows and columns too.  So where a sixteenth of the entries or more lie
+// in rows of more than kBtLongRow, the entries less a half of those, 0.6 per
+// row and 0.3 per column beyond a tenth of the entries have to reach
+// kBtLongNnz: fitted to 1340 matrices (2-20 M entries, means of 1 to 100 per
+// row, 0.1 to 8 columns per row, Poisson rows and rows of 1 to 200 000
+// entries), of which none takes more than 1.07 of the CSC kernels' time.
+// bf16, CSC -> bucketed kernels: Poisson rows of 8-40 entries 2.2 M 31-36 ->
+// 23-30, 3 M 45-49 -> 24-31, 5 M 77-82 -> 32-40; half of the entries in long
+// rows, a mean of 2: 3 M 32 -> 44, 6 M 56 -> 57, 12 M 118 -> 99; of 8: 3 M 32
+// -> 33, 4 M 38 -> 39, 6 M 52 -> 41; of 20: 3 M 37 -> 32, 6 M 55 -> 38.
 constexpr int64_t kBtWideNnz = int64_t{1} << 21;
+constexpr int64_t kBtLongNnz = 2500000;
 __global__ __launch_bounds__(kDecideThreads) void BtDecideKernel(StageParams q)
 {
     __shared__ int ok;
     const unsigned long long sums = SumMetric<kBtRunBits>(q);
     const unsigned long long runs = sums & 0xFFFFFFFFULL;
-    const int64_t wide = q.nnz - (q.fp32_values != 0 ? 0 : static_cast<int64_t>(sums >> 32) * 3 / 2);
+    const int64_t inLong = static_cast<int64_t>(sums >> 32);  // (0 for fp32 values)
+    const int64_t tenth = q.nnz / 10;
+    const int64_t rows = q.rows > tenth ? q.rows - tenth : 0, cols = q.cols > tenth ? q.cols - tenth : 0;
+    const bool pays = 16 * inLong < q.nnz || 10 * q.nnz - 5 * inLong - 6 * rows - 3 * cols >= 10 * kBtLongNnz;
     const bool scattered =
-        runs * static_cast<unsigned long long>(kBtRunEntries) > static_cast<unsigned long long>(q.nnz) ||
-        (wide >= kBtWideNnz && 2ULL * runs >= static_cast<unsigned long long>(q.tiles) *
-                                                     static_cast<unsigned long long>(q.buckets));
+        pays && (runs * static_cast<unsigned long long>(kBtRunEntries) > static_cast<unsigned long long>(q.nnz) ||
+                 (q.nnz >= kBtWideNnz && 2ULL * runs >= static_cast<unsigned long long>(q.tiles) *
+                                                            static_cast<unsigned long long>(q.buckets)));
     if (threadIdx.x == 0) ok = 1;
     __syncthreads();
     for (int64_t b = threadIdx.x; b < q.buckets; b += kDecideThreads) {

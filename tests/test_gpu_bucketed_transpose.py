@@ -453,3 +453,34 @@ def test_banded_16_bit_transpose_keeps_the_csc_kernels(dev):
     y, plan = run(w)
     assert header(plan)[0] == 0
     assert_close(w.to("cpu"), y)
+
+
+# 40% of the entries in long rows; a row of 512 entries does not count as long, one of 513 does
+@pytest.mark.parametrize("nnz,mean,long_row,flag", [(3_000_000, 2, 512, 1), (3_000_000, 2, 513, 0),
+                                                    (4_000_000, 20, 4096, 1)])
+def test_16_bit_values_with_long_rows(dev, nnz, mean, long_row, flag):
+    """Long rows keep 16-bit transposes of few entries per row on the CSC kernels; either path's sums are within one
+    rounding of 64-bit ones."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(nnz + long_row)
+    rows = cols = nnz // mean
+    lengths = torch.zeros(rows, dtype=torch.int64, device=dev)
+    many = torch.arange(2 * nnz // 5 // long_row, device=dev) * 317 % rows
+    rest = nnz - many.numel() * long_row
+    lengths += rest // rows
+    lengths[: rest - int(lengths.sum())] += 1
+    lengths[many] = long_row
+    row_ptr, col = wl.csr_from_lengths(lengths, cols, g, dev, distinct=False)
+    vals = torch.randn(col.numel(), generator=g, device=dev).half()
+    x = (torch.rand(rows, generator=g, device=dev) * 2 - 1).half()
+    y = torch.full((cols,), float("nan"), device=dev).half()
+    plan = CsrSpMV(rows, cols, row_ptr.to(torch.int32), col, vals, x, y, 1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    assert header(plan)[0] == flag
+    prod = vals.double().cpu().numpy() * np.repeat(x.double().cpu().numpy(), lengths.cpu().numpy())
+    c = col.cpu().numpy()
+    exact = np.bincount(c, weights=prod, minlength=cols)
+    scale = np.bincount(c, weights=np.abs(prod), minlength=cols)
+    assert np.all(np.abs(y.double().cpu().numpy() - exact) <= 2.0**-11 * np.abs(exact) + 1e-5 * scale + 1e-7)
