@@ -17,8 +17,8 @@
 // entries 77 µs on hipCUB, 98 on the tiles; 100 000: 96 and 102; 500 000: 181
 // and 119), so those sizes keep it.
 //
-// Bound: HBM traffic, 12 bytes per entry in the first pass (the column twice,
-// one pair written less the position read) and 20 in the others.
+// Bound: HBM traffic, 16 bytes per entry in the first pass (the column read
+// twice, a pair written) and 20 in the others (the key twice, the position).
 // Reference counterpart: sparse/spmv/arch35/spmv_kernel.cpp:861-879 orders its
 // deterministic transpose by column.
 #include <hip/hip_runtime.h>

@@ -331,8 +331,9 @@ def test_mixed_row_lengths_meet_the_middle_of_every_tile(dev, seed):
 
 # rows, cols, mean: columns per bucket W and buckets S around the limits of the slot and place kernels
 PLACE_CASES = [
-    (600_000, 1 << 23, 4.0),  # W = 65536 (16 passes of 4096 columns), hyper-sparse columns
-    (1 << 20, (1 << 21) + 5, 4.0),  # W = 8192: two passes, the last bucket 5 columns wide
+    (600_000, 1 << 23, 4.0),  # W = 65536 (32 passes of 2048 columns), hyper-sparse columns
+    (1 << 20, (1 << 21) + 5, 4.0),  # W = 8192: four passes, the last bucket 5 columns wide
+    (1 << 20, (1 << 20) + 2049, 4.5),  # W = 4096: two passes, the last bucket 2049 columns wide
     (1 << 20, (1 << 20) + 4095, 6.5),  # W = 2048, a last bucket of 2047 columns
     (262_147, 8192, 8.5),  # W = 64, columns of about 270 entries
     (1 << 21, 1_800_001, 14.0),  # over 1400 buckets: the slot kernel's LDS beyond 64 KiB
