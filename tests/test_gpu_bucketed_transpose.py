@@ -485,3 +485,32 @@ def test_16_bit_values_with_long_rows(dev, nnz, mean, long_row, flag):
     exact = np.bincount(c, weights=prod, minlength=cols)
     scale = np.bincount(c, weights=np.abs(prod), minlength=cols)
     assert np.all(np.abs(y.double().cpu().numpy() - exact) <= 2.0**-11 * np.abs(exact) + 1e-5 * scale + 1e-7)
+
+
+# the line between the two kernels that write the column offsets (more columns than entries), with columns crowded at
+# either end, so that one entry is followed by almost all column starts
+@pytest.mark.parametrize("nnz", [1, 1023, 1024, 5000, 140_000])
+@pytest.mark.parametrize("more", [-1, 0, 1, 70_000])
+@pytest.mark.parametrize("crowd", ["low", "high", "spread"])
+@pytest.mark.parametrize("i64", [False, True])
+def test_column_offsets_line(dev, nnz, more, crowd, i64):
+    cols = nnz + more
+    if cols < 1:
+        pytest.skip("no columns")
+    rng = np.random.default_rng(nnz + more)
+    rows = nnz // 3 + 1
+    row_ptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, rows - 1)), [nnz]])
+    few = max(1, cols // 50)
+    col = rng.integers(0, cols if crowd == "spread" else few, nnz).astype(np.int32)
+    col = cols - 1 - col if crowd == "high" else col
+    val, x = rng.uniform(-1, 1, nnz).astype(np.float32), rng.uniform(-1, 1, rows).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    y = torch.full((cols,), float("nan"), device=dev)
+    plan = CsrSpMV(rows, cols, d(row_ptr.astype(np.int64 if i64 else np.int32)), d(col.astype(np.int32)), d(val), d(x), y,
+                   1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    prod = val.astype(np.float64) * x[np.repeat(np.arange(rows), np.diff(row_ptr))]
+    want, scale = np.bincount(col, weights=prod, minlength=cols), np.bincount(col, weights=np.abs(prod), minlength=cols)
+    assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * scale)
