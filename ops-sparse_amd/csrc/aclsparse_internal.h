@@ -515,8 +515,12 @@ inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valu
 
 // Sort of the entries by column for the CSC build (spmv_csc_sort.hip): a
 // stable radix sort in digits of at most kSortDigitBits bits over tiles of
-// kSortTile entries, whose temporary storage holds a count per digit and tile
-// and a total per digit; below kSortMinNnz entries hipCUB's.
+// kSortTile entries, which keeps a count per digit and tile and a total per
+// digit in an array of the entries' size that is written later (counts); below
+// kSortMinNnz entries hipCUB's, in place between two buffers and with
+// CscSortTempBytes of temporary storage.  (Neither takes workspace beyond the
+// pattern's own arrays to speak of: a call that allocates nothing has a fixed
+// number of bytes for it.)
 constexpr int64_t kSortTile = 16384;
 constexpr int kSortDigitBits = 8;
 constexpr int64_t kSortMinNnz = int64_t{1} << 17;
@@ -529,12 +533,13 @@ struct CscSort {
     const void* norm;     // normalised row offsets, int32 or int64 (rowptr64)
     bool rowptr64;
     int32_t *key, *val;   // results: the columns (cols for entries outside the matrix) in order, their CSR positions
-    int32_t *key_tmp, *val_tmp;
+    int32_t *key_tmp, *val_tmp;  // (the sort may swap results and temporaries)
+    uint32_t* counts;     // nnz words
     void* temp;           // CscSortTempBytes (+ 256: re-aligned to 256 bytes at use)
     size_t temp_bytes;
     const uint32_t* gate; // non-null (kSortMinNnz entries at least): a device word; nothing is written when it reads 1
 };
-int LaunchCscSort(const CscSort& c, void* stream);
+int LaunchCscSort(CscSort& c, void* stream);
 
 // Entries per group of the transpose's compact row table (one wave of 4 entries per lane).
 constexpr int64_t kRowGroup = 256;

@@ -38,6 +38,7 @@ constexpr int kSortRounds = static_cast<int>(kSortTile) / kSortThreads;  // entr
 constexpr int kSegment = kSortRounds * kWave;                            // consecutive entries per wave
 constexpr int kDigits = 1 << kSortDigitBits;
 static_assert(kSortTile % kSortThreads == 0, "whole rounds");
+static_assert((kSortMinNnz / kSortTile + 2) * kDigits <= kSortMinNnz, "counts fit a word per entry");
 
 struct SortParams {
     // first pass: keys from the matrix
@@ -281,13 +282,18 @@ __global__ __launch_bounds__(kSortThreads) void SortKeysKernel(SortParams q)
     q.val_out[k] = static_cast<int32_t>(k);
 }
 
-// (size query when temp is null)
-hipError_t SmallSort(void* temp, size_t& bytes, const SortParams& q, int32_t* key, int32_t* val, int bits,
-                     hipStream_t s)
+// Sorts (c.key, c.val); the result may lie in the temporaries, which then
+// change places with them (size query when temp is null).
+hipError_t SmallSort(void* temp, size_t& bytes, CscSort& c, int bits, hipStream_t s)
 {
-    return hipcub::DeviceRadixSort::SortPairs(temp, bytes, static_cast<const int32_t*>(q.key_out), key,
-                                              static_cast<const int32_t*>(q.val_out), val, static_cast<int>(q.nnz), 0,
-                                              bits, s);
+    hipcub::DoubleBuffer<int32_t> keys(c.key, c.key_tmp), vals(c.val, c.val_tmp);
+    const hipError_t e =
+        hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, vals, static_cast<int>(c.nnz), 0, bits, s);
+    c.key = keys.Current();
+    c.key_tmp = keys.Alternate();
+    c.val = vals.Current();
+    c.val_tmp = vals.Alternate();
+    return e;
 }
 
 template <typename RowT, bool kFirst>
@@ -303,22 +309,19 @@ void Pass(const SortParams& q, hipStream_t s)
 
 size_t CscSortTempBytes(int64_t nnz)
 {
-    if (nnz >= kSortMinNnz) {
-        const size_t tiles = static_cast<size_t>((nnz + kSortTile - 1) / kSortTile);
-        return (tiles + 1) * kDigits * sizeof(uint32_t);
-    }
+    if (nnz >= kSortMinNnz) return 0;
     return LastResult(nnz, [](int64_t n) {
         size_t bytes = 0;
-        SortParams q{};
-        q.nnz = n;
-        if (SmallSort(nullptr, bytes, q, nullptr, nullptr, 31, nullptr) != hipSuccess) {
+        CscSort c{};
+        c.nnz = n;
+        if (SmallSort(nullptr, bytes, c, 31, nullptr) != hipSuccess) {
             bytes = static_cast<size_t>(n) * 16 + (1 << 20);  // no device to ask: a generous bound
         }
         return bytes;
     });
 }
 
-int LaunchCscSort(const CscSort& c, void* stream)
+int LaunchCscSort(CscSort& c, void* stream)
 {
     if (c.nnz <= 0) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -331,20 +334,20 @@ int LaunchCscSort(const CscSort& c, void* stream)
     q.norm = c.norm;
     q.nnz = c.nnz;
     q.tiles = (c.nnz + kSortTile - 1) / kSortTile;
-    q.counts = static_cast<uint32_t*>(c.temp);
+    q.counts = c.counts;
     q.totals = q.counts + q.tiles * kDigits;
     q.gate = c.gate;
     int bits = 1;  // keys are 0 .. cols
     while (bits < 31 && (int64_t{1} << bits) <= c.cols) ++bits;
     if (c.nnz < kSortMinNnz) {
-        q.key_out = c.key_tmp;
-        q.val_out = c.val_tmp;
+        q.key_out = c.key;
+        q.val_out = c.val;
         const dim3 grid(static_cast<unsigned>((c.nnz + kSortThreads - 1) / kSortThreads));
         if (c.rowptr64) hipLaunchKernelGGL(SortKeysKernel<int64_t>, grid, dim3(kSortThreads), 0, s, q);
         else hipLaunchKernelGGL(SortKeysKernel<int32_t>, grid, dim3(kSortThreads), 0, s, q);
         void* temp = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(c.temp) + 255) & ~uintptr_t{255});
         size_t bytes = c.temp_bytes;
-        return SmallSort(temp, bytes, q, c.key, c.val, bits, s) == hipSuccess ? 0 : 1;
+        return SmallSort(temp, bytes, c, bits, s) == hipSuccess ? 0 : 1;
     }
     const int passes = (bits + kSortDigitBits - 1) / kSortDigitBits;
     for (int p = 0; p < passes; ++p) {

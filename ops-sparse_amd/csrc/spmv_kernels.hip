@@ -2172,8 +2172,18 @@ __global__ __launch_bounds__(kWave) void CscFinishKernel(const int32_t* keys, Ro
     for (int64_t w = blockIdx.x; w * kFinishSpan < n; w += gridDim.x) {
         const int64_t base = w * kFinishSpan;
         const int64_t end = base + kFinishSpan < n ? base + kFinishSpan : n;
-        if constexpr (sizeof(RowT) == 8) {
-            for (int64_t k = base + lane; k < end; k += kWave) pos[k] = sortedPos[k];
+        if (sizeof(RowT) == 8 || static_cast<const void*>(sortedPos) != pos) {
+            int32_t v[kFinishPer];
+#pragma unroll
+            for (int u = 0; u < kFinishPer; ++u) {  // one round trip (a loop of copies: 3 µs more)
+                const int64_t k = base + u * kWave + lane;
+                v[u] = k < end ? sortedPos[k] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < kFinishPer; ++u) {
+                const int64_t k = base + u * kWave + lane;
+                if (k < end) pos[k] = v[u];
+            }
         }
         if (cols <= n) {
             for (int64_t k = base + lane; k < (end == n ? n + 1 : end); k += kWave) CscColumnStarts(keys, colptr, cols, n, k);
@@ -3643,13 +3653,14 @@ int BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
     c.nnz = nnz;
     c.norm = At<void>(l.ws, l.layout.rowptr_offset);
     c.rowptr64 = sizeof(RowT) == 8;
-    // 32-bit positions; CscFinishKernel widens them into csc_pos for int64 offsets
-    int32_t* a = At<int32_t>(l.ws, l.layout.csc_pos_offset);
+    // 32-bit positions; for int64 offsets both buffers lie in val_b, and
+    // CscFinishKernel widens them into csc_pos
     int32_t* b = At<int32_t>(l.ws, l.layout.val_b_offset);
     c.key = At<int32_t>(l.ws, l.layout.key_a_offset);
     c.key_tmp = At<int32_t>(l.ws, l.layout.key_b_offset);
-    c.val = c.rowptr64 ? b : a;
-    c.val_tmp = c.rowptr64 ? a : b;
+    c.val = c.rowptr64 ? b : At<int32_t>(l.ws, l.layout.csc_pos_offset);
+    c.val_tmp = c.rowptr64 ? b + nnz : b;
+    c.counts = At<uint32_t>(l.ws, l.layout.entry_row_offset);  // CscFinishKernel's, after the sort
     c.temp = At<void>(l.ws, l.layout.sort_offset);
     c.temp_bytes = l.layout.sort_bytes;
     c.gate = gate;

@@ -182,3 +182,29 @@ def test_no_alloc_first_call_made_under_capture(dev):
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=240)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     assert "first-call-under-capture ok" in r.stdout
+
+
+@pytest.mark.parametrize("nnz,cols,i64", [(131_071, 3_789_000, False), (131_072, 3_788_900, False), (5000, 4_116_000, False),
+                                          (131_071, 1_837_000, True), (140_000, 1_821_000, True)])
+def test_transposes_close_to_the_limit(dev, nnz, cols, i64):
+    """Transposes whose tables fit the array with less than 0.1% to spare: the sort of the entries by column takes no
+    storage of its own beyond the pattern's arrays."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(nnz)
+    rows = cols
+    row = torch.sort(torch.randint(0, rows, (nnz,), generator=g, device=dev)).values
+    col = torch.randint(0, cols, (nnz,), generator=g, device=dev)
+    row_ptr = torch.zeros(rows + 1, dtype=torch.int64, device=dev)
+    row_ptr[1:] = torch.cumsum(torch.bincount(row, minlength=rows), 0)
+    vals = torch.rand(nnz, generator=g, device=dev) * 2 - 1
+    x = torch.rand(rows, generator=g, device=dev) * 2 - 1
+    y = torch.full((cols,), float("nan"), device=dev)
+    plan = CsrSpMV(rows, cols, row_ptr.to(torch.int64 if i64 else torch.int32), col.to(torch.int32), vals, x, y, 1.0, 0.0,
+                   op=Operation.TRANSPOSE)
+    assert 0.999 * MAX_BYTES < plan.workspace.numel() <= MAX_BYTES
+    assert no_alloc(plan) == Status.SUCCESS
+    torch.cuda.synchronize()
+    prod = vals.double() * x.double()[row]
+    want = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod)
+    scale = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod.abs())
+    assert bool(((y.double() - want).abs() <= 1e-5 * scale).all())
