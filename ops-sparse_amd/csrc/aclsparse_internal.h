@@ -516,15 +516,36 @@ inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valu
 // Sort of the entries by column for the CSC build (spmv_csc_sort.hip): a
 // stable radix sort in digits of at most kSortDigitBits bits over tiles of
 // kSortTile entries, which keeps a count per digit and tile and a total per
-// digit in an array of the entries' size that is written later (counts); below
-// kSortMinNnz entries hipCUB's, in place between two buffers and with
+// digit in an array of the entries' size that is written later (counts); for
+// fewer entries than OwnSort asks for hipCUB's, in place between two buffers and with
 // CscSortTempBytes of temporary storage.  (Neither takes workspace beyond the
 // pattern's own arrays to speak of: a call that allocates nothing has a fixed
 // number of bytes for it.)
 constexpr int64_t kSortTile = 16384;
 constexpr int kSortDigitBits = 8;
 constexpr int64_t kSortMinNnz = int64_t{1} << 17;
-size_t CscSortTempBytes(int64_t nnz);
+
+// Bits of the keys 0 .. cols, and the sort's passes over them.
+inline int SortBits(int64_t cols)
+{
+    int bits = 1;
+    while (bits < 31 && (int64_t{1} << bits) <= cols) ++bits;
+    return bits;
+}
+inline int SortPasses(int64_t cols) { return (SortBits(cols) + kSortDigitBits - 1) / kSortDigitBits; }
+
+// From 2^17 entries on, 2^17 more for every pass after the second: below, a
+// tile or a few per pass leave the chip idle and hipCUB's merge sort of so few
+// pairs is faster.  Preprocess, µs, hipCUB -> tiles: one pass (200 columns)
+// 135 000 entries 82 -> 58; two (60 000) 135 000 90 -> 93, 200 000 95 -> 93,
+// 260 000 127 -> 95; three (1 M) 200 000 109 -> 124, 260 000 138 -> 131; four
+// (20 M) 260 000 277 -> 292, 330 000 342 -> 339, 420 000 319 -> 315.
+inline bool OwnSort(int64_t cols, int64_t nnz)
+{
+    const int more = SortPasses(cols) - 2;
+    return nnz >= kSortMinNnz * (1 + (more > 0 ? more : 0));
+}
+size_t CscSortTempBytes(int64_t cols, int64_t nnz);
 struct CscSort {
     const int32_t* col;
     int64_t col_stride;
@@ -537,7 +558,7 @@ struct CscSort {
     uint32_t* counts;     // nnz words
     void* temp;           // CscSortTempBytes (+ 256: re-aligned to 256 bytes at use)
     size_t temp_bytes;
-    const uint32_t* gate; // non-null (kSortMinNnz entries at least): a device word; nothing is written when it reads 1
+    const uint32_t* gate; // non-null (only where OwnSort holds): a device word; nothing is written when it reads 1
 };
 int LaunchCscSort(CscSort& c, void* stream);
 
@@ -606,7 +627,7 @@ inline SpmvLayout ComputeLayout(uint64_t rows, uint64_t cols, uint64_t nnz, acls
             l.val_b_offset = AlignUp(l.key_b_offset + n * sizeof(int32_t));
             l.prod_offset = l.key_a_offset;  // prod[nnz] of <= 8 bytes ends before val_b
             l.sort_offset = AlignUp(l.val_b_offset + n * rb);
-            l.sort_bytes = CscSortTempBytes(static_cast<int64_t>(nnz));
+            l.sort_bytes = CscSortTempBytes(static_cast<int64_t>(cols), static_cast<int64_t>(nnz));
             l.csc_items_per_block = ItemsPerBlock(cols, nnz);
             l.csc_num_blocks = NumBlocks(cols, nnz);
             l.csc_blocks_offset = AlignUp(l.sort_offset + l.sort_bytes + 256);  // sort temp re-aligned to 256 at use

@@ -12,10 +12,7 @@
 // path decision (taken on the device) does not need the CSC pattern skips the
 // sort without the host knowing.
 //
-// Below kSortMinNnz entries a tile or a few leave the chip idle and hipCUB's
-// sort of so few pairs is faster (a transposed call with its set-up: 30 000
-// entries 77 µs on hipCUB, 98 on the tiles; 100 000: 96 and 102; 500 000: 181
-// and 119), so those sizes keep it.
+// Small matrices keep hipCUB's sort (OwnSort).
 //
 // Bound: HBM traffic, 16 bytes per entry in the first pass (the column read
 // twice, a pair written) and 20 in the others (the key twice, the position).
@@ -307,9 +304,9 @@ void Pass(const SortParams& q, hipStream_t s)
 
 }  // namespace
 
-size_t CscSortTempBytes(int64_t nnz)
+size_t CscSortTempBytes(int64_t cols, int64_t nnz)
 {
-    if (nnz >= kSortMinNnz) return 0;
+    if (OwnSort(cols, nnz)) return 0;
     return LastResult(nnz, [](int64_t n) {
         size_t bytes = 0;
         CscSort c{};
@@ -337,9 +334,8 @@ int LaunchCscSort(CscSort& c, void* stream)
     q.counts = c.counts;
     q.totals = q.counts + q.tiles * kDigits;
     q.gate = c.gate;
-    int bits = 1;  // keys are 0 .. cols
-    while (bits < 31 && (int64_t{1} << bits) <= c.cols) ++bits;
-    if (c.nnz < kSortMinNnz) {
+    const int bits = SortBits(c.cols);
+    if (!OwnSort(c.cols, c.nnz)) {
         q.key_out = c.key;
         q.val_out = c.val;
         const dim3 grid(static_cast<unsigned>((c.nnz + kSortThreads - 1) / kSortThreads));
@@ -349,7 +345,7 @@ int LaunchCscSort(CscSort& c, void* stream)
         size_t bytes = c.temp_bytes;
         return SmallSort(temp, bytes, c, bits, s) == hipSuccess ? 0 : 1;
     }
-    const int passes = (bits + kSortDigitBits - 1) / kSortDigitBits;
+    const int passes = SortPasses(c.cols);
     for (int p = 0; p < passes; ++p) {
         const int w = bits / passes + (p < bits % passes ? 1 : 0);
         q.digits = 1 << w;

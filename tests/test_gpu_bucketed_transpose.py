@@ -375,8 +375,10 @@ def test_columns_are_summed_in_row_order(dev, rows, cols, mean, x_offset):
     assert np.all(np.abs(got - exact) <= 1e-5 * scale)
 
 
-# entry counts around the CSC sort's smallest own size (2^17) and tile (16384) edges; columns of one to four digits
-@pytest.mark.parametrize("nnz", [1, 1025, 131_071, 131_072, 131_073, 147_455, 147_457])
+# entry counts around the CSC sort's smallest own sizes (2^17, with three digits 2^18, with four 3 * 2^17) and tile
+# (16384) edges; columns of one to four digits
+@pytest.mark.parametrize("nnz", [1, 1025, 131_071, 131_072, 131_073, 147_455, 147_457, 262_143, 262_145, 393_215,
+                                 393_217])
 @pytest.mark.parametrize("cols", [1, 255, 256, 70_000, 20_000_000])
 @pytest.mark.parametrize("i64", [False, True])
 def test_csc_sort_edges(dev, nnz, cols, i64):
