@@ -2109,8 +2109,8 @@ __device__ __forceinline__ bool CscGated(const uint32_t* gate) { return gate != 
 // none or spans more than 255 rows) and each entry's row minus it; the sorted
 // positions move to their final array if the sort left them in another
 // buffer, and the sorted columns give the column offsets (colptr[c] = first
-// sorted entry with column >= c, for c in [0, cols]) unless there are more
-// columns than entries (CscColPtrKernel).  One wave per
+// sorted entry with column >= c, for c in [0, cols]) unless CscColPtrKernel
+// does (OwnColumnStarts).  One wave per
 // workgroup; a wave takes kFinishSpan
 // consecutive entries: it finds the rows ra and rb of its first and last
 // in-range entry (wave-uniform searches), marks in LDS the first entry of
@@ -2122,6 +2122,7 @@ __device__ __forceinline__ bool CscGated(const uint32_t* gate) { return gate != 
 constexpr int kFinishPer = 16;
 constexpr int kFinishSpan = kFinishPer * kWave;
 constexpr int64_t kFinishWgs = 8192;  // one wave each, every wave slot of the chip
+constexpr int64_t kOwnStartsNnz = int64_t{1} << 20;
 template <typename RowT>
 __device__ __forceinline__ int64_t LastRowAtOrBefore(const RowT* norm, int64_t lo, int64_t hi, int64_t k)
 {
@@ -2142,10 +2143,18 @@ __device__ __forceinline__ void CscColumnStarts(const int32_t* keys, RowT* colpt
     for (int64_t c = prev + 1; c <= cur; ++c) colptr[c] = static_cast<RowT>(k);
 }
 
-// Column offsets of a matrix with more columns than entries, one thread per
-// entry: the waves of CscFinishKernel, of kFinishPer rounds each, take too
-// long over the columns between two entries (60 000 entries in 20 M columns:
-// Preprocess 902 µs there, 277 here; 1 M columns 112 and 78).
+// Column offsets by a launch of their own, one thread per entry, where the
+// waves of CscFinishKernel, of kFinishPer rounds each, take longer than that:
+// over the columns between two entries when there are more columns than
+// entries (60 000 entries in 20 M columns: Preprocess 902 µs there, 277 here;
+// 1 M columns 112 and 78), and when there are too few waves to fill the chip
+// (60 000 entries in 60 000 columns: Preprocess 75 -> 69 µs, 800 000 103 -> 99;
+// from kOwnStartsNnz on the launch may be one that only exits).
+__host__ __device__ constexpr bool OwnColumnStarts(int64_t cols, int64_t nnz)
+{
+    return cols > nnz || nnz < kOwnStartsNnz;
+}
+
 template <typename RowT>
 __global__ __launch_bounds__(kThreads) void CscColPtrKernel(const int32_t* keys, RowT* colptr, int64_t cols, int64_t n,
                                                             const uint32_t* gate)
@@ -2185,7 +2194,7 @@ __global__ __launch_bounds__(kWave) void CscFinishKernel(const int32_t* keys, Ro
                 if (k < end) pos[k] = v[u];
             }
         }
-        if (cols <= n) {
+        if (!OwnColumnStarts(cols, n)) {
             for (int64_t k = base + lane; k < (end == n ? n + 1 : end); k += kWave) CscColumnStarts(keys, colptr, cols, n, k);
         }
         const int64_t a = base > first ? base : first;
@@ -3665,7 +3674,7 @@ int BuildCsc(const SpmvLaunch& l, const uint32_t* gate, hipStream_t s)
     c.temp_bytes = l.layout.sort_bytes;
     c.gate = gate;
     if (LaunchCscSort(c, s) != 0) return 1;
-    if (l.cols > nnz) {
+    if (OwnColumnStarts(l.cols, nnz)) {
         hipLaunchKernelGGL((CscColPtrKernel<RowT>), dim3(GridFor(nnz + 1)), dim3(kThreads), 0, s, c.key,
                            At<RowT>(l.ws, l.layout.colptr_offset), l.cols, nnz, gate);
     }

@@ -489,9 +489,9 @@ def test_16_bit_values_with_long_rows(dev, nnz, mean, long_row, flag):
     assert np.all(np.abs(y.double().cpu().numpy() - exact) <= 2.0**-11 * np.abs(exact) + 1e-5 * scale + 1e-7)
 
 
-# the line between the two kernels that write the column offsets (more columns than entries), with columns crowded at
-# either end, so that one entry is followed by almost all column starts
-@pytest.mark.parametrize("nnz", [1, 1023, 1024, 5000, 140_000])
+# the lines between the two kernels that write the column offsets (more columns than entries, or fewer than 2^20 of
+# them), with columns crowded at either end, so that one entry is followed by almost all column starts
+@pytest.mark.parametrize("nnz", [1, 1023, 1024, 5000, 140_000, (1 << 20) - 1, 1 << 20])
 @pytest.mark.parametrize("more", [-1, 0, 1, 70_000])
 @pytest.mark.parametrize("crowd", ["low", "high", "spread"])
 @pytest.mark.parametrize("i64", [False, True])
