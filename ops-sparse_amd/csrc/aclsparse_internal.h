@@ -505,10 +505,26 @@ inline int32_t BtBucketShift(uint64_t cols, uint64_t nnz)
     return shift;
 }
 
+// 16-bit values have no banded kernel, whose choice is part of the bucketed
+// Preprocess, so for them the tables are only made for matrices that the
+// bucketed kernels may take: of 2^21 entries or more (below, a call with its
+// set-up took 177 -> 196 µs for tables that were not chosen), and whose rows
+// and columns, which those kernels pay for and the CSC kernels hardly do, are
+// not too many: fitted to 16 x 5 matrices with 0.1 to 3 rows and columns per
+// entry, of which none so left out takes less than 0.7 of the CSC kernels'
+// time on the bucketed ones, and none taken more than 1.03 of it (fp16, a
+// product, CSC -> bucketed: 2.2 M entries and columns, 6.6 M rows 38 -> 44
+// µs, 6.6 M columns and 2.2 M rows 49 -> 62; 9 M entries, 6.3 M columns, 9 M
+// rows 175 -> 85).
 inline bool BtEligible(uint64_t rows, uint64_t cols, uint64_t nnz, uint32_t valueBytes)
 {
     if (valueBytes == 0U || rows == 0U || cols == 0U) return false;
     if (nnz < static_cast<uint64_t>(kBtMinNnz) || nnz > 0x7FFFFFFFULL) return false;
+    if (valueBytes == 2U) {
+        const uint64_t tenth = nnz / 10;
+        const uint64_t r = rows > tenth ? rows - tenth : 0U, c = cols > tenth ? cols - tenth : 0U;
+        if (nnz < 2U * static_cast<uint64_t>(kBtMinNnz) || 7U * r + 8U * c + 36000000U > 32U * nnz) return false;
+    }
     const uint64_t w = uint64_t{1} << BtBucketShift(cols, nnz);
     return (cols + w - 1) / w <= static_cast<uint64_t>(kBtMaxBuckets);
 }

@@ -516,3 +516,28 @@ def test_column_offsets_line(dev, nnz, more, crowd, i64):
     prod = val.astype(np.float64) * x[np.repeat(np.arange(rows), np.diff(row_ptr))]
     want, scale = np.bincount(col, weights=prod, minlength=cols), np.bincount(col, weights=np.abs(prod), minlength=cols)
     assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * scale)
+
+
+# rows and columns per entry on both sides of the line from which 16-bit transposes may take the bucketed kernels
+@pytest.mark.parametrize("nnz,rows,cols,flag", [(1_200_000, 4_000_000, 4_000_000, 0), (2_097_151, 300_000, 300_000, 0),
+                                                (2_110_000, 300_000, 300_000, 1), (2_200_000, 6_600_000, 300_000, 0),
+                                                (2_200_000, 300_000, 6_600_000, 0), (4_400_000, 4_000_000, 300_000, 1)])
+def test_16_bit_values_of_many_rows_and_columns(dev, nnz, rows, cols, flag):
+    g = torch.Generator(device=dev)
+    g.manual_seed(nnz + cols)
+    row = torch.sort(torch.randint(0, rows, (nnz,), generator=g, device=dev)).values
+    col = torch.randint(0, cols, (nnz,), generator=g, device=dev)
+    row_ptr = torch.zeros(rows + 1, dtype=torch.int32, device=dev)
+    row_ptr[1:] = torch.cumsum(torch.bincount(row, minlength=rows), 0)
+    vals = torch.randn(nnz, generator=g, device=dev).bfloat16()
+    x = (torch.rand(rows, generator=g, device=dev) * 2 - 1).bfloat16()
+    y = torch.full((cols,), float("nan"), device=dev).bfloat16()
+    plan = CsrSpMV(rows, cols, row_ptr, col.to(torch.int32), vals, x, y, 1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    assert header(plan)[0] == flag
+    prod = vals.double() * x.double()[row]
+    want = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod)
+    scale = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod.abs())
+    assert bool(((y.double() - want).abs() <= 2.0**-8 * want.abs() + 1e-5 * scale + 1e-7).all())
