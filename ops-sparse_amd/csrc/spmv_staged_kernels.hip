@@ -1417,9 +1417,10 @@ __global__ __launch_bounds__(kSortThreads) void BtRankKernel(StageParams q)
 
 // One workgroup per bucket: its slots' places in column order (cl), stable,
 // so that a column's products lie in row order, and its columns' offsets
-// (colptr).  Columns are taken kBtPlaceCols at a time (once, unless the
-// matrix averages under six entries per column); per wave, counters per
-// column of its own consecutive stretch of the bucket's slots.
+// (colptr).  Columns are taken kBtPlaceCols at a time (once, or twice where
+// the matrix averages three to six entries per column; with fewer
+// BtPlaceWideKernel takes it); per wave, counters per column of its own
+// consecutive stretch of the bucket's slots.
 constexpr int kBtPlaceCols = 2048;
 constexpr int kBtPlaceRounds = 8;  // rounds of 64 slots in flight per wave
 inline unsigned BtPlaceLdsBytes(int32_t wshift)
@@ -1521,6 +1522,151 @@ __global__ __launch_bounds__(kSortThreads) void BtPlaceKernel(StageParams q)
         for (int i = s0; i < w1; i += kStep) place(i, k0, std::false_type{});
         for (int i = w1; i < s1; i += kStep) place(i, k0, std::true_type{});
         __syncthreads();
+    }
+    if (b + 1 == q.buckets && tid < 2) colptr[q.cols + tid] = static_cast<RowT>(rs + n);  // the end, and its pad entry
+}
+
+// BtPlaceKernel for buckets of kBtWideShift and more bits of columns, which it
+// would go over in four to 32 passes of about 19 µs each: the bucket's slots
+// sorted by column in LDS instead, stably and by two digits of eight bits, a
+// slot and its column in one word.  A round's lanes with equal digits find
+// each other by a ballot per bit, as in the column sort.  The sorted columns
+// then give the column offsets, 64 columns a turn per wave.  Bound by VALU
+// issue and by how few buckets such matrices have (54 to 128 workgroups).
+// Preprocess of fp32 transposes, µs, passes -> sorted: 2.2 M entries in 1.5 M
+// columns 274 -> 166, 3.3 M 422 -> 175, 6.6 M 730 -> 194; 9 M in 27 M columns
+// 1236 -> 334.  At 12 bits the two passes are the faster: about 16 µs.
+constexpr int kBtWideShift = 13;
+constexpr int kBtWideThreads = 1024;
+constexpr int kBtWideWaves = kBtWideThreads / kWave;
+constexpr int kBtWideRounds = static_cast<int>(kBtRegionCap) / kBtWideThreads;
+constexpr int kBtWideDigits = 256;
+constexpr unsigned kBtWideLdsBytes = 4U * (static_cast<unsigned>(kBtRegionCap) + kBtWideWaves * kBtWideDigits);
+static_assert(kBtWideRounds * kBtWideThreads == kBtRegionCap && kBtRegionCap <= 1 << 16, "whole rounds, 16-bit slots");
+
+template <typename RowT>
+__global__ __launch_bounds__(kBtWideThreads) void BtPlaceWideKernel(StageParams q)
+{
+    using Scan = hipcub::BlockScan<uint32_t, kBtWideThreads>;
+    extern __shared__ uint32_t btWideDyn[];
+    __shared__ typename Scan::TempStorage scanStorage;
+    if (FlagSet(q.flag) != 1U) return;
+    const int64_t b = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int64_t rs = q.start_bm[b * (q.tiles + 1)];
+    const int n = static_cast<int>(static_cast<int64_t>(q.start_bm[(b + 1) * (q.tiles + 1)]) - rs);
+    uint32_t* ex = btWideDyn;                 // [kBtRegionCap]
+    uint32_t* table = ex + kBtRegionCap;      // [kBtWideWaves][kBtWideDigits]
+    uint32_t* own = table + wv * kBtWideDigits;
+    const int seg = CeilDiv(CeilDiv(n, kBtWideWaves), kWave) * kWave;  // the wave's stretch
+    const int i0 = wv * seg + lane;
+    uint32_t e[kBtWideRounds], pos[kBtWideRounds];  // slot (high half) and column; place
+#pragma unroll
+    for (int r = 0; r < kBtWideRounds; ++r) {
+        if (r * kWave >= seg) break;  // uniform
+        const int i = i0 + r * kWave;
+        e[r] = i < n ? static_cast<uint32_t>(i) << 16 | q.bt_col[rs + i] : 0U;
+    }
+    // pos[r] = place of e[r] in a stable order by the digit at shift
+    const auto rank = [&](int shift) {
+        for (int i = tid; i < kBtWideWaves * kBtWideDigits; i += kBtWideThreads) table[i] = 0U;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBtWideRounds; ++r) {
+            if (r * kWave >= seg) break;
+            const bool in = i0 + r * kWave < n;
+            const uint32_t d = e[r] >> shift & (kBtWideDigits - 1);
+            uint64_t peers = __ballot(in);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const bool bit = (d >> k & 1U) != 0U;
+                const uint64_t set = __ballot(bit);
+                peers &= bit ? set : ~set;
+            }
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                static_cast<uint32_t>(peers >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0U));
+            const uint32_t before = __hip_atomic_load(own + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (in && below == 0U) {
+                __hip_atomic_fetch_add(own + d, static_cast<uint32_t>(__popcll(peers)), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            pos[r] = before + below;
+        }
+        __syncthreads();
+        uint32_t total = 0U;
+        if (tid < kBtWideDigits) {
+#pragma unroll
+            for (int v = 0; v < kBtWideWaves; ++v) total += table[v * kBtWideDigits + tid];
+        }
+        uint32_t first;
+        Scan(scanStorage).ExclusiveSum(total, first);
+        if (tid < kBtWideDigits) WaveBases<kBtWideWaves>(table, kBtWideDigits, tid, first);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBtWideRounds; ++r) {
+            if (r * kWave >= seg) break;
+            pos[r] += own[e[r] >> shift & (kBtWideDigits - 1)];
+        }
+    };
+    rank(0);
+#pragma unroll
+    for (int r = 0; r < kBtWideRounds; ++r) {
+        if (r * kWave >= seg) break;
+        if (i0 + r * kWave < n) ex[pos[r]] = e[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBtWideRounds; ++r) {
+        if (r * kWave >= seg) break;
+        e[r] = i0 + r * kWave < n ? ex[i0 + r * kWave] : 0U;
+    }
+    rank(8);  // (its barriers come before ex is written again)
+    uint16_t* place = reinterpret_cast<uint16_t*>(ex);  // [kBtRegionCap], by slot
+    uint16_t* sorted = place + kBtRegionCap;            // [kBtRegionCap], columns by place
+#pragma unroll
+    for (int r = 0; r < kBtWideRounds; ++r) {
+        if (r * kWave >= seg) break;
+        if (i0 + r * kWave < n) {
+            place[e[r] >> 16] = static_cast<uint16_t>(pos[r]);
+            sorted[pos[r]] = static_cast<uint16_t>(e[r]);
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kBtWideThreads) q.cl[rs + i] = place[i];
+
+    // a stripe of columns per wave (a multiple of 64): colptr[c] = rs + number of entries of columns below c
+    const int64_t c0 = b << q.wshift;
+    const int cols = 1 << q.wshift;
+    const int inside = q.cols - c0 < cols ? static_cast<int>(q.cols - c0) : cols;
+    const int cs = wv * (cols / kBtWideWaves);
+    const int ce = cs + cols / kBtWideWaves < inside ? cs + cols / kBtWideWaves : inside;
+    RowT* colptr = static_cast<RowT*>(q.colptr);
+    int at = 0;  // the entries before it lie in columns below the current ones
+    for (int hi = n; at < hi;) {
+        const int mid = (at + hi) / 2;
+        if (sorted[mid] < cs) at = mid + 1;
+        else hi = mid;
+    }
+    for (int c = cs; c < ce; c += kWave) {
+        const int col = c + lane;
+        int before = 0;
+        bool open = true;  // 64 entries looked at, all of them before col
+        while (true) {
+            const int k = at + lane < n ? sorted[at + lane] : 1 << 16;
+            int below = 0;
+#pragma unroll
+            for (int step = kWave / 2; step >= 1; step /= 2) {
+                below += __shfl(k, below + step - 1, kWave) < col ? step : 0;
+            }
+            below += __shfl(k, below, kWave) < col ? 1 : 0;
+            if (open) {
+                before = at + below;
+                open = below == kWave;
+            }
+            if (__ballot(open) == 0) break;
+            at += kWave;
+        }
+        if (col < ce) colptr[c0 + col] = static_cast<RowT>(rs + before);
     }
     if (b + 1 == q.buckets && tid < 2) colptr[q.cols + tid] = static_cast<RowT>(rs + n);  // the end, and its pad entry
 }
@@ -2075,6 +2221,7 @@ void AllowRankLds()
     static const bool once = [] {
         AllowLds(reinterpret_cast<const void*>(&BtRankKernel<RowT>), BtRankLdsBytes(kBtMaxBuckets + 1));
         AllowLds(reinterpret_cast<const void*>(&BtPlaceKernel<RowT>), BtPlaceLdsBytes(16));
+        AllowLds(reinterpret_cast<const void*>(&BtPlaceWideKernel<RowT>), kBtWideLdsBytes);
         return true;
     }();
     (void)once;
@@ -2137,8 +2284,12 @@ int BtPreprocessTyped(const SpmvLaunch& l, hipStream_t s)
     AllowRankLds<RowT>();
     hipLaunchKernelGGL((BtRankKernel<RowT>), dim3(XcdGrid(T)), dim3(kSortThreads), BtRankLdsBytes(L.st_buckets + 1), s,
                        q);
-    hipLaunchKernelGGL((BtPlaceKernel<RowT>), dim3(static_cast<unsigned>(L.st_buckets)), dim3(kSortThreads),
-                       BtPlaceLdsBytes(L.st_wshift), s, q);
+    const dim3 buckets(static_cast<unsigned>(L.st_buckets));
+    if (L.st_wshift >= kBtWideShift) {
+        hipLaunchKernelGGL((BtPlaceWideKernel<RowT>), buckets, dim3(kBtWideThreads), kBtWideLdsBytes, s, q);
+    } else {
+        hipLaunchKernelGGL((BtPlaceKernel<RowT>), buckets, dim3(kSortThreads), BtPlaceLdsBytes(L.st_wshift), s, q);
+    }
     return 0;
 }
 

@@ -331,9 +331,11 @@ def test_mixed_row_lengths_meet_the_middle_of_every_tile(dev, seed):
 
 # rows, cols, mean: columns per bucket W and buckets S around the limits of the slot and place kernels
 PLACE_CASES = [
-    (600_000, 1 << 23, 4.0),  # W = 65536 (32 passes of 2048 columns), hyper-sparse columns
-    (1 << 20, (1 << 21) + 5, 4.0),  # W = 8192: four passes, the last bucket 5 columns wide
-    (1 << 20, (1 << 20) + 2049, 4.5),  # W = 4096: two passes, the last bucket 2049 columns wide
+    (600_000, 1 << 23, 4.0),  # W = 65536 (sorted in LDS), hyper-sparse columns
+    (600_000, (1 << 22) + 65, 4.0),  # W = 32768, the last bucket 65 columns wide
+    (1 << 20, (1 << 21) + 16383, 2.2),  # W = 16384, the last bucket one column short
+    (1 << 20, (1 << 21) + 5, 4.0),  # W = 8192, the last bucket 5 columns wide
+    (1 << 20, (1 << 20) + 2049, 4.5),  # W = 4096: two passes of 2048 columns, the last bucket 2049 columns wide
     (1 << 20, (1 << 20) + 4095, 6.5),  # W = 2048, a last bucket of 2047 columns
     (262_147, 8192, 8.5),  # W = 64, columns of about 270 entries
     (1 << 21, 1_800_001, 14.0),  # over 1400 buckets: the slot kernel's LDS beyond 64 KiB
@@ -541,3 +543,39 @@ def test_16_bit_values_of_many_rows_and_columns(dev, nnz, rows, cols, flag):
     want = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod)
     scale = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, col, prod.abs())
     assert bool(((y.double() - want).abs() <= 2.0**-8 * want.abs() + 1e-5 * scale + 1e-7).all())
+
+
+# wide buckets (sorted in LDS) whose entries crowd in a few columns: one column of most of the bucket's entries at its
+# start, middle or end, empty buckets, buckets of 1, 63, 64, 65 and the most entries that the kernels take
+@pytest.mark.parametrize("width_bits", [13, 14, 15, 16])
+def test_wide_buckets_with_crowded_columns(dev, width_bits):
+    w = 1 << width_bits
+    rng = np.random.default_rng(width_bits)
+    counts = [32768, 0, 1, 63, 64, 65, 20000, 1024, 1025, 32767, 0, 5000] + [24000] * 90
+    cols = w * (len(counts) - 1) + w // 2 + 3
+    col = []
+    for b, n in enumerate(counts):
+        at = (0, w // 2, w - 1)[b % 3]
+        many = np.full(n * 2 // 3, at) if b % 2 else np.zeros(0, np.int64)
+        col.append(np.minimum(np.concatenate([many, rng.integers(0, w, n - len(many))]) + b * w, cols - 1))
+    col = rng.permutation(np.concatenate(col)).astype(np.int32)
+    nnz = len(col)
+    assert bucket_width(cols, nnz) == w
+    rows = nnz // 3
+    row_ptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, rows - 1)), [nnz]])
+    val, x = rng.uniform(-1, 1, nnz).astype(np.float32), rng.uniform(-1, 1, rows).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    y = torch.full((cols,), float("nan"), device=dev)
+    plan = CsrSpMV(rows, cols, d(row_ptr.astype(np.int32)), d(col), d(val), d(x), y, 1.0, 0.0, op=Operation.TRANSPOSE)
+    plan.preprocess()
+    plan.run()
+    torch.cuda.synchronize()
+    assert header(plan)[0] == 1
+    prod = val * x[np.repeat(np.arange(rows), np.diff(row_ptr))]
+    got = y.cpu().numpy()
+    want = np.zeros(cols, np.float32)
+    np.add.at(want, col, prod)
+    short = np.bincount(col, minlength=cols) <= 64
+    np.testing.assert_array_equal(got[short].view(np.uint32), (want[short] + 0.0).view(np.uint32))
+    exact = np.bincount(col, weights=prod.astype(np.float64), minlength=cols)
+    assert np.all(np.abs(got - exact) <= 1e-5 * np.bincount(col, weights=np.abs(prod), minlength=cols))
