@@ -911,13 +911,17 @@ constexpr int64_t kLdsPerCu = 160 * 1024;
 
 // A workgroup stages its tile, then its 16 waves take r turns of a row each.
 // The workgroups go over the CUs evenly, two at a time where two tiles fit a
-// CU's LDS.  Fewer rows make more, smaller workgroups: fuller last rounds,
-// more staging.
-int64_t LdsCost(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t tiles, int r, bool byElement)
+// CU's LDS and two workgroups its registers (single: fp32 tiles of 4 columns
+// per lane over 64 KiB, whose kernel runs four waves per SIMD; taken for pairs
+// at k of 65 to 80, 2748 x 76 x 830, 30% full, took 21.8 µs at the rows so
+// chosen, 18.4 at four, which it has now).  Fewer rows make more, smaller workgroups:
+// fuller last rounds, more staging.
+int64_t LdsCost(const LdsRate& c, int64_t m, int64_t nnz, int64_t lds, int64_t tiles, int r, bool byElement,
+                bool single)
 {
     const int64_t perBlock = int64_t{kLdsThreads / kMmWave} * r;
     const int64_t perCu = ((m + perBlock - 1) / perBlock * tiles + kCus - 1) / kCus;
-    const int64_t pairs = 2 * lds <= kLdsPerCu ? perCu / 2 : 0;
+    const int64_t pairs = 2 * lds <= kLdsPerCu && !single ? perCu / 2 : 0;
     const int64_t work = lds / c.bytes * (byElement ? 2 : 1) + r * (c.entry * nnz / m + c.turn);
     return pairs * (2 * work + c.group) + (perCu - 2 * pairs) * (work * c.alone / 16 + c.group);
 }
@@ -941,9 +945,10 @@ LdsShape LdsChoose(const SpmmLaunch& l, bool kahan, int fp32J, bool byElement)
     for (int j = l.fp16 ? 4 : fp32J; j >= (l.fp16 ? 1 : fp32J); j /= 2) {
         const int64_t tw = int64_t{kMmWave} * j;
         const int64_t lds = l.k * tw * (l.fp16 ? 2 : 4);
-        const LdsRate c = LdsRateOf(j, l.fp16 != 0, kahan && !l.fp16, lds > kLdsBytes);
+        const bool wide = lds > kLdsBytes;
+        const LdsRate c = LdsRateOf(j, l.fp16 != 0, kahan && !l.fp16, wide);
         for (int r = kLdsMaxRows; r >= 1; r /= 2) {
-            const int64_t cost = LdsCost(c, l.m, l.nnz, lds, (l.n + tw - 1) / tw, r, byElement);
+            const int64_t cost = LdsCost(c, l.m, l.nnz, lds, (l.n + tw - 1) / tw, r, byElement, wide && !l.fp16);
             if (best.j == 0 || cost < bestCost) {
                 best = {j, r};
                 bestCost = cost;

@@ -444,7 +444,7 @@ def test_bench_laplacian_block_full_size_bit_exact(dev):
 # k up to their limit of 256; last column tiles of 44 (whole 4-column groups), 1 and 255 columns
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("m", [1, 16, 17, 65, 1030, 2300])
-@pytest.mark.parametrize("k,n", [(33, 300), (128, 257), (256, 511), (200, 1024)])
+@pytest.mark.parametrize("k,n", [(33, 300), (76, 125), (128, 257), (256, 511), (200, 1024)])
 def test_lds_rows_and_tiles(dev, half, m, k, n):
     rp, col, val = _rand_csr(m, k, 0.3, m + k, bad_cols=m % 2 == 1, long_rows=True)
     rng = np.random.default_rng(n)
